@@ -551,6 +551,7 @@ struct Plan {
   bool staged = false;
   int64_t* st_order = nullptr;
   unsigned* st_hist = nullptr;
+  bool unchecked_order = false;  // io->order taken without the permutation check
   KernelRef k_count;
   KernelRef k;
   Shape shape;
@@ -801,7 +802,9 @@ int check_order_host(sdeh_ctx* c, const int64_t* order, int64_t n) {
 // Launch the prepared plan on `s` (kernel bracketed by the context events).
 int run_plan(sdeh_ctx* c, Plan& pl, hipStream_t s, unsigned long long* queue, bool timed) {
   sdeh_kargs& a = pl.a;
-  if (pl.save == SAVE_AT) {
+  // The kernels write NaN to the rows a trajectory does not reach, so only an order that
+  // may leave trajectories out (one not checked to be a permutation) needs the fill.
+  if (pl.save == SAVE_AT && pl.unchecked_order) {
     const int64_t cnt = a.n_saveat * pl.n_state * a.n;
     if (pl.es == 8) HIPCHK(c, sdeh_util_fill_f64((double*)a.u_saveat, __builtin_nan(""), cnt, s));
     else HIPCHK(c, sdeh_util_fill_f32((float*)a.u_saveat, __builtin_nanf(""), cnt, s));
@@ -1137,6 +1140,7 @@ int solve_impl(sdeh_ctx* c, const sdeh_solve_desc* d, const sdeh_io* io, int32_t
   // Permutation check on the device, except for the order sdeh_plan_order wrote last
   // (the kernels still never read an entry outside [0, n)).
   const bool planned = io->order == c->planned_order && n == c->planned_n;
+  pl.unchecked_order = !host && io->order && planned;
   if (!host && io->order && n > 0 && !planned) {
     int32_t* seen = (int32_t*)ar.take(sz.i32);
     HIPCHK(c, sdeh_util_zero_u64(c->counters + 5, 1, s));
