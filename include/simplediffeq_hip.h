@@ -122,7 +122,11 @@ typedef enum sdeh_save_layout {
 
 /* Scheduling of trajectories onto lanes. */
 typedef enum sdeh_schedule {
-  SDEH_SCHED_AUTO = 0,       /* library choice (autotuned) */
+  SDEH_SCHED_AUTO = 0,       /* the tuned schedule (sdeh_autotune); without one, by size:
+                                one launch while the ensemble is a few times what fits
+                                the GPU at once, beyond that staged where it applies and
+                                persistent elsewhere (persistent at any size when grid,
+                                chunk or refill is set) */
   SDEH_SCHED_ONE_LAUNCH = 1, /* one lane per trajectory, grid covers the ensemble */
   SDEH_SCHED_PERSISTENT = 2, /* resident grid; lanes refill from a device atomic queue */
   SDEH_SCHED_STAGED = 3      /* adaptive solvers with endpoint output, one lane per
@@ -166,7 +170,8 @@ typedef struct sdeh_solve_desc {
                                0: corrected */
   int32_t schedule;         /* sdeh_schedule */
   int32_t precision;        /* sdeh_precision */
-  int32_t block;            /* 0 = tuned; else workgroup size (multiple of 64, <= 1024) */
+  int32_t block;            /* 0 = tuned, else by schedule and layout (64 or 256); else
+                               workgroup size (64, 128, 192 or 256) */
   int32_t grid;             /* 0 = tuned; persistent schedule: number of workgroups */
   int32_t chunk;            /* 0 = tuned; persistent schedule: trajectories per queue
                                grab (the last grab takes what is left) */

@@ -549,6 +549,7 @@ struct Plan {
   // staged schedule (see run_plan): hand-out order of the second launch and its
   // sort scratch; the parked state lives in the kargs' st_* buffers
   bool staged = false;
+  bool default_staged = false;  // the library's choice: persistent where scratch is short
   int64_t* st_order = nullptr;
   unsigned* st_hist = nullptr;
   bool unchecked_order = false;  // io->order taken without the permutation check
@@ -558,8 +559,87 @@ struct Plan {
   sdeh_kargs a{};
 };
 
+// Whether the staged schedule applies: an adaptive solve with endpoint output, one lane
+// and one trajectory per lane, in the library's own order.
+bool stageable(const sdeh_solve_desc* d, const sdeh_io* io, const Plan& pl) {
+  return is_adaptive(d->alg) && pl.save == SAVE_END && !pl.packed && pl.k.lanes == 1 &&
+         pl.k.tpl == 1 && !io->order && d->n_traj > 1 && d->n_traj < (1ll << 32);
+}
+
+// Bytes from one parked record of a staged solve to the next (whole 64-byte sectors).
+size_t staged_stride(const sdeh_solve_desc* d, const Plan& pl) {
+  const size_t rec = SDEH_PARK_BYTES((size_t)pl.n_state, (size_t)pl.n_param, pl.es,
+                                     d->alg == SDEH_ALG_ATSIT5 ? 1 : 0, pl.kahan ? 1 : 0);
+  return (rec + 63) & ~size_t(63);
+}
+
+// The launch shape of an adaptive solve that names none and has not been tuned, for `n`
+// trajectories of which `sorted` says whether they are handed out longest first (the
+// span order, or an order that sdeh_plan_order made) and `can_stage` whether the staged
+// schedule is open to the solve.  `resident` = lanes that fit the GPU at once.
+//   one launch   up to 3 x resident lanes (4 x in the layouts with several lanes per
+//                trajectory, and for binary32 in a planned order at any size, binary64
+//                up to 8 x).  While every wave is resident the queue only costs: its
+//                atomics, its reset, and waves that take 64 slots each while others
+//                get none.  Beyond that the hardware's block dispatch serves as the
+//                queue until the waves' unequal lengths cost more than lane refills.
+//   staged       one tspan, endpoint output, beyond resident: its first pass ranks the
+//                trajectories (scratch bounded by kStagedBytes; no visit counters, which
+//                would count a resumed trajectory twice).
+//   persistent   the rest.
+// Measured (us, persistent | one launch | staged; Lorenz, tolerances 1e-7/1e-5 for
+// ATsit5, 1e-8/1e-6 AVern7, 1e-9 AVern9):
+//   one tspan  ATsit5 binary64   n = 1,024     617 |   487 |   630
+//              (resident 327,680)  65,536      834 |   543 |   672
+//                                 262,144    1,406 | 1,066 | 1,025
+//                                 524,288    1,896 | 1,860 | 1,505
+//                               2,097,152    5,428 | 6,542 | 4,810
+//   own spans  ATsit5 binary64    524,288      838 |   723 |   859
+//                               1,048,576    1,265 | 1,266 | 1,248
+//                               4,194,304    4,381 | 5,068 | 4,332
+//              AVern9 binary64    700,001    1,732 | 1,656 | 1,775
+//              AVern7 binary64  4,194,304    4,393 | 5,152 | 4,600
+//              ATsit5 binary32  1,048,576      585 |   509 |   651
+//   planned    ATsit5 binary64  1,048,576    1,256 | 1,055
+//                               4,194,304    4,192 | 4,289
+//              binary32 compensated, same    1,759 | 1,646
+//   saveat 31  AVern7 binary64    524,288    3,437 | 3,455
+//              (resident 196,608) 1,048,576  5,534 | 6,553
+//   GLV-16, 256 points, AVern9 on the matrix cores (resident 32,768 trajectories)
+//                                   1,024    5,570 | 1,506
+//                                  65,536    8,293 | 4,400
+//                                 131,072    8,173 | 7,943
+// One-lane kernels launch blocks of 64 (small ensembles spread over more CUs: 487
+// against 538 us at n = 1,024; the same beyond 65,536), the others blocks of 256 (their
+// LDS exchange buffers are sized for four waves: 12.9 against 7.9 ms in blocks of 64).
+// Persistent layouts with several lanes per trajectory claim one wave's slots at a time
+// (GLV-16 ATsit5, 500,000: 2,972 against 3,491 us claiming 64).
+constexpr size_t kStagedBytes = size_t(1) << 30;
+Shape default_shape(sdeh_ctx* c, const Plan& pl, int dtype, int64_t n, bool sorted, bool planned,
+                    bool can_stage) {
+  Shape sh;
+  const int lanes = pl.k.lanes > 0 ? pl.k.lanes : 1;
+  const int64_t work = (n + pl.k.tpl - 1) / pl.k.tpl * lanes;
+  const int64_t resident = (int64_t)c->cus * blocks_per_cu(c, pl.k, 256) * 256;
+  int64_t times = lanes > 1 ? 4 : 3;
+  if (planned) times = dtype == SDEH_F32 ? INT64_MAX / resident : 8;
+  sh.chunk = 64 / lanes;
+  if (can_stage && !sorted && work > resident) {
+    sh.schedule = SDEH_SCHED_STAGED;
+  } else if (work <= times * resident) {
+    sh.schedule = SDEH_SCHED_ONE_LAUNCH;
+    if (lanes == 1) sh.block = 64;
+  } else {
+    sh.schedule = SDEH_SCHED_PERSISTENT;
+  }
+  return sh;
+}
+
 // Validate the descriptor and fill everything except the device pointers.
-int plan_solve(sdeh_ctx* c, const sdeh_solve_desc* d, const sdeh_io* io, Plan* pl) {
+// `path`: which entry point runs the plan (the default launch shape depends on it).
+enum class Path { kDevice, kHost, kStatic, kGraph };
+int plan_solve(sdeh_ctx* c, const sdeh_solve_desc* d, const sdeh_io* io, Plan* pl,
+               Path path = Path::kDevice) {
   if (!d || !io) return fail(c, SDEH_E_INVALID, "desc and io must not be NULL");
   if (d->alg < SDEH_ALG_TSIT5 || d->alg > SDEH_ALG_EULER)
     return fail(c, SDEH_E_INVALID, "alg %d out of range", d->alg);
@@ -690,6 +770,24 @@ int plan_solve(sdeh_ctx* c, const sdeh_solve_desc* d, const sdeh_io* io, Plan* p
         sh.per_lane = tpl;
       }
     }
+    // (a caller that sets the queue's grid, chunk or refill batch gets the queue)
+    if (it == c->tuned.end() && d->schedule == SDEH_SCHED_AUTO && !d->grid && !d->chunk &&
+        !d->refill && d->n_traj > 0) {
+      const bool piped =
+          path == Path::kHost && d->n_traj >= kPipeMin && !io->order && !pl->packed;
+      const int64_t n = piped ? (d->n_traj + kPipeChunks - 1) / kPipeChunks : d->n_traj;
+      const bool planned = path == Path::kDevice && io->order && io->order == c->planned_order &&
+                           d->n_traj == c->planned_n;
+      const bool can_stage = (path == Path::kDevice || (path == Path::kHost && !piped)) &&
+                             stageable(d, io, *pl) && !io->visits &&
+                             (size_t)n * (staged_stride(d, *pl) + 16) <= kStagedBytes;
+      const int32_t w = sh.waves, tp = sh.per_lane;
+      sh = default_shape(c, *pl, d->dtype, n, planned || (pl->span && path != Path::kStatic),
+                         planned, can_stage);
+      sh.waves = w;
+      sh.per_lane = tp;
+      pl->default_staged = sh.schedule == SDEH_SCHED_STAGED;
+    }
     if (d->schedule != SDEH_SCHED_AUTO) sh.schedule = d->schedule;
     if (d->block) sh.block = d->block;
     if (d->chunk) sh.chunk = d->chunk;
@@ -712,8 +810,7 @@ int plan_solve(sdeh_ctx* c, const sdeh_solve_desc* d, const sdeh_io* io, Plan* p
   if (sh.schedule == SDEH_SCHED_STAGED) {
     // endpoint output, one lane per trajectory, the library's own order; the
     // second launch is the persistent one, so a staged shape falls back to it
-    pl->staged = adaptive && pl->save == SAVE_END && !pl->packed && pl->k.lanes == 1 &&
-                 pl->k.tpl == 1 && !io->order && d->n_traj > 1 && d->n_traj < (1ll << 32);
+    pl->staged = stageable(d, io, *pl);
     if (!pl->staged) sh.schedule = SDEH_SCHED_PERSISTENT;
     // (a staged solve orders its second launch itself; pl->span stays for the paths
     // that run the shape as persistent: graph capture, the host pipeline)
@@ -769,9 +866,7 @@ Sizes sizes_of(const sdeh_solve_desc* d, const sdeh_io* io, const Plan& pl) {
     s.span_hist = sdeh_util_span_scratch_bytes();
   }
   if (pl.staged) {
-    const size_t rec = SDEH_PARK_BYTES((size_t)pl.n_state, (size_t)pl.n_param, pl.es,
-                                       d->alg == SDEH_ALG_ATSIT5 ? 1 : 0, pl.kahan ? 1 : 0);
-    s.st_stride = (rec + 63) & ~size_t(63);  // whole 64-byte sectors per record
+    s.st_stride = staged_stride(d, pl);
     s.st_rec = n * s.st_stride;
     s.st_key = n * 8;
     s.st_order = n * 8;
@@ -982,11 +1077,11 @@ int solve_impl(sdeh_ctx* c, const sdeh_solve_desc* d, const sdeh_io* io, int32_t
                hipStream_t s, int32_t sync) {
   const auto t_start = std::chrono::steady_clock::now();
   Plan pl;
-  int r = plan_solve(c, d, io, &pl);
+  int r = plan_solve(c, d, io, &pl, memory == SDEH_MEM_HOST ? Path::kHost : Path::kDevice);
   if (r) return r;
   r = after_pending(c, s);
   if (r) return r;
-  const Sizes sz = sizes_of(d, io, pl);
+  Sizes sz = sizes_of(d, io, pl);
   const int64_t n = d->n_traj;
   if (n > 0) {
     if (!io->u0 || !io->u_end || !io->t_end || !io->retcode)
@@ -1018,25 +1113,35 @@ int solve_impl(sdeh_ctx* c, const sdeh_solve_desc* d, const sdeh_io* io, int32_t
   }
 
   // Device layout: saveat copy + (host mode) all buffers + counters always.
-  size_t need = round256(sz.saveat);
   const bool own_counts = !io->naccept || !io->nreject || host;
-  if (host) {
-    need += round256(sz.u0) + round256(sz.p) + round256(sz.ps) + round256(sz.tspan) +
-            round256(sz.dt0) + round256(sz.order) + round256(sz.u_end) + round256(sz.t_end) +
-            round256(sz.i32) + round256(sz.u_saveat) + round256(sz.u_steps) +
-            round256(sz.t_steps) + round256(sz.i32);
+  auto scratch_need = [&]() {
+    size_t need = round256(sz.saveat);
+    if (host) {
+      need += round256(sz.u0) + round256(sz.p) + round256(sz.ps) + round256(sz.tspan) +
+              round256(sz.dt0) + round256(sz.order) + round256(sz.u_end) + round256(sz.t_end) +
+              round256(sz.i32) + round256(sz.u_saveat) + round256(sz.u_steps) +
+              round256(sz.t_steps) + round256(sz.i32);
+    }
+    if (own_counts) need += 2 * round256(sz.i32);
+    if (!host && io->order) need += round256(sz.i32);
+    if (pl.packed) {
+      need += round256(sz.pk_tiles);
+      if (host) need += round256(sz.pk_off);
+    }
+    if (pl.span) need += round256(sz.span_order) + 2 * round256(sz.span_hist);
+    if (pl.staged)
+      need += round256(sz.st_rec) + round256(sz.st_key) + round256(sz.st_order) +
+              round256(sz.st_hist);
+    return need;
+  };
+  r = ensure_arena(c, scratch_need());
+  if (r == SDEH_E_NOMEM && pl.default_staged) {  // no room for the parked records
+    pl.staged = false;
+    pl.shape.schedule = SDEH_SCHED_PERSISTENT;
+    c->err.clear();
+    sz = sizes_of(d, io, pl);
+    r = ensure_arena(c, scratch_need());
   }
-  if (own_counts) need += 2 * round256(sz.i32);
-  if (!host && io->order) need += round256(sz.i32);
-  if (pl.packed) {
-    need += round256(sz.pk_tiles);
-    if (host) need += round256(sz.pk_off);
-  }
-  if (pl.span) need += round256(sz.span_order) + 2 * round256(sz.span_hist);
-  if (pl.staged)
-    need += round256(sz.st_rec) + round256(sz.st_key) + round256(sz.st_order) +
-            round256(sz.st_hist);
-  r = ensure_arena(c, need);
   if (r) return r;
   Arena ar{c->arena};
   double* d_saveat = (double*)ar.take(sz.saveat);
@@ -1234,7 +1339,7 @@ int solve_static_impl(sdeh_ctx* c, const sdeh_solve_desc* d, const sdeh_io* io, 
                       int32_t sync) {
   const auto t_start = std::chrono::steady_clock::now();
   Plan pl;
-  int r = plan_solve(c, d, io, &pl);
+  int r = plan_solve(c, d, io, &pl, Path::kStatic);
   if (r) return r;
   if (pl.save == SAVE_STEPS)
     return fail(c, SDEH_E_UNSUPPORTED,
@@ -1514,7 +1619,7 @@ int sdeh_graph_capture(sdeh_ctx* c, const sdeh_solve_desc* d, const sdeh_io* io,
   if (!c || !graph_handle) return SDEH_E_INVALID;
   HIPCHK(c, hipSetDevice(c->device));
   Plan pl;
-  int r = plan_solve(c, d, io, &pl);
+  int r = plan_solve(c, d, io, &pl, Path::kGraph);
   if (r) return r;
   if (io->order) return fail(c, SDEH_E_UNSUPPORTED, "graph capture takes no order permutation");
   if (pl.staged) {  // a captured solve runs the staged shape as its persistent launch
