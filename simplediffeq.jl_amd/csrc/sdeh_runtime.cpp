@@ -1256,14 +1256,16 @@ int solve_impl(sdeh_ctx* c, const sdeh_solve_desc* d, const sdeh_io* io, int32_t
     if (bad) return fail(c, SDEH_E_INVALID, "order is not a permutation of 0..n_traj-1");
   }
 
+  // the events' times are only read by synchronous calls, and each event is a barrier
+  // packet of its own between the kernels of back-to-back solves
+  const bool do_sync = host || sync;
   if (piped) {
     // p_shared and the saveat times went up on `s`; the kernels queue behind them
     r = run_host_pipeline(c, pl, io, s);
   } else {
-    r = run_plan(c, pl, s, c->counters, true);
+    r = run_plan(c, pl, s, c->counters, do_sync);
   }
   if (r) return r;
-  const bool do_sync = host || sync;
   note_pending(c, s, false);
   unsigned long long cnt[6] = {0, 0, 0, 0, 0, 0};  // counters [1..6]
   if (do_sync) {  // counters are only read back by synchronous calls
@@ -1409,7 +1411,7 @@ int solve_static_impl(sdeh_ctx* c, const sdeh_solve_desc* d, const sdeh_io* io, 
   a.nreject = io->nreject;
   a.u_saveat = io->u_saveat;
   a.visits = io->visits;
-  r = run_plan(c, pl, s, words, true);  // run_plan clears the queue word before a persistent launch
+  r = run_plan(c, pl, s, words, sync != 0);  // run_plan clears the queue word before a persistent launch
   if (r) return r;
   note_pending(c, s, false);
   c->stats = sdeh_stats{};
