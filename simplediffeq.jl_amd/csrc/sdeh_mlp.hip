@@ -341,233 +341,282 @@ __global__ void __launch_bounds__(256) mlp_forward_mfma(const float* __restrict_
 }
 
 // ---- training pass on the matrix cores ---------------------------------------
-// One wave per block; each wave takes 32-sample tiles and accumulates the gradient
-// of its tiles.  The three 64 x 64 products run on v_mfma_f32_32x32x2f32 (layouts as
-// in mlp_forward_mfma; A[i][k]: lane i + 32 (k % 2), B[k][j]: lane j + 32 (k % 2),
-// D register r of lane l: row 8(r/4) + 4(l/32) + r%4, column l % 32):
-//   forward  Z2[s][j] = sum_k H1[s][k] W2[j][k]      (M = samples, K = units)
-//   backward D1[s][k] = sum_j D2[s][j] W2[j][k]      (M = samples, K = units)
-//   gradient gW2[j][k] += sum_s D2[s][j] H1[s][k]    (M = units, K = samples)
-// H1, H2, D2 and the output gradients of a tile pass through the wave's LDS tile
-// to change layout.  Layers 1 and 3, the biases, the loss and the ReLU derivative
-// (1 where the unit's output is positive, else 0) are vector work.  The wave's gradient (and squared-error sum) goes to
-// partial[blockIdx.x]; mlp_grad_reduce adds the waves in a fixed order.
-struct GradTile {
-  float x[32 * NIN];
-  float h1[32 * H2P];
-  float h2[32 * H2P];
-  float d2[32 * H2P];
-  float g[32 * NOUT];
+// Blocks of four waves; a round takes 128 samples, 32 per wave.  Forward and backward
+// run transposed (D^T = W X^T: M = units, N = the wave's 32 samples) on
+// v_mfma_f32_32x32x2f32, as the binning step does on f16: output register r of tile t
+// in lane l holds sample l % 32 and unit 32 t + 8 (r / 4) + 4 (l / 32) + r % 4, which
+// is also the next product's B operand under that labelling of K, so nothing changes
+// layout between the layers:
+//   Z1^T = W1 X^T + b1,  Z2^T = W2 H1^T + b2,  D2^T = (W3^T g) [H2 > 0],
+//   D1^T = (W2^T D2^T) [H1 > 0]
+// (W2 and its transpose sit in LDS: one ds_read_b128 gives the A operands of four K
+// steps).  The weight gradients contract over samples instead, so H1, D2 and D1 pass
+// through LDS once ([sample][unit]), and the block's waves share them: wave w takes
+// the quadrant (w / 2, w % 2) of gW2 = D2^T H1 over all 128 samples (16 registers
+// instead of 64, and no gradient to add up across waves), and rows 16 w .. 16 w + 15 of
+// [gW1 | gb1] = D1^T [X | 1] on v_mfma_f32_16x16x4f32.  gb2 is the sum of the gW2
+// operand a wave reads anyway; gW3 = g H2^T stays in the sample layout (64 registers
+// per lane) until the block's end.  Each block's gradient and squared-error sum goes to
+// partial[blockIdx.x]; mlp_grad_reduce adds the blocks in a fixed order.
+// Bound by the FP32 matrix cores: 214 MFMAs of 64 cycles per 32 samples (10.3 us of
+// 65,536 samples on 1,024 SIMDs in the 64 x 64 products alone).  One wave per block held
+// all of gW2 and 46 KB of LDS, so three waves fit a CU and 1,024 blocks took two rounds:
+// 94.8 us at 65,536 samples, now 32.5 (the rest: vector work and LDS traffic between the
+// products, which one wave per SIMD does not overlap with them).
+constexpr int GP = NH + 4;          // LDS row of 64 floats, rows 16-byte aligned
+constexpr int GRAD_ROUND = 128;     // samples per block and round
+constexpr int GRAD_BLOCKS = 256;    // one block per CU (143 KB of LDS)
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+
+struct GradShared {
+  float w2[NH * GP];        // W2[j][k]
+  float w2t[NH * GP];       // W2[j][k] at [k][j]
+  float h1[4][32 * GP];     // per wave [sample][unit]
+  float d2[4][32 * GP];
+  float d1[4][32 * GP];
+  float x[4][32 * 8];       // features, 1, 0
+  float b1[NH], b2[NH], w3[NOUT][NH];
+  float sums[4][4];         // per wave: gb3, squared error
 };
 
-__global__ void __launch_bounds__(64) mlp_grad_mfma(const float* __restrict__ params,
-                                                    const float* __restrict__ x,
-                                                    const float* __restrict__ y, int64_t n,
-                                                    float* partial) {
-  __shared__ float sw[NPARAM];
-  __shared__ GradTile L;
-  load_params(sw, params);
-  const int l = threadIdx.x, li = l & 31, q = l >> 5;
-  const float inv = 1.0f / (float)(n * NOUT);
-  float wb[2][32];
+// Registers of a transposed output tile pair <-> four consecutive units in memory.
+template <class F>
+__device__ __forceinline__ void for_unit_quads(int q, F f) {
 #pragma unroll
   for (int t = 0; t < 2; ++t)
 #pragma unroll
-    for (int m = 0; m < 32; ++m) wb[t][m] = sw[OFF_W2 + (32 * t + li) * NH + 2 * m + q];
-  const float b2v[2] = {sw[OFF_B2 + li], sw[OFF_B2 + 32 + li]};
-  const float w3c[2][2] = {{sw[OFF_W3 + li], sw[OFF_W3 + 32 + li]},
-                           {sw[OFF_W3 + NH + li], sw[OFF_W3 + NH + 32 + li]}};
-  floatx16 gw2[2][2];
-#pragma unroll
-  for (int a = 0; a < 2; ++a)
-#pragma unroll
-    for (int b = 0; b < 2; ++b) gw2[a][b] = floatx16{};
-  float gw1[2][NIN], gb1[2] = {0.f, 0.f}, gb2[2] = {0.f, 0.f}, gw3[NOUT][2], gb3[NOUT] = {0.f, 0.f};
-  float gl = 0.f;
-#pragma unroll
-  for (int t = 0; t < 2; ++t) {
-#pragma unroll
-    for (int j = 0; j < NIN; ++j) gw1[t][j] = 0.f;
-#pragma unroll
-    for (int o = 0; o < NOUT; ++o) gw3[o][t] = 0.f;
+    for (int g = 0; g < 4; ++g) f(t, 4 * g, 32 * t + 8 * g + 4 * q);
+}
+
+__global__ void __launch_bounds__(256) mlp_grad_mfma(const float* __restrict__ params,
+                                                     const float* __restrict__ x,
+                                                     const float* __restrict__ y, int64_t n,
+                                                     float* partial) {
+  __shared__ __align__(16) GradShared L;
+  const int l = threadIdx.x & 63, w = threadIdx.x >> 6, li = l & 31, q = l >> 5;
+  for (int i = threadIdx.x; i < NH * NH; i += 256) {
+    const float v = params[OFF_W2 + i];
+    L.w2[(i >> 6) * GP + (i & 63)] = v;
+    L.w2t[(i & 63) * GP + (i >> 6)] = v;
   }
-  const int64_t tiles = (n + 31) / 32;
-  for (int64_t tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
-    const int64_t smp = tile * 32 + li;
+  if (threadIdx.x < NH) {
+    L.b1[threadIdx.x] = params[OFF_B1 + threadIdx.x];
+    L.b2[threadIdx.x] = params[OFF_B2 + threadIdx.x];
+  } else if (threadIdx.x < NH + NOUT * NH) {
+    (&L.w3[0][0])[threadIdx.x - NH] = params[OFF_W3 + threadIdx.x - NH];
+  }
+  float w1a[2][3];
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int m = 0; m < 3; ++m) w1a[t][m] = params[OFF_W1 + (32 * t + li) * NIN + 2 * m + q];
+  const float b30 = params[OFF_B3], b31 = params[OFF_B3 + 1];
+  const float inv = 1.0f / (float)(n * NOUT);
+  const int tj = w >> 1, tk = w & 1;
+  floatx16 gw2 = {};
+  floatx4 gw1 = {};
+  float gw3[NOUT][2][16] = {};
+  float gb2 = 0.f, gb30 = 0.f, gb31 = 0.f, gl = 0.f;
+  __syncthreads();
+  for (int64_t s0 = (int64_t)blockIdx.x * GRAD_ROUND; s0 < n;
+       s0 += (int64_t)gridDim.x * GRAD_ROUND) {
+    const int64_t smp = s0 + 32 * w + li;
     const bool valid = smp < n;
-    float xi[NIN];
+    float xv[3];
 #pragma unroll
-    for (int j = 0; j < NIN; ++j) xi[j] = valid ? x[smp * NIN + j] : 0.f;
-    wave_sync_lds();  // the previous tile's LDS reads are done
-    if (q == 0)
-#pragma unroll
-      for (int j = 0; j < NIN; ++j) L.x[li * NIN + j] = xi[j];
-    // layer 1 in the A layout: lane (li, q) holds units k = 2m + q of sample li
-    float h1a[32];
-#pragma unroll
-    for (int m = 0; m < 32; ++m) {
-      const int k = 2 * m + q;
-      float z = sw[OFF_B1 + k];
-#pragma unroll
-      for (int j = 0; j < NIN; ++j) z = fmaf(sw[OFF_W1 + k * NIN + j], xi[j], z);
-      h1a[m] = relu(z);
-      L.h1[li * H2P + k] = h1a[m];
+    for (int m = 0; m < 3; ++m) {
+      xv[m] = valid ? x[smp * NIN + 2 * m + q] : 0.f;
+      L.x[w][li * 8 + 2 * m + q] = xv[m];
     }
-    floatx16 z0 = {}, z1 = {};
+    L.x[w][li * 8 + 6 + q] = q == 0 ? 1.f : 0.f;
+    const float y0 = valid ? y[smp * NOUT] : 0.f, y1 = valid ? y[smp * NOUT + 1] : 0.f;
+    // layer 1
+    floatx16 h1[2];
+    for_unit_quads(q, [&](int t, int r, int u) {
+      const floatx4 b = *(const floatx4*)&L.b1[u];
 #pragma unroll
-    for (int m = 0; m < 32; ++m) {
-      z0 = __builtin_amdgcn_mfma_f32_32x32x2f32(h1a[m], wb[0][m], z0, 0, 0, 0);
-      z1 = __builtin_amdgcn_mfma_f32_32x32x2f32(h1a[m], wb[1][m], z1, 0, 0, 0);
-    }
+      for (int j = 0; j < 4; ++j) h1[t][r + j] = b[j];
+    });
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int row = 8 * (r >> 2) + 4 * q + (r & 3);
-      L.h2[row * H2P + li] = relu(z0[r] + b2v[0]);
-      L.h2[row * H2P + 32 + li] = relu(z1[r] + b2v[1]);
-    }
-    wave_sync_lds();
+    for (int m = 0; m < 3; ++m)
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+        h1[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(w1a[t][m], xv[m], h1[t], 0, 0, 0);
+    for_unit_quads(q, [&](int t, int r, int u) {
+      floatx4 v;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[j] = h1[t][r + j] = relu(h1[t][r + j]);
+      *(floatx4*)&L.h1[w][li * GP + u] = v;
+    });
+    // layer 2
+    floatx16 h2[2];
+    for_unit_quads(q, [&](int t, int r, int u) {
+      const floatx4 b = *(const floatx4*)&L.b2[u];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) h2[t][r + j] = b[j];
+    });
+    for_unit_quads(q, [&](int t, int r, int u) {
+      const floatx4 a0 = *(const floatx4*)&L.w2[li * GP + u];
+      const floatx4 a1 = *(const floatx4*)&L.w2[(32 + li) * GP + u];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        h2[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a0[j], h1[t][r + j], h2[0], 0, 0, 0);
+        h2[1] = __builtin_amdgcn_mfma_f32_32x32x2f32(a1[j], h1[t][r + j], h2[1], 0, 0, 0);
+      }
+    });
     // layer 3, error and output gradient of sample li (the two halves add up)
     float o0 = 0.f, o1 = 0.f;
+    for_unit_quads(q, [&](int t, int r, int u) {
+      const floatx4 c0 = *(const floatx4*)&L.w3[0][u], c1 = *(const floatx4*)&L.w3[1][u];
 #pragma unroll
-    for (int m = 0; m < 32; ++m) {
-      const int k = 2 * m + q;
-      const float h = L.h2[li * H2P + k];
-      o0 = fmaf(sw[OFF_W3 + k], h, o0);
-      o1 = fmaf(sw[OFF_W3 + NH + k], h, o1);
-    }
+      for (int j = 0; j < 4; ++j) {
+        const float h = h2[t][r + j] = relu(h2[t][r + j]);
+        o0 = fmaf(c0[j], h, o0);
+        o1 = fmaf(c1[j], h, o1);
+      }
+    });
     o0 += __shfl_xor(o0, 32);
     o1 += __shfl_xor(o1, 32);
-    const float e0 = valid ? o0 + sw[OFF_B3] - y[smp * NOUT] : 0.f;
-    const float e1 = valid ? o1 + sw[OFF_B3 + 1] - y[smp * NOUT + 1] : 0.f;
+    const float e0 = valid ? o0 + b30 - y0 : 0.f, e1 = valid ? o1 + b31 - y1 : 0.f;
+    const float g0 = 2.f * e0 * inv, g1 = 2.f * e1 * inv;
     if (q == 0) {
-      const float g0 = 2.f * e0 * inv, g1 = 2.f * e1 * inv;
-      L.g[li * NOUT] = g0;
-      L.g[li * NOUT + 1] = g1;
-      gb3[0] += g0;
-      gb3[1] += g1;
+      gb30 += g0;
+      gb31 += g1;
       gl = fmaf(e0, e0, gl);
       gl = fmaf(e1, e1, gl);
     }
-    wave_sync_lds();
-    // D2 = (W3^T g) [H2 > 0] in the D layout (rows: samples, column: unit)
+    floatx16 d2[2], d1[2] = {};
+    for_unit_quads(q, [&](int t, int r, int u) {
+      const floatx4 c0 = *(const floatx4*)&L.w3[0][u], c1 = *(const floatx4*)&L.w3[1][u];
+      floatx4 v;
 #pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int row = 8 * (r >> 2) + 4 * q + (r & 3);
-        const float g0 = L.g[row * NOUT], g1 = L.g[row * NOUT + 1];
-        const float h = L.h2[row * H2P + 32 * t + li];
-        const float d = h > 0.f ? fmaf(w3c[0][t], g0, w3c[1][t] * g1) : 0.f;
-        L.d2[row * H2P + 32 * t + li] = d;
-        gb2[t] += d;
-        gw3[0][t] = fmaf(g0, h, gw3[0][t]);
-        gw3[1][t] = fmaf(g1, h, gw3[1][t]);
+      for (int j = 0; j < 4; ++j) {
+        const float h = h2[t][r + j];
+        gw3[0][t][r + j] = fmaf(g0, h, gw3[0][t][r + j]);
+        gw3[1][t][r + j] = fmaf(g1, h, gw3[1][t][r + j]);
+        v[j] = d2[t][r + j] = h > 0.f ? fmaf(c0[j], g0, c1[j] * g1) : 0.f;
       }
-    wave_sync_lds();
-    // D1 = D2 W2 on the matrix cores, then times [H1 > 0]
-    floatx16 d0 = {}, d1 = {};
+      *(floatx4*)&L.d2[w][li * GP + u] = v;
+    });
+    for_unit_quads(q, [&](int t, int r, int u) {
+      const floatx4 a0 = *(const floatx4*)&L.w2t[li * GP + u];
+      const floatx4 a1 = *(const floatx4*)&L.w2t[(32 + li) * GP + u];
 #pragma unroll
-    for (int m = 0; m < 32; ++m) {
-      const float a = L.d2[li * H2P + 2 * m + q];
-      d0 = __builtin_amdgcn_mfma_f32_32x32x2f32(a, sw[OFF_W2 + (2 * m + q) * NH + li], d0, 0, 0,
-                                                0);
-      d1 = __builtin_amdgcn_mfma_f32_32x32x2f32(a, sw[OFF_W2 + (2 * m + q) * NH + 32 + li], d1,
-                                                0, 0, 0);
-    }
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int row = 8 * (r >> 2) + 4 * q + (r & 3);
-#pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        const float h = L.h1[row * H2P + 32 * t + li];
-        const float dd = h > 0.f ? (t == 0 ? d0[r] : d1[r]) : 0.f;
-        gb1[t] += dd;
-#pragma unroll
-        for (int j = 0; j < NIN; ++j) gw1[t][j] = fmaf(dd, L.x[row * NIN + j], gw1[t][j]);
+      for (int j = 0; j < 4; ++j) {
+        d1[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a0[j], d2[t][r + j], d1[0], 0, 0, 0);
+        d1[1] = __builtin_amdgcn_mfma_f32_32x32x2f32(a1[j], d2[t][r + j], d1[1], 0, 0, 0);
       }
-    }
-    // gW2 += D2^T H1 on the matrix cores (K = the tile's samples)
+    });
+    for_unit_quads(q, [&](int t, int r, int u) {
+      floatx4 v;
 #pragma unroll
-    for (int m = 0; m < 16; ++m) {
-      const int srow = 2 * m + q;
+      for (int j = 0; j < 4; ++j) v[j] = h1[t][r + j] > 0.f ? d1[t][r + j] : 0.f;
+      *(floatx4*)&L.d1[w][li * GP + u] = v;
+    });
+    __syncthreads();  // the round's H1, D2, D1 and X are in LDS
 #pragma unroll
-      for (int tj = 0; tj < 2; ++tj) {
-        const float a = L.d2[srow * H2P + 32 * tj + li];
+    for (int ww = 0; ww < 4; ++ww)
 #pragma unroll
-        for (int tk = 0; tk < 2; ++tk)
-          gw2[tj][tk] = __builtin_amdgcn_mfma_f32_32x32x2f32(
-              a, L.h1[srow * H2P + 32 * tk + li], gw2[tj][tk], 0, 0, 0);
+      for (int m = 0; m < 16; ++m) {
+        const float a = L.d2[ww][(2 * m + q) * GP + 32 * tj + li];
+        const float b = L.h1[ww][(2 * m + q) * GP + 32 * tk + li];
+        gw2 = __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, gw2, 0, 0, 0);
+        gb2 += a;
       }
-    }
-  }
-  // the two halves of the wave hold different sample rows of the same units
 #pragma unroll
-  for (int t = 0; t < 2; ++t) {
-    gb1[t] += __shfl_xor(gb1[t], 32);
-    gb2[t] += __shfl_xor(gb2[t], 32);
+    for (int ww = 0; ww < 4; ++ww)
 #pragma unroll
-    for (int j = 0; j < NIN; ++j) gw1[t][j] += __shfl_xor(gw1[t][j], 32);
-#pragma unroll
-    for (int o = 0; o < NOUT; ++o) gw3[o][t] += __shfl_xor(gw3[o][t], 32);
-  }
-  // per-sample sums over the 32 sample lanes (the q == 1 lanes hold zeros)
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    gb3[0] += __shfl_xor(gb3[0], off);
-    gb3[1] += __shfl_xor(gb3[1], off);
-    gl += __shfl_xor(gl, off);
+      for (int m = 0; m < 8; ++m) {
+        const int row = 4 * m + (l >> 4);
+        gw1 = __builtin_amdgcn_mfma_f32_16x16x4f32(L.d1[ww][row * GP + 16 * w + (l & 15)],
+                                                   L.x[ww][row * 8 + (l & 7)], gw1, 0, 0, 0);
+      }
+    __syncthreads();  // before the next round overwrites them
   }
   float* pb = partial + (int64_t)blockIdx.x * (NPARAM + 1);
 #pragma unroll
-  for (int tj = 0; tj < 2; ++tj)
+  for (int r = 0; r < 16; ++r)
+    pb[OFF_W2 + (32 * tj + 8 * (r >> 2) + 4 * q + (r & 3)) * NH + 32 * tk + li] = gw2[r];
+  gb2 += __shfl_xor(gb2, 32);  // the halves hold the odd and even samples
+  if (tk == 0 && q == 0) pb[OFF_B2 + 32 * tj + li] = gb2;
 #pragma unroll
-    for (int tk = 0; tk < 2; ++tk)
+  for (int r = 0; r < 4; ++r) {  // D of 16x16x4: row 4 (l / 16) + r, column l % 16
+    const int u = 16 * w + 4 * (l >> 4) + r, c = l & 15;
+    if (c < NIN) pb[OFF_W1 + u * NIN + c] = gw1[r];
+    if (c == NIN) pb[OFF_B1 + u] = gw1[r];
+  }
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int jrow = 32 * tj + 8 * (r >> 2) + 4 * q + (r & 3);
-        pb[OFF_W2 + jrow * NH + 32 * tk + li] = gw2[tj][tk][r];
-      }
-  if (q == 0) {
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      const int k = 32 * t + li;
-#pragma unroll
-      for (int j = 0; j < NIN; ++j) pb[OFF_W1 + k * NIN + j] = gw1[t][j];
-      pb[OFF_B1 + k] = gb1[t];
-      pb[OFF_B2 + k] = gb2[t];
-#pragma unroll
-      for (int o = 0; o < NOUT; ++o) pb[OFF_W3 + o * NH + k] = gw3[o][t];
-    }
+  for (int off = 32; off > 0; off >>= 1) {  // the q == 1 lanes hold zeros
+    gb30 += __shfl_xor(gb30, off);
+    gb31 += __shfl_xor(gb31, off);
+    gl += __shfl_xor(gl, off);
   }
   if (l == 0) {
-    pb[OFF_B3] = gb3[0];
-    pb[OFF_B3 + 1] = gb3[1];
-    pb[NPARAM] = gl;
+    L.sums[w][0] = gb30;
+    L.sums[w][1] = gb31;
+    L.sums[w][2] = gl;
+  }
+  // gW3: [wave][value][lane] through LDS (rows of 65), then two threads per entry
+  constexpr int VP = 65;
+  float* sv = &L.h1[0][0];
+  static_assert(4 * 64 * VP <= 3 * 4 * 32 * GP, "gW3's exchange fits h1, d2 and d1");
+#pragma unroll
+  for (int o = 0; o < NOUT; ++o)
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        sv[(w * 64 + o * 32 + t * 16 + r) * VP + l] = gw3[o][t][r];
+  __syncthreads();
+  {
+    // entry e: value e / 2 of lane half e % 2; thread halves take waves 0, 1 and 2, 3
+    const int e = threadIdx.x >> 1, half = threadIdx.x & 1, v = e >> 1, eq = e & 1;
+    float s = 0.f;
+#pragma unroll
+    for (int ww = 0; ww < 2; ++ww)
+#pragma unroll
+      for (int i = 0; i < 32; ++i) s += sv[((2 * half + ww) * 64 + v) * VP + 32 * eq + i];
+    s += __shfl_xor(s, 1);
+    const int o = v >> 5, t = (v >> 4) & 1, r = v & 15;
+    if (half == 0)
+      pb[OFF_W3 + o * NH + 32 * t + 8 * (r >> 2) + 4 * eq + (r & 3)] = s;
+  }
+  if (threadIdx.x < 3) {
+    const int k = threadIdx.x;
+    pb[k < 2 ? OFF_B3 + k : NPARAM] =
+        ((L.sums[0][k] + L.sums[1][k]) + L.sums[2][k]) + L.sums[3][k];
   }
 }
 
-// Sum the block partials in a fixed order (deterministic): accumulator r takes
-// blocks r, r + 16, r + 32, ... in turn, then the 16 accumulators are added in
-// order.  Sixteen independent loads per step keep the memory pipeline busy.
-__global__ void mlp_grad_reduce(const float* __restrict__ partial, int nblocks, float* grad,
-                                float* loss, float inv_count) {
-  constexpr int R = 16;
-  const int j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j > NPARAM) return;
-  float acc[R];
+// Sum the block partials in a fixed order (deterministic): 32 columns per block, the
+// rows split over 8 groups of threads (group g takes rows g, g + 8, ...), each with
+// four accumulators, all added in order.  Latency-bound: with one thread per column 19
+// CUs read the 19.4 MB of 1,024 partials in 58 us; 149 blocks read the 4.9 MB of 256 in
+// 6.6 us.
+__global__ void __launch_bounds__(256) mlp_grad_reduce(const float* __restrict__ partial,
+                                                       int nblocks, float* grad, float* loss,
+                                                       float inv_count) {
+  __shared__ float part[8][33];
+  const int col = threadIdx.x & 31, g = threadIdx.x >> 5;
+  const int j = blockIdx.x * 32 + col;
+  float acc[4] = {0.f, 0.f, 0.f, 0.f};
+  if (j <= NPARAM) {
+    int b = g;
+    for (; b + 24 < nblocks; b += 32) {
 #pragma unroll
-  for (int r = 0; r < R; ++r) acc[r] = 0.f;
-  int b = 0;
-  for (; b + R <= nblocks; b += R) {
-#pragma unroll
-    for (int r = 0; r < R; ++r) acc[r] += partial[(int64_t)(b + r) * (NPARAM + 1) + j];
+      for (int r = 0; r < 4; ++r) acc[r] += partial[(int64_t)(b + 8 * r) * (NPARAM + 1) + j];
+    }
+    for (; b < nblocks; b += 8) acc[0] += partial[(int64_t)b * (NPARAM + 1) + j];
   }
-  for (int r = 0; b + r < nblocks; ++r) acc[r] += partial[(int64_t)(b + r) * (NPARAM + 1) + j];
-  float s = acc[0];
+  part[g][col] = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+  __syncthreads();
+  if (g == 0 && j <= NPARAM) {
+    float s = part[0][col];
 #pragma unroll
-  for (int r = 1; r < R; ++r) s += acc[r];
-  if (j < NPARAM) grad[j] = s;
-  else *loss = s * inv_count;
+    for (int k = 1; k < 8; ++k) s += part[k][col];
+    if (j < NPARAM) grad[j] = s;
+    else *loss = s * inv_count;
+  }
 }
 
 __global__ void mlp_adam(float* p, const float* __restrict__ g, float* m, float* v, float lr,
@@ -643,12 +692,12 @@ extern "C" SDEH_HIDDEN int sdeh_mlp_plan_lorenz_impl(const float* params, const 
   return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 
-// Blocks of the gradient pass: one 64-lane block per 64 samples, at most 1024
-// (the blocks then stride over the rest).  The partial sums need
-// sdeh_mlp_grad_scratch_bytes(n) bytes of scratch.
+// Blocks of the gradient pass: one per round of samples, at most one per CU (the blocks
+// then stride over the rest).  The partial sums need sdeh_mlp_grad_scratch_bytes(n)
+// bytes of scratch.
 static int64_t grad_blocks(int64_t n) {
-  int64_t nb = (n + 31) / 32;  // one wave of 32-sample tiles per block
-  return nb > 1024 ? 1024 : (nb < 1 ? 1 : nb);
+  const int64_t nb = (n + GRAD_ROUND - 1) / GRAD_ROUND;
+  return nb > GRAD_BLOCKS ? GRAD_BLOCKS : (nb < 1 ? 1 : nb);
 }
 
 extern "C" SDEH_HIDDEN size_t sdeh_mlp_grad_scratch_bytes(int64_t n) {
@@ -660,10 +709,10 @@ extern "C" SDEH_HIDDEN int sdeh_mlp_loss_grad_impl(const float* params, const fl
                                                    const float* y, int64_t n, float* loss,
                                                    float* grad, float* scratch, hipStream_t s) {
   const int64_t nb = grad_blocks(n);
-  hipLaunchKernelGGL(mlp_grad_mfma, dim3((unsigned)nb), dim3(64), 0, s, params, x, y, n,
+  hipLaunchKernelGGL(mlp_grad_mfma, dim3((unsigned)nb), dim3(256), 0, s, params, x, y, n,
                      scratch);
   if (hipGetLastError() != hipSuccess) return -2;
-  hipLaunchKernelGGL(mlp_grad_reduce, dim3((NPARAM + 1 + 255) / 256), dim3(256), 0, s, scratch,
+  hipLaunchKernelGGL(mlp_grad_reduce, dim3((NPARAM + 1 + 31) / 32), dim3(256), 0, s, scratch,
                      (int)nb, grad, loss, 1.0f / (float)(n * NOUT));
   return hipGetLastError() == hipSuccess ? 0 : -2;
 }
