@@ -135,6 +135,10 @@ const void* by_save(int save, int kahan, int waves, int tpl) {
       case sdeh::SAVE_END: return adaptive_or_null<T, ALG, sdeh::SAVE_END, false>();
       case sdeh::SAVE_AT: return adaptive_or_null<T, ALG, sdeh::SAVE_AT, false>();
       case sdeh::SAVE_STEPS: return adaptive_or_null<T, ALG, sdeh::SAVE_STEPS, false>();
+      case sdeh::SAVE_RUNS:
+        if constexpr (sdeh::PkWave<T, R>::value)
+          return adaptive_or_null<T, ALG, sdeh::SAVE_RUNS, false>();
+        return nullptr;
     }
     return nullptr;
   }

@@ -49,7 +49,8 @@ namespace sdeh {
 
 enum { ALG_TSIT5 = 0, ALG_ATSIT5 = 1, ALG_VERN7 = 2, ALG_AVERN7 = 3, ALG_VERN9 = 4,
        ALG_AVERN9 = 5, ALG_RK4 = 6, ALG_EULER = 7 };
-enum { SAVE_END = 0, SAVE_AT = 1, SAVE_STEPS = 2 };
+// SAVE_RUNS: SAVE_STEPS in the packed layout, the rows written by the wave (flush_wave).
+enum { SAVE_END = 0, SAVE_AT = 1, SAVE_STEPS = 2, SAVE_RUNS = 3 };
 enum { RET_DEFAULT = 0, RET_DTMIN = 1, RET_NAN = 2, RET_MAXITERS = 3, RET_SAVE_OVERFLOW = 4 };
 // A staged solve's first launch parks trajectories still running after
 // stage_cap attempts; the second launch resumes them and overwrites the code.
@@ -846,18 +847,64 @@ __device__ __forceinline__ void store_save_time(const sdeh_kargs& a, int64_t row
   else a.t_steps[row * a.n + traj] = t;
 }
 
+// This lane's rank among the lanes of `mask`.
+__device__ __forceinline__ unsigned lane_rank(unsigned long long mask) {
+  return __builtin_amdgcn_mbcnt_hi((unsigned)(mask >> 32),
+                                   __builtin_amdgcn_mbcnt_lo((unsigned)mask, 0u));
+}
+
 // save_everystep output of one trajectory.  Fixed rows: point k goes to row k of
 // the trajectory's max_saves rows.  Packed (a.packed): point k goes to row
 // base + k of the shared output while k < lim, where base = steps_off[traj] and lim
 // = n_steps[traj] come from the counting pass and the offsets scan.  Packed rows
-// are held back in registers and written PK_ROWS at a time (consecutive rows:
-// contiguous bytes, so L2 sees whole runs of a trajectory's lines instead of one
-// 24-byte row per step, lines it would otherwise write back partly filled); the
-// trajectory's end writes the rest.
+// are held back and written PK_ROWS at a time (consecutive rows: contiguous bytes, so L2
+// sees whole runs of a trajectory's lines instead of one 24-byte row per step, lines it
+// would otherwise write back partly filled).
+//
+// The SAVE_RUNS kernels (adaptive solvers, small states; the host takes them for ensembles
+// beyond what fits the GPU at once) hold their rows in LDS and the wave writes them
+// together (flush_wave), run by run: a run is PK_ROWS output rows
+// that start at a multiple of PK_ROWS, so its 96 bytes of state and 32 of time (three
+// binary64 components) begin on 32-byte boundaries.  What costs is lines written in part:
+// runs of 96 bytes anywhere go to HBM at 0.96 TB/s, on 32-byte boundaries at 1.4, whole
+// 128-byte lines at 5.1.  Saving pass of the 2^20 Lorenz ATsit5 ensemble (67 M rows): each
+// lane storing its rows from registers 1,717 us, the wave storing unaligned runs 1,708,
+// aligned runs 1,440 (870 with the stores left out).  Small ensembles keep the registers:
+// a lone wave per SIMD waits for the flush's LDS round trips (1,024 trajectories 382
+// against 431 us).  Eight-row runs leave room for two waves per SIMD: 1,618 us.
 #ifndef SDEH_PK_ROWS
 #define SDEH_PK_ROWS 4
 #endif
 constexpr int PK_ROWS = SDEH_PK_ROWS;
+static_assert(PK_ROWS >= 2 && PK_ROWS <= 4 && (PK_ROWS & (PK_ROWS - 1)) == 0, "2 or 4 rows");
+
+// Whether packed rows go through LDS: one lane per trajectory and at most 32 bytes of
+// state, so that four waves' rows take at most a quarter of a CU's LDS for the states up
+// to three binary64 components (four waves per SIMD, as the registers allow).
+template <class T, class R>
+struct PkWave {
+  static constexpr bool value = R::G == 1 && R::N * sizeof(T) <= 32;
+};
+
+// One wave's rows in LDS.  Row `row` of the output goes to slot row % PK_ROWS of its
+// lane: u [lane][slot][component], t [lane][slot], the lanes an odd number of elements
+// apart (conflict-free for the lanes' own writes); list: the flush's runs.
+template <class T, int N>
+struct PkBuf {
+  static constexpr int US = PK_ROWS * N + 1 - (PK_ROWS * N) % 2, TS = PK_ROWS + 1;
+  // lanes that write one run: PK_ROWS * N of u and PK_ROWS of t, in a power of two
+  static constexpr int NEED = PK_ROWS * (N + 1);
+  static constexpr int LANES = NEED <= 8 ? 8 : NEED <= 16 ? 16 : NEED <= 32 ? 32 : 64;
+  static_assert(NEED <= 64, "a run fits the wave");
+  double t[64 * TS];
+  uint64_t list[64];
+  T u[64 * US];
+};
+template <class T, int N>
+__device__ __forceinline__ PkBuf<T, N>& pk_buf() {
+  __shared__ PkBuf<T, N> buf[4];  // blocks of at most 256 threads
+  return buf[threadIdx.x >> 6];
+}
 
 template <class T, int N>
 struct StepSink {
@@ -865,7 +912,7 @@ struct StepSink {
   int32_t lim;   // rows available (packed) or max_saves
   int32_t n;     // points offered
   int32_t kept;  // points stored (written or held back)
-  int32_t held;  // packed: rows held back, the last `held` of bt/bu
+  int32_t held;  // packed: rows held back, in LDS or the last `held` of bt/bu
   double bt[PK_ROWS];
   T bu[PK_ROWS][N];
 };
@@ -883,7 +930,7 @@ __device__ __forceinline__ void sink_start(const sdeh_kargs& a, StepSink<T, N>& 
   }
 }
 
-// Packed: write the rows held back (rows kept - held .. kept - 1).
+// Packed, rows in registers: write the rows held back (rows kept - held .. kept - 1).
 template <class T, class R>
 __device__ __forceinline__ void flush_steps(const sdeh_kargs& a, StepSink<T, R::N>& s) {
   if (!a.packed || s.held == 0) return;
@@ -902,12 +949,106 @@ __device__ __forceinline__ void flush_steps(const sdeh_kargs& a, StepSink<T, R::
   s.held = 0;
 }
 
+// Packed, rows in LDS: write the rows of the lanes flagged in `mine` (each at least one,
+// all of one aligned run of PK_ROWS rows), called by the whole wave.  The flagged lanes
+// list their runs; PkBuf::LANES consecutive lanes write one run, each lane always the same
+// element of u or t, so a run needs one list entry and one value read per lane.
 template <class T, class R>
+__device__ __forceinline__ void flush_wave(const sdeh_kargs& a, StepSink<T, R::N>& s, bool mine) {
+  constexpr int N = R::N;
+  typedef PkBuf<T, N> B;
+  constexpr unsigned PER = 64 / B::LANES;  // runs per pass
+  B& b = pk_buf<T, N>();
+  const unsigned long long mask = __ballot(mine);
+  const unsigned runs = (unsigned)__popcll(mask), l = (unsigned)__lane_id();
+  if (mine) {
+    const uint64_t end = (uint64_t)(s.base + s.kept);  // rows [end - held, end)
+    const uint64_t run = (end - 1) / PK_ROWS;
+    const uint64_t lo = (end - (uint64_t)s.held) - run * PK_ROWS, hi = end - run * PK_ROWS;
+    b.list[lane_rank(mask)] = run << 12 | l << 6 | lo << 3 | hi;
+    s.held = 0;
+  }
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  // this lane's element of a run: where it lies in a lane's LDS rows and in the output
+  const unsigned e = l % B::LANES;
+  const bool is_u = e < (unsigned)(PK_ROWS * N), is_t = !is_u && e < (unsigned)B::NEED;
+  const unsigned slot = is_u ? e / N : e - PK_ROWS * N;
+  const T* const lu = b.u + e;
+  const double* const lt = b.t + (is_t ? slot : 0);
+  T* const gu = (T*)a.u_steps + e;
+  double* const gt = a.t_steps + slot;
+  // four passes at a time, so that their LDS reads are in flight together (a lone wave
+  // otherwise waits for each: 2.8 us for 64 runs)
+  constexpr int Q = 4;
+  for (unsigned r0 = l / B::LANES; r0 < runs; r0 += Q * PER) {
+    uint64_t d[Q];
+#pragma unroll
+    for (int j = 0; j < Q; ++j) {
+      const unsigned r = r0 + j * PER;
+      d[j] = b.list[r < runs ? r : r0];
+      if (r >= runs) d[j] &= ~uint64_t(7);  // no rows
+    }
+    if constexpr (sizeof(T) == 8) {  // u and t alike: one read and one store per lane
+      const T* const lp = is_u ? lu : (const T*)lt;
+      T* const gp = is_u ? gu : (T*)gt;
+      const unsigned ls = is_u ? B::US : B::TS, gs = is_u ? PK_ROWS * N : PK_ROWS;
+      T v[Q];
+#pragma unroll
+      for (int j = 0; j < Q; ++j) v[j] = lp[((unsigned)(d[j] >> 6) & 63u) * ls];
+#pragma unroll
+      for (int j = 0; j < Q; ++j)
+        if (slot >= ((unsigned)(d[j] >> 3) & 7u) && slot < ((unsigned)d[j] & 7u))
+          gp[(d[j] >> 12) * gs] = v[j];
+    } else {
+      T vu[Q];
+      double vt[Q];
+#pragma unroll
+      for (int j = 0; j < Q; ++j) {
+        const unsigned src = (unsigned)(d[j] >> 6) & 63u;
+        if (is_u) vu[j] = lu[src * B::US];
+        else vt[j] = lt[src * B::TS];
+      }
+#pragma unroll
+      for (int j = 0; j < Q; ++j)
+        if (slot >= ((unsigned)(d[j] >> 3) & 7u) && slot < ((unsigned)d[j] & 7u)) {
+          if (is_u) gu[(d[j] >> 12) * (PK_ROWS * N)] = vu[j];
+          else gt[(d[j] >> 12) * PK_ROWS] = vt[j];
+        }
+    }
+  }
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();  // the reads are done before a lane writes its next row
+}
+
+// RUNS: rows go to LDS, and the caller calls flush_wave at the end of each aligned run.
+template <class T, class R, bool RUNS = false>
 __device__ __forceinline__ void save_step(const sdeh_kargs& a, StepSink<T, R::N>& s,
                                           int64_t traj, double t, const T (&u)[R::N]) {
   const bool lead = lane_comp<R>() == 0;
   ++s.n;
   if (s.kept >= s.lim) return;
+  if constexpr (RUNS) {
+    PkBuf<T, R::N>& b = pk_buf<T, R::N>();
+    const int l = (int)__lane_id();
+    const int64_t row = s.base + s.kept;
+    const int slot = (int)row & (PK_ROWS - 1);
+    if (s.kept == 0 && slot == PK_ROWS - 1) {
+      // a first row that ends its run goes out at once: the step after it may come
+      // before the next flush
+#pragma unroll
+      for (int c = 0; c < R::N; ++c) ((T*)a.u_steps)[row * R::N + c] = u[c];
+      a.t_steps[row] = t;
+    } else {
+#pragma unroll
+      for (int c = 0; c < R::N; ++c) b.u[l * PkBuf<T, R::N>::US + slot * R::N + c] = u[c];
+      b.t[l * PkBuf<T, R::N>::TS + slot] = t;
+      ++s.held;
+    }
+    ++s.kept;
+    return;
+  }
   if (a.packed) {
 #pragma unroll
     for (int k = 0; k + 1 < PK_ROWS; ++k) {  // shift: static register indices
@@ -927,8 +1068,7 @@ __device__ __forceinline__ void save_step(const sdeh_kargs& a, StepSink<T, R::N>
   ++s.kept;
 }
 
-// Leader's end-of-trajectory write of the save_everystep count (after
-// flush_steps on every lane of the trajectory).
+// Leader's end-of-trajectory write of the save_everystep count.
 template <class T, int N>
 __device__ __forceinline__ void finish_steps(const sdeh_kargs& a, const StepSink<T, N>& s,
                                              int64_t traj) {
@@ -977,11 +1117,6 @@ template <bool ON, class X>
 __device__ __forceinline__ X in_vgpr_if(X x) {
   if constexpr (ON) return in_vgpr(x);
   return x;
-}
-
-__device__ __forceinline__ unsigned lane_rank(unsigned long long mask) {
-  return __builtin_amdgcn_mbcnt_hi((unsigned)(mask >> 32),
-                                   __builtin_amdgcn_mbcnt_lo((unsigned)mask, 0u));
 }
 
 // Claim queue slots for the lanes flagged in `need` (called in uniform control
@@ -1461,6 +1596,8 @@ __device__ __forceinline__ void adaptive_body(const sdeh_kargs& a) {
   double t = 0.0, tf = 0.0;
   T dt = T(0), qold = T(0), qold_pow = T(0);
   int32_t nacc = 0, nrej = 0, cur = 0;
+  constexpr bool RUNS = SAVE == SAVE_RUNS, STEPS = RUNS || SAVE == SAVE_STEPS;
+  static_assert(!RUNS || PkWave<T, R>::value, "runs of a small state");
   StepSink<T, N> sk{};
   double ts_next = 0.0;  // save_time(cur)
   int64_t attempts = 0, traj = -1;
@@ -1492,6 +1629,14 @@ __device__ __forceinline__ void adaptive_body(const sdeh_kargs& a) {
                                               : a.maxiters);
 
   for (;;) {
+    if constexpr (RUNS) {
+      // Rows held in LDS: each lane's once they end an aligned run; those of ended
+      // trajectories before their lanes can take new ones, or at the wave's end.
+      const bool ends = a.persistent || __ballot(active) == 0ull;
+      const bool out = sk.held > 0 && (((sk.base + sk.kept) & (PK_ROWS - 1)) == 0 ||
+                                       (ends && !active));
+      if (__ballot(out) != 0ull) flush_wave<T, R>(a, sk, out);
+    }
     if (a.persistent) {
       bool want = !active && lead;
       // a batch of at least refill_min free slots (at most the wave's slot count, so
@@ -1551,9 +1696,9 @@ __device__ __forceinline__ void adaptive_body(const sdeh_kargs& a) {
         }
         ts_next = save_time(a, cur);
       }
-      if constexpr (SAVE == SAVE_STEPS) {
+      if constexpr (STEPS) {
         sink_start<R>(a, sk, traj);
-        save_step<T, R>(a, sk, traj, t, uprev);
+        save_step<T, R, RUNS>(a, sk, traj, t, uprev);
       }
       if constexpr (ALG == ALG_ATSIT5) R::f(fsal, uprev, pl, ps, t);  // FSAL seed, :241
     }
@@ -1679,7 +1824,7 @@ __device__ __forceinline__ void adaptive_body(const sdeh_kargs& a) {
               }
             }
           }
-          if constexpr (SAVE == SAVE_STEPS) save_step<T, R>(a, sk, traj, t, u);
+          if constexpr (STEPS) save_step<T, R, RUNS>(a, sk, traj, t, u);
           copyv(uprev, u);
           if constexpr (ALG == ALG_ATSIT5) copyv(fsal, k7);
           if constexpr (KAHAN) copyv(comp, comp_new);
@@ -1689,7 +1834,7 @@ __device__ __forceinline__ void adaptive_body(const sdeh_kargs& a) {
     }
 
     if (ret != -1) {  // trajectory ends or parks: write outputs (gpuatsit5.jl:322-329)
-      if (SAVE == SAVE_STEPS && ret == RET_DEFAULT && sk.kept < sk.n) ret = RET_SAVE_OVERFLOW;
+      if (STEPS && ret == RET_DEFAULT && sk.kept < sk.n) ret = RET_SAVE_OVERFLOW;
       const bool parked = STAGED && ret == RET_PARKED;
       if (!parked) {
         store_state<T, R>(a.u_end, 0, n, traj, uprev);
@@ -1700,7 +1845,7 @@ __device__ __forceinline__ void adaptive_body(const sdeh_kargs& a) {
           a.retcode[traj] = ret;
           if (a.naccept) a.naccept[traj] = nacc;
           if (a.nreject) a.nreject[traj] = nrej;
-          if constexpr (SAVE == SAVE_STEPS) finish_steps(a, sk, traj);
+          if constexpr (STEPS) finish_steps(a, sk, traj);
         }
       }
       if (STAGED && a.stage_cap > 0) {

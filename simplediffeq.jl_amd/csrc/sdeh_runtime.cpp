@@ -57,6 +57,8 @@ SDEH_HIDDEN int sdeh_util_static_saveat_max();
 SDEH_HIDDEN hipError_t sdeh_util_pack_offsets(const int32_t*, int32_t, int64_t, int64_t*, int64_t,
                                               int64_t*, int32_t*, unsigned long long*,
                                               hipStream_t);
+SDEH_HIDDEN hipError_t sdeh_util_count_order(const int32_t*, const int32_t*, int64_t, unsigned*,
+                                             int64_t*, hipStream_t);
 SDEH_HIDDEN int sdeh_mlp_forward_impl(const float*, const float*, float*, int64_t, hipStream_t);
 SDEH_HIDDEN int sdeh_mlp_plan_lorenz_impl(const float*, const double*, const double*,
                                           const double*, int64_t, const double*, float, float,
@@ -72,7 +74,7 @@ SDEH_HIDDEN int sdeh_mlp_adam_impl(float*, const float*, float*, float*, float, 
 
 namespace {
 
-enum { SAVE_END = 0, SAVE_AT = 1, SAVE_STEPS = 2 };
+enum { SAVE_END = 0, SAVE_AT = 1, SAVE_STEPS = 2, SAVE_RUNS = 3 };
 constexpr int64_t kUserBase = 1000;
 constexpr int64_t kDefaultMaxiters = 10000000;
 // Host-memory solves of at least kPipeMin trajectories run as kPipeChunks chunks:
@@ -85,6 +87,8 @@ constexpr int64_t kPipeMin = 1 << 17;
 // (0.95 after 16, 0.74 after 8).
 constexpr int32_t kStageAttempts = 32;
 constexpr int kPipeChunks = 4;
+// Default refill batch with one lane per trajectory (see plan_solve).
+constexpr int32_t kRefill = 4;
 // Register-cap variants (waves per SIMD) the autotuner tries after the launch shape.
 constexpr int kWaveVariants[] = {4, 6, 8};
 static_assert(8 + kPipeChunks <= 16, "chunk queues live in counters[8..16)");
@@ -538,6 +542,10 @@ struct Plan {
   // packed save_everystep: a counting pass (k_count, the endpoint kernel; adaptive
   // solvers only), the offsets scan, then the saving kernel
   bool packed = false;
+  // the counting pass runs staged and the saving kernel takes the trajectories by
+  // decreasing attempts, as counted, in one launch (see run_plan)
+  bool pk_ranked = false;
+  KernelRef k_runs;  // its kernel where it is not k
   int64_t pk_cap = 0;
   int64_t* pk_off = nullptr;
   int64_t* pk_tiles = nullptr;
@@ -787,6 +795,21 @@ int plan_solve(sdeh_ctx* c, const sdeh_solve_desc* d, const sdeh_io* io, Plan* p
       sh.waves = w;
       sh.per_lane = tp;
       pl->default_staged = sh.schedule == SDEH_SCHED_STAGED;
+      // packed output beyond resident: rank the saving pass by the counting pass
+      pl->pk_ranked = pl->packed && pl->k.lanes == 1 && !io->order && !io->visits && n > 1 &&
+                      n < (1ll << 32) &&
+                      n > (int64_t)c->cus * blocks_per_cu(c, pl->k, 256) * 256 &&
+                      (size_t)n * (staged_stride(d, *pl) + 16) <= kStagedBytes;
+      if (pl->pk_ranked) {
+        sh.schedule = SDEH_SCHED_ONE_LAUNCH;
+        sh.block = 256;
+        pl->span = false;
+        // the kernel that writes its rows by runs, for states of at most 32 bytes
+        KernelRef kr;
+        if ((size_t)pl->n_state * pl->es <= 32 &&
+            !resolve_kernel(c, d->rhs, d->alg, d->dtype, SAVE_RUNS, pl->kahan, 1, &kr))
+          pl->k_runs = kr;
+      }
     }
     if (d->schedule != SDEH_SCHED_AUTO) sh.schedule = d->schedule;
     if (d->block) sh.block = d->block;
@@ -825,7 +848,7 @@ int plan_solve(sdeh_ctx* c, const sdeh_solve_desc* d, const sdeh_io* io, Plan* p
   } else if (a.persistent) {
     const int slots = 64 / (pl->k.lanes > 0 ? pl->k.lanes : 1);
     int rf = d->refill ? d->refill : sh.refill;
-    if (!rf) rf = pl->k.lanes == 1 ? 4 : 1;
+    if (!rf) rf = pl->k.lanes == 1 ? kRefill : 1;
     sh.refill = rf < slots ? rf : slots;
   } else {
     sh.refill = 0;
@@ -865,7 +888,7 @@ Sizes sizes_of(const sdeh_solve_desc* d, const sdeh_io* io, const Plan& pl) {
     s.span_order = n * 8;
     s.span_hist = sdeh_util_span_scratch_bytes();
   }
-  if (pl.staged) {
+  if (pl.staged || pl.pk_ranked) {
     s.st_stride = staged_stride(d, pl);
     s.st_rec = n * s.st_stride;
     s.st_key = n * 8;
@@ -894,6 +917,35 @@ int check_order_host(sdeh_ctx* c, const int64_t* order, int64_t n) {
   return SDEH_OK;
 }
 
+// The staged launches of kernel `k` (`grid` persistent blocks of `block`): every
+// trajectory runs its first kStageAttempts attempts in a one-launch pass; those still
+// running park their state and an estimate of the attempts they still need, the
+// estimates are counting-sorted (largest first), and a persistent launch resumes the
+// parked trajectories in that order, so the longest start first and the end of the
+// launch drains less.  Parking stores the whole per-trajectory state (one record each,
+// so the resumed pass reads one or two cache lines per trajectory whatever the order),
+// and every trajectory takes the same steps as in one launch.
+int launch_staged(sdeh_ctx* c, const Plan& pl, const KernelRef& k, int grid, int block,
+                  unsigned long long* queue, hipStream_t s) {
+  sdeh_kargs a1 = pl.a;
+  a1.persistent = 0;
+  a1.order = nullptr;
+  a1.stage_cap = kStageAttempts;
+  a1.resume = 0;
+  const int64_t g1 = (a1.n * k.lanes + block - 1) / block;
+  HIPCHK(c, launch(k, (int)g1, block, &a1, s));
+  HIPCHK(c, sdeh_util_key_order(a1.st_key, a1.n, pl.st_hist, pl.st_order, s));
+  sdeh_kargs a2 = pl.a;
+  a2.persistent = 1;
+  a2.order = pl.st_order;
+  a2.stage_cap = 0;
+  a2.resume = 1;
+  if (a2.refill_min == 0) a2.refill_min = kRefill;  // the plan's own launch has no queue
+  HIPCHK(c, sdeh_util_zero_u64(queue, 1, s));
+  HIPCHK(c, launch(k, grid, block, &a2, s));
+  return SDEH_OK;
+}
+
 // Launch the prepared plan on `s` (kernel bracketed by the context events).
 int run_plan(sdeh_ctx* c, Plan& pl, hipStream_t s, unsigned long long* queue, bool timed) {
   sdeh_kargs& a = pl.a;
@@ -911,41 +963,33 @@ int run_plan(sdeh_ctx* c, Plan& pl, hipStream_t s, unsigned long long* queue, bo
       // rows per trajectory: naccept + 1 from an endpoint pass (the same arithmetic,
       // so the same steps), or the grid length of a fixed-step solver
       const bool counted = pl.k_count.aot || pl.k_count.fn;
-      if (counted) {
+      if (pl.pk_ranked) {
+        const int grid = c->cus * blocks_per_cu(c, pl.k_count, 256);
+        const int st = launch_staged(c, pl, pl.k_count, grid, 256, queue, s);
+        if (st) return st;
+      } else if (counted) {
         if (a.persistent) HIPCHK(c, sdeh_util_zero_u64(queue, 1, s));
         HIPCHK(c, launch(pl.k_count, pl.shape.grid, pl.shape.block, &a, s));
       }
       const int32_t add = counted ? 1 : (int32_t)std::max<int64_t>(a.g_len, 1);
       HIPCHK(c, sdeh_util_pack_offsets(counted ? a.naccept : nullptr, add, a.n, pl.pk_tiles,
                                        pl.pk_cap, pl.pk_off, a.n_steps, c->counters + 6, s));
+      // The counts rank the saving pass exactly: waves of equal lengths, longest first.
+      // (Lorenz ATsit5, 2^20 trajectories, 67 M rows: 3,120 us with both passes persistent;
+      // 2,820 with the staged endpoint pass and the ranked saving pass; 2,620 with the
+      // latter writing by runs.)
+      if (pl.pk_ranked) {
+        HIPCHK(c, sdeh_util_count_order(a.naccept, a.nreject, a.n, pl.st_hist, pl.st_order, s));
+        a.order = pl.st_order;
+      }
     }
     if (pl.staged) {
-      // Staged: every trajectory runs its first kStageAttempts attempts in a
-      // one-launch pass; those still running park their state and an estimate of
-      // the attempts they still need, the estimates are counting-sorted (largest
-      // first), and a persistent launch resumes the parked trajectories in that
-      // order, so the longest start first and the end of the launch drains less.
-      // Parking stores the whole per-trajectory state (one record each, so the
-      // resumed pass reads one or two cache lines per trajectory whatever the
-      // order), and every trajectory takes the same steps as in one launch.
-      sdeh_kargs a1 = a;
-      a1.persistent = 0;
-      a1.order = nullptr;
-      a1.stage_cap = kStageAttempts;
-      a1.resume = 0;
-      const int64_t g1 = (a.n * pl.k.lanes + pl.shape.block - 1) / pl.shape.block;
-      HIPCHK(c, launch(pl.k, (int)g1, pl.shape.block, &a1, s));
-      HIPCHK(c, sdeh_util_key_order(a.st_key, a.n, pl.st_hist, pl.st_order, s));
-      sdeh_kargs a2 = a;
-      a2.persistent = 1;
-      a2.order = pl.st_order;
-      a2.stage_cap = 0;
-      a2.resume = 1;
-      HIPCHK(c, sdeh_util_zero_u64(queue, 1, s));
-      HIPCHK(c, launch(pl.k, pl.shape.grid, pl.shape.block, &a2, s));
+      const int st = launch_staged(c, pl, pl.k, pl.shape.grid, pl.shape.block, queue, s);
+      if (st) return st;
     } else {
       if (a.persistent) HIPCHK(c, sdeh_util_zero_u64(queue, 1, s));
-      HIPCHK(c, launch(pl.k, pl.shape.grid, pl.shape.block, &a, s));
+      const bool runs = pl.pk_ranked && (pl.k_runs.aot || pl.k_runs.fn);
+      HIPCHK(c, launch(runs ? pl.k_runs : pl.k, pl.shape.grid, pl.shape.block, &a, s));
     }
     if (timed) HIPCHK(c, hipEventRecord(c->ev1, s));
   }
@@ -1129,14 +1173,20 @@ int solve_impl(sdeh_ctx* c, const sdeh_solve_desc* d, const sdeh_io* io, int32_t
       if (host) need += round256(sz.pk_off);
     }
     if (pl.span) need += round256(sz.span_order) + 2 * round256(sz.span_hist);
-    if (pl.staged)
+    if (pl.staged || pl.pk_ranked)
       need += round256(sz.st_rec) + round256(sz.st_key) + round256(sz.st_order) +
               round256(sz.st_hist);
     return need;
   };
   r = ensure_arena(c, scratch_need());
-  if (r == SDEH_E_NOMEM && pl.default_staged) {  // no room for the parked records
-    pl.staged = false;
+  if (r == SDEH_E_NOMEM && (pl.default_staged || pl.pk_ranked)) {
+    // no room for the parked records: the persistent schedule needs none
+    if (pl.pk_ranked) {
+      pl.shape.block = d->block ? d->block : 256;
+      pl.shape.grid = c->cus * blocks_per_cu(c, pl.k, pl.shape.block);
+      a.persistent = 1;
+    }
+    pl.staged = pl.pk_ranked = false;
     pl.shape.schedule = SDEH_SCHED_PERSISTENT;
     c->err.clear();
     sz = sizes_of(d, io, pl);
@@ -1234,7 +1284,7 @@ int solve_impl(sdeh_ctx* c, const sdeh_solve_desc* d, const sdeh_io* io, int32_t
       a.order = pl.span_ord;
     }
   }
-  if (pl.staged) {
+  if (pl.staged || pl.pk_ranked) {
     a.st_rec = ar.take(sz.st_rec);
     a.st_stride = (int64_t)sz.st_stride;
     a.st_key = (double*)ar.take(sz.st_key);

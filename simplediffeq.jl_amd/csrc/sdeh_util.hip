@@ -172,7 +172,7 @@ __global__ void write_i64(int64_t* p, int64_t v) {
 // a narrow span distribution fills would serialise them.  Within a (bucket, block)
 // the order is whatever the LDS atomics produce; no result depends on it.  The same
 // sort runs on other weights (BucketSrc): a staged solve's expected remaining
-// attempts (binary64 keys), and the cost model's predicted step counts, given as
+// attempts (binary64 keys), a counting pass's attempts, and the cost model's predicted step counts, given as
 // the plan's keys -log(count) in FP32.
 constexpr int SPAN_BUCKETS = 1024;
 constexpr int SPAN_BLOCKS = 256;
@@ -190,6 +190,8 @@ struct BucketSrc {
   const double* tspan;  // [2][n]: weight tf - t0
   const double* key;    // [n]: weight key[i]
   const float* lkey;    // [n]: weight exp(-lkey[i]), bucketed from lkey directly
+  const int32_t* cnt;   // [n]: weight cnt[i] + cnt2[i]
+  const int32_t* cnt2;
   int64_t n;
   __device__ __forceinline__ int operator()(int64_t i) const {
     if (lkey) {
@@ -202,6 +204,7 @@ struct BucketSrc {
       const int b = (int)__builtin_floorf(c) + 480;
       return b < 1 ? 1 : b;
     }
+    if (cnt) return weight_bucket((double)cnt[i] + (double)cnt2[i]);
     return weight_bucket(key ? key[i] : tspan[n + i] - tspan[i]);
   }
 };
@@ -395,14 +398,22 @@ static hipError_t bucket_order(BucketSrc src, unsigned* bh, int64_t* order, hipS
 
 extern "C" __attribute__((visibility("hidden"))) hipError_t sdeh_util_span_order(
     const double* tspan, int64_t n, unsigned* bh, int64_t* order, hipStream_t s) {
-  return bucket_order(BucketSrc{tspan, nullptr, nullptr, n}, bh, order, s);
+  return bucket_order(BucketSrc{tspan, nullptr, nullptr, nullptr, nullptr, n}, bh, order, s);
 }
 
 // order[0..n) = trajectories by decreasing key[i] (keys <= 0 and NaN last), on the
 // same buckets and scratch as sdeh_util_span_order.
 extern "C" __attribute__((visibility("hidden"))) hipError_t sdeh_util_key_order(
     const double* key, int64_t n, unsigned* bh, int64_t* order, hipStream_t s) {
-  return bucket_order(BucketSrc{nullptr, key, nullptr, n}, bh, order, s);
+  return bucket_order(BucketSrc{nullptr, key, nullptr, nullptr, nullptr, n}, bh, order, s);
+}
+
+// order[0..n) = trajectories by decreasing cnt[i] + cnt2[i] (the attempts a counting pass
+// made), same scratch.
+extern "C" __attribute__((visibility("hidden"))) hipError_t sdeh_util_count_order(
+    const int32_t* cnt, const int32_t* cnt2, int64_t n, unsigned* bh, int64_t* order,
+    hipStream_t s) {
+  return bucket_order(BucketSrc{nullptr, nullptr, nullptr, cnt, cnt2, n}, bh, order, s);
 }
 
 // order[0..n) = trajectories by increasing lkey[i] (the cost model's -log predicted
@@ -410,7 +421,7 @@ extern "C" __attribute__((visibility("hidden"))) hipError_t sdeh_util_key_order(
 // keys last.  Same scratch as sdeh_util_span_order.
 extern "C" __attribute__((visibility("hidden"))) hipError_t sdeh_util_logkey_order(
     const float* lkey, int64_t n, unsigned* bh, int64_t* order, hipStream_t s) {
-  return bucket_order(BucketSrc{nullptr, nullptr, lkey, n}, bh, order, s);
+  return bucket_order(BucketSrc{nullptr, nullptr, lkey, nullptr, nullptr, n}, bh, order, s);
 }
 
 // Scratch of the bucket sorts: the per-block counts and the tile sums.
