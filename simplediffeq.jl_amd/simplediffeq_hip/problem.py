@@ -322,14 +322,13 @@ def _solve_batch(eprob, alg, ens, idx, dt0s, order, kw):
     """One batch: solve, output_func, and the reruns it asks for."""
     repeats = [1] * len(idx)
     sols, raw = _solve_many(eprob, alg, ens, idx, repeats, dt0s, order, kw)
+    if eprob.output_func is None:
+        return sols, raw
     outs = [None] * len(idx)
     pending = list(range(len(idx)))
     while pending:
         again = []
         for j, s in zip(pending, sols):
-            if eprob.output_func is None:
-                outs[j] = s
-                continue
             x = eprob.output_func(s, idx[j] + 1)
             if not isinstance(x, tuple) or len(x) != 2:
                 raise TypeError("output_func must return (output, rerun)")
@@ -447,22 +446,28 @@ def _solve_many(eprob, alg, ens, idx, repeats, dt0s, order, kw):
     # ts = Vector{eltype(dt)} for the six Tsit5/Verner solvers without saveat
     t_type = (np.float32 if kw["t_f32"] and saveat_arr is None
               and alg.code not in _abi.FIXED_GRID_ONLY_ALGS else np.float64)
-    sols = []
-    for i in range(n):
-        rc = _abi.RETCODE_NAMES[int(bufs.retcode[i])]
-        if saveat_arr is not None:
-            t = saveat_arr
-            u = list(bufs.u_saveat[i])
-        elif everystep:
-            t, us = bufs.steps_of(i)
-            t = t.astype(t_type)
-            u = list(us)
-        else:
-            t = np.array([t0s[i], bufs.t_end[i]]).astype(t_type)
-            u = [u0s[:, i].astype(bufs.u_end.dtype), bufs.u_end[:, i]]
-        if out_np is not None:
-            u = [np.asarray(x).astype(out_np) for x in u]
-        if base.scalar_u:
-            u = [x[0] for x in u]
-        sols.append(ODESolution(t, u, rc, bufs.naccept[i], bufs.nreject[i], alg))
+    # One array operation per output for the whole ensemble, then one list of its rows:
+    # per-trajectory conversions took most of a solve of a few thousand trajectories.
+    if saveat_arr is not None:
+        block = bufs.u_saveat if out_np is None else bufs.u_saveat.astype(out_np)
+        ts = [saveat_arr] * n
+        us = [list(x) for x in (block[:, :, 0] if base.scalar_u else block)]
+    elif everystep:
+        off = bufs.steps_offset.tolist()
+        t_rows = bufs.t_steps[:off[n]].astype(t_type)
+        rows = bufs.u_steps[:off[n]] if out_np is None else bufs.u_steps[:off[n]].astype(out_np)
+        rows = list(rows[:, 0] if base.scalar_u else rows)
+        ts = [t_rows[i:j] for i, j in zip(off, off[1:])]
+        us = [rows[i:j] for i, j in zip(off, off[1:])]
+    else:
+        u_np = bufs.u_end.dtype if out_np is None else out_np
+        ends = np.empty((2 * n, n_state), dtype=u_np)
+        ends[::2], ends[1::2] = u0s.T.astype(bufs.u_end.dtype), bufs.u_end.T
+        rows = list(ends[:, 0] if base.scalar_u else ends)
+        ts = list(np.stack([t0s, bufs.t_end], axis=1).astype(t_type))
+        us = [[u, v] for u, v in zip(rows[::2], rows[1::2])]
+    names = _abi.RETCODE_NAMES
+    sols = [ODESolution(t, u, names[rc], na, nr, alg)
+            for t, u, rc, na, nr in zip(ts, us, bufs.retcode.tolist(), bufs.naccept.tolist(),
+                                        bufs.nreject.tolist())]
     return sols, bufs
