@@ -77,9 +77,13 @@ struct Ops<double> {
   // The controller's arguments stay in pow_log_ctrl's domain (normal, 0, Inf or
   // NaN; exponents 7/50 and 2/25), where it returns pow_ctrl's bits.
   __device__ static inline double pw(double x, double y) { return sdeh_math::pow_ctrl(x, y); }
-  __device__ static inline Log plog(double x) { return sdeh_math::pow_log_ctrl(x); }
-  __device__ static inline double pw_from(const Log& l, double y) {
-    return sdeh_math::pow_from_ctrl(l, y);
+  template <class Tab>
+  __device__ static inline Log plog(double x, const Tab& tab) {
+    return sdeh_math::pow_log_ctrl(x, tab);
+  }
+  template <class Tab>
+  __device__ static inline double pw_from(const Log& l, double y, const Tab& tab) {
+    return sdeh_math::pow_from_ctrl(l, y, tab);
   }
 
   // Division and square root with the range handling of the IEEE sequences left
@@ -133,9 +137,47 @@ struct Ops<float> {
   __device__ static inline float pw(float x, float y) {
     return __builtin_amdgcn_exp2f(y * __builtin_amdgcn_logf(x));
   }
-  __device__ static inline Log plog(float x) { return __builtin_amdgcn_logf(x); }
-  __device__ static inline float pw_from(Log l, float y) { return __builtin_amdgcn_exp2f(y * l); }
+  template <class Tab>
+  __device__ static inline Log plog(float x, const Tab&) { return __builtin_amdgcn_logf(x); }
+  template <class Tab>
+  __device__ static inline float pw_from(Log l, float y, const Tab&) {
+    return __builtin_amdgcn_exp2f(y * l);
+  }
 };
+
+// The reduction tables of the binary64 controller's pow in LDS, one array per column
+// (5 KB per block, copied when the kernel starts; every thread of the block calls init).
+// Each attempt gathers three rows at 64 unrelated indices, one after the other: @TAB@
+struct LdsTab {
+  const double* t;
+  __device__ void log_row(int i, double* invc, double* lh, double* ll) const {
+    *invc = t[i];
+    *lh = t[128 + i];
+    *ll = t[256 + i];
+  }
+  __device__ void exp_row(int j, double* th, double* tl) const {
+    *th = t[384 + j];
+    *tl = t[512 + j];
+  }
+  __device__ static LdsTab init() {
+    __shared__ double t[640];
+    for (unsigned i = threadIdx.x; i < 128; i += blockDim.x) {
+      t[i] = sdeh_powtab::LOG_TAB[i][0];
+      t[128 + i] = sdeh_powtab::LOG_TAB[i][1];
+      t[256 + i] = sdeh_powtab::LOG_TAB[i][2];
+      t[384 + i] = sdeh_powtab::EXP_TAB[i][0];
+      t[512 + i] = sdeh_powtab::EXP_TAB[i][1];
+    }
+    __syncthreads();
+    return LdsTab{t};
+  }
+};
+// The tables of a kernel: in LDS where ON (binary64), else the constant arrays.
+template <bool ON>
+__device__ __forceinline__ auto pow_tables() {
+  if constexpr (ON) return LdsTab::init();
+  else return sdeh_math::ConstTab{};
+}
 
 // ---------------------------------------------------------------------------
 // Lane layout.  A right-hand side type R declares G, its lanes per trajectory.
@@ -407,16 +449,17 @@ __device__ __forceinline__ bool ctrl_in_range(T s, T dt) {
   if constexpr (!Ops<T>::kFast) return false;
   else return s >= T(0x1p-700) && s <= T(0x1p700) && dt <= T(0x1p700);
 }
-template <class T, class R, bool IN>
-__device__ __forceinline__ CtrlOut<T> controller(T s, T dt, T qold_pow, const CtrlK<T>& k) {
+template <class T, class R, bool IN, class Tab>
+__device__ __forceinline__ CtrlOut<T> controller(T s, T dt, T qold_pow, const CtrlK<T>& k,
+                                                 const Tab& tab) {
   constexpr int L = NormLen<R>::value;
   CtrlOut<T> o;
   T x;
   if constexpr (!IN || NormLen<R>::pow2) x = Ops<T>::div(s, T(L));  // a power of 2: exact
   else x = Ops<T>::div_r(s, T(L), k.r_len);
   o.EEst = IN ? Ops<T>::root_in(x) : Ops<T>::root(x);
-  o.lg = Ops<T>::plog(o.EEst);
-  const T q11 = Ops<T>::pw_from(o.lg, k.beta1);
+  o.lg = Ops<T>::plog(o.EEst, tab);
+  const T q11 = Ops<T>::pw_from(o.lg, k.beta1, tab);
   const bool accept = !(o.EEst > T(1));
   const bool zero = (o.EEst == T(0));
   const T num = (accept && zero) ? k.inv_qmax : q11;
@@ -1255,6 +1298,7 @@ __device__ __forceinline__ void adaptive_body_wave(const sdeh_kargs& a) {
           gamma = T(9.0 / 10), qoldinit = T(1.0e-4);
   const T inv_qmax = T(1) / qmax, inv_qmin = T(1) / qmin;
   const T qoldinit_pow = Ops<T>::pw(qoldinit, beta2);
+  const auto tab = pow_tables<sizeof(T) == 8>();
   const T abstol = (T)a.abstol, reltol = (T)a.reltol;
   const CtrlK<T> ck{beta1, inv_qmax, inv_qmin, gamma, Ops<T>::rcp_nr(T(NormLen<R>::value)),
                     Ops<T>::rcp_nr(gamma)};
@@ -1374,10 +1418,10 @@ __device__ __forceinline__ void adaptive_body_wave(const sdeh_kargs& a) {
     const T ssq = err_sumsq<T, R, NWL>(err, uprev, u, abstol, reltol);
     CtrlOut<T> co;
     if constexpr (Ops<T>::kFast) {
-      co = controller<T, R, true>(ssq, dt, qold_pow, ck);
-      if (run && !ctrl_in_range(ssq, dt)) co = controller<T, R, false>(ssq, dt, qold_pow, ck);
+      co = controller<T, R, true>(ssq, dt, qold_pow, ck, tab);
+      if (run && !ctrl_in_range(ssq, dt)) co = controller<T, R, false>(ssq, dt, qold_pow, ck, tab);
     } else {
-      co = controller<T, R, false>(ssq, dt, qold_pow, ck);
+      co = controller<T, R, false>(ssq, dt, qold_pow, ck, tab);
     }
     const T EEst = co.EEst;
 
@@ -1395,7 +1439,7 @@ __device__ __forceinline__ void adaptive_body_wave(const sdeh_kargs& a) {
         ++nrej;
       } else {
         qold = sdeh_math::fast_max(EEst, qoldinit);  // jl_max: EEst >= 0, not NaN
-        qold_pow = (qold == EEst) ? Ops<T>::pw_from(co.lg, beta2) : qoldinit_pow;
+        qold_pow = (qold == EEst) ? Ops<T>::pw_from(co.lg, beta2, tab) : qoldinit_pow;
         dtold = dt;
         const double rem = tf - t - (double)dtold;
         dt = (T)sdeh_math::fast_min((double)fabs(co.dtq), fabs(rem));
@@ -1584,6 +1628,8 @@ __device__ __forceinline__ void adaptive_body(const sdeh_kargs& a) {
           gamma = T(9.0 / 10), qoldinit = T(1.0e-4);
   const T inv_qmax = T(1) / qmax, inv_qmin = T(1) / qmin;
   const T qoldinit_pow = Ops<T>::pw(qoldinit, beta2);
+  // (the runs' buffers leave no LDS for a fourth block of four waves)
+  const auto tab = pow_tables<sizeof(T) == 8 && SAVE != SAVE_RUNS>();
   constexpr bool PIN = sizeof(T) == 8 && SAVE == SAVE_END;
   const T abstol = in_vgpr_if<PIN>((T)a.abstol), reltol = in_vgpr_if<PIN>((T)a.reltol);
   const CtrlK<T> ck{beta1, inv_qmax, inv_qmin, gamma, Ops<T>::rcp_nr(T(NormLen<R>::value)),
@@ -1751,15 +1797,15 @@ __device__ __forceinline__ void adaptive_body(const sdeh_kargs& a) {
         else ssq = err_sumsq<T, R>(err, uprev, u, abstol, reltol);
         const bool in = ctrl_in_range(ssq, dt);
         if (!in && a.err_bare) ssq = err_sumsq<T, R>(err, uprev, u, abstol, reltol);
-        co = controller<T, R, true>(ssq, dt, qold_pow, ck);
-        if (!in) co = controller<T, R, false>(ssq, dt, qold_pow, ck);
+        co = controller<T, R, true>(ssq, dt, qold_pow, ck, tab);
+        if (!in) co = controller<T, R, false>(ssq, dt, qold_pow, ck, tab);
       } else if constexpr (Ops<T>::kFast) {
         const T ssq = err_sumsq<T, R>(err, uprev, u, abstol, reltol);
-        co = controller<T, R, true>(ssq, dt, qold_pow, ck);
-        if (!ctrl_in_range(ssq, dt)) co = controller<T, R, false>(ssq, dt, qold_pow, ck);
+        co = controller<T, R, true>(ssq, dt, qold_pow, ck, tab);
+        if (!ctrl_in_range(ssq, dt)) co = controller<T, R, false>(ssq, dt, qold_pow, ck, tab);
       } else {
         const T ssq = err_sumsq<T, R>(err, uprev, u, abstol, reltol);
-        co = controller<T, R, false>(ssq, dt, qold_pow, ck);
+        co = controller<T, R, false>(ssq, dt, qold_pow, ck, tab);
       }
       const T EEst = co.EEst;
       if (EEst != EEst) {
@@ -1774,7 +1820,7 @@ __device__ __forceinline__ void adaptive_body(const sdeh_kargs& a) {
           ++nrej;
         } else {
           qold = sdeh_math::fast_max(EEst, qoldinit);  // jl_max: EEst >= 0, not NaN
-          qold_pow = (qold == EEst) ? Ops<T>::pw_from(co.lg, beta2) : qoldinit_pow;
+          qold_pow = (qold == EEst) ? Ops<T>::pw_from(co.lg, beta2, tab) : qoldinit_pow;
           const T dtold = dt;
           const double rem = tf - t - (double)dtold;
           // Julia's min: neither argument is NaN here (dtq is dt / q with q in
@@ -1890,6 +1936,7 @@ __device__ __forceinline__ void adaptive_body_multi(const sdeh_kargs& a) {
           gamma = T(9.0 / 10), qoldinit = T(1.0e-4);
   const T inv_qmax = T(1) / qmax, inv_qmin = T(1) / qmin;
   const T qoldinit_pow = Ops<T>::pw(qoldinit, beta2);
+  const auto tab = pow_tables<sizeof(T) == 8>();
   const T abstol = (T)a.abstol, reltol = (T)a.reltol;
   const CtrlK<T> ck{beta1, inv_qmax, inv_qmin, gamma, Ops<T>::rcp_nr(T(NormLen<R>::value)),
                     Ops<T>::rcp_nr(gamma)};
@@ -2003,14 +2050,14 @@ __device__ __forceinline__ void adaptive_body_multi(const sdeh_kargs& a) {
 #pragma unroll
       for (int c = 0; c < N; ++c) err[k][c] = dt[k] * err[k][c];
       ssq[k] = err_sumsq<T, R>(err[k], uprev[k], u[k], abstol, reltol);
-      if constexpr (Ops<T>::kFast) co[k] = controller<T, R, true>(ssq[k], dt[k], qold_pow[k], ck);
-      else co[k] = controller<T, R, false>(ssq[k], dt[k], qold_pow[k], ck);
+      if constexpr (Ops<T>::kFast) co[k] = controller<T, R, true>(ssq[k], dt[k], qold_pow[k], ck, tab);
+      else co[k] = controller<T, R, false>(ssq[k], dt[k], qold_pow[k], ck, tab);
     }
     if constexpr (Ops<T>::kFast) {
 #pragma unroll
       for (int k = 0; k < TPL; ++k)  // the IEEE controller again where the check fails
         if (go[k] && !ctrl_in_range(ssq[k], dt[k]))
-          co[k] = controller<T, R, false>(ssq[k], dt[k], qold_pow[k], ck);
+          co[k] = controller<T, R, false>(ssq[k], dt[k], qold_pow[k], ck, tab);
     }
     // ---- each attempting slot's decision (gpuatsit5.jl:279-299, gpuvern7.jl:406-426) ----
 #pragma unroll
@@ -2027,7 +2074,7 @@ __device__ __forceinline__ void adaptive_body_multi(const sdeh_kargs& a) {
         continue;
       }
       const T qold = sdeh_math::fast_max(EEst, qoldinit);
-      qold_pow[k] = (qold == EEst) ? Ops<T>::pw_from(co[k].lg, beta2) : qoldinit_pow;
+      qold_pow[k] = (qold == EEst) ? Ops<T>::pw_from(co[k].lg, beta2, tab) : qoldinit_pow;
       const T dtold = dt[k];
       const double rem = tf[k] - t[k] - (double)dtold;
       dt[k] = (T)sdeh_math::fast_min((double)fabs(co[k].dtq), fabs(rem));

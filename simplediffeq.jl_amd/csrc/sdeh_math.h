@@ -99,14 +99,30 @@ SDEH_HD inline T fast_max(T x, T y) { return y > x ? y : x; }
 // (ln2_hi has 42 significant bits, |k| < 2^11).
 // log_norm_dd is the core for a normal x scaled by 2^-kadj (log of x * 2^kadj);
 // log_pos_dd scales subnormal inputs into the normal range first.
-SDEH_HD inline void log_norm_dd(double xs, int kadj, double* hi, double* lo) {
+// `tab` holds the reduction tables (ConstTab: the constant arrays).
+struct ConstTab {
+  SDEH_HD void log_row(int i, double* invc, double* lh, double* ll) const {
+    *invc = sdeh_powtab::LOG_TAB[i][0];
+    *lh = sdeh_powtab::LOG_TAB[i][1];
+    *ll = sdeh_powtab::LOG_TAB[i][2];
+  }
+  SDEH_HD void exp_row(int j, double* th, double* tl) const {
+    *th = sdeh_powtab::EXP_TAB[j][0];
+    *tl = sdeh_powtab::EXP_TAB[j][1];
+  }
+};
+
+template <class Tab = ConstTab>
+SDEH_HD inline void log_norm_dd(double xs, int kadj, double* hi, double* lo,
+                                const Tab& tab = Tab()) {
   using namespace sdeh_powtab;
   const uint64_t ix = bits_of(xs);
   const uint64_t tmp = ix - LOG_OFF;
   const int i = (int)((tmp >> LOG_SHIFT) & (uint64_t)LOG_MASK);
   const int k = (int)((int64_t)tmp >> 52) - kadj;
   const double z = double_of(ix - (tmp & 0xfff0000000000000ULL));
-  const double invc = LOG_TAB[i][0], lh = LOG_TAB[i][1], ll = LOG_TAB[i][2];
+  double invc, lh, ll;
+  tab.log_row(i, &invc, &lh, &ll);
   const double r = fma(z, invc, -1.0);  // exact
   const double dk = (double)k;
   const double a = dk * LN2_HI;  // exact
@@ -152,7 +168,8 @@ SDEH_HD inline void log_pos_dd(double x, double* hi, double* lo) {
 // exp_core returns res and m with e^(zh + zl) = res * 2^m; exp_dd applies 2^m as
 // two exact power-of-two factors so that a subnormal result is rounded by the
 // last multiply only.
-SDEH_HD inline double exp_core(double zc, double zl, int* m_out) {
+template <class Tab = ConstTab>
+SDEH_HD inline double exp_core(double zc, double zl, int* m_out, const Tab& tab = Tab()) {
   using namespace sdeh_powtab;
   const double nd = __builtin_rint(zc * INV_LN2N);
   const int n = (int)nd;
@@ -166,7 +183,8 @@ SDEH_HD inline double exp_core(double zc, double zl, int* m_out) {
   const double em1 = fma(u * u, q, u);
   const int j = n & EXP_MASK;
   const int m = n >> EXP_BITS;  // arithmetic shift: floor(n / 128)
-  const double th = EXP_TAB[j][0], tl = EXP_TAB[j][1];
+  double th, tl;
+  tab.exp_row(j, &th, &tl);
   *m_out = m;
   return th + fma(th, em1, tl);
 }
@@ -224,22 +242,24 @@ SDEH_HD inline double pow_ctrl(double x, double y) { return pow_from(pow_log(x),
 // normal number.  No subnormal input scaling, no range saturation, and 2^m applied
 // as one factor (exact for a normal result).  On that domain the results are
 // pow_ctrl's bit for bit.
-SDEH_HD inline PowLog pow_log_ctrl(double x) {
+template <class Tab = ConstTab>
+SDEH_HD inline PowLog pow_log_ctrl(double x, const Tab& tab = Tab()) {
   const bool nan_or_neg = !(x >= 0.0);
   const bool zero = x == 0.0;
   const bool inf = x == __builtin_inf();
   PowLog r;
   r.is_special = nan_or_neg || zero || inf;
   r.special = zero ? 0.0 : ((x != x || inf) ? x : __builtin_nan(""));
-  log_norm_dd(r.is_special ? 1.0 : x, 0, &r.hi, &r.lo);
+  log_norm_dd(r.is_special ? 1.0 : x, 0, &r.hi, &r.lo, tab);
   return r;
 }
 
-SDEH_HD inline double pow_from_ctrl(const PowLog& l, double y) {
+template <class Tab = ConstTab>
+SDEH_HD inline double pow_from_ctrl(const PowLog& l, double y, const Tab& tab = Tab()) {
   const double ph = y * l.hi;
   const double pl = fma(y, l.hi, -ph) + y * l.lo;
   int m;
-  const double res = exp_core(ph, pl, &m);
+  const double res = exp_core(ph, pl, &m, tab);
   const double v = res * double_of((uint64_t)(m + 1023) << 52);
   return l.is_special ? l.special : v;
 }
