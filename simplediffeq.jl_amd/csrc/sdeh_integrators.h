@@ -86,6 +86,19 @@ struct Ops<double> {
     return sdeh_math::pow_from_ctrl(l, y, tab);
   }
 
+  // max(|a|, |b|) and min(|a|, |b|) of values that are not NaN, one instruction each (a
+  // NaN operand is dropped, not passed on).
+  __device__ static inline double max_abs(double a, double b) {
+    double r;
+    asm("v_max_f64 %0, |%1|, |%2|" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+  }
+  __device__ static inline double min_abs(double a, double b) {
+    double r;
+    asm("v_min_f64 %0, |%1|, |%2|" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+  }
+
   // Division and square root with the range handling of the IEEE sequences left
   // out, for operands the caller has checked.  gfx950 divides binary64 as
   // v_div_scale (twice), Newton's iteration on v_rcp_f64, v_div_fmas and
@@ -128,6 +141,9 @@ template <>
 struct Ops<float> {
   typedef float Log;
   static constexpr bool kFast = false;  // binary32 divides through v_rcp_f32 already
+  __device__ static inline double min_abs(double a, double b) {
+    return sdeh_math::fast_min(fabs(a), fabs(b));
+  }
   __device__ static inline float rcp_nr(float b) { return b; }
   __device__ static inline float div_r(float a, float b, float) { return div(a, b); }
   __device__ static inline float div_in(float a, float b) { return div(a, b); }
@@ -147,7 +163,11 @@ struct Ops<float> {
 
 // The reduction tables of the binary64 controller's pow in LDS, one array per column
 // (5 KB per block, copied when the kernel starts; every thread of the block calls init).
-// Each attempt gathers three rows at 64 unrelated indices, one after the other: @TAB@
+// Each attempt gathers three rows at 64 unrelated indices, one after the other.  From
+// constant memory those gathers went through the vector L1, which was busy as long as the
+// arithmetic was.  Lorenz, from constant memory / from LDS: 2^20 ATsit5 1,042 / 980 us,
+// 2^22 ATsit5 over spans 4,294 / 4,003 us, 2^20 uneven AVern7 9,997 / 9,428 us, 1,024 ATsit5
+// 37.7 / 35.0 us.
 struct LdsTab {
   const double* t;
   __device__ void log_row(int i, double* invc, double* lh, double* ll) const {
@@ -394,6 +414,11 @@ __device__ __forceinline__ T err_sumsq(T (&tmp)[R::N], const T (&uprev)[R::N],
 // the same operations.  |t| < 2^-540 (or e = 0): both quotients square to +0.
 // |t| > 2^350 (or e Inf or NaN): the bare quotient is at least 2^349, Inf or NaN, so
 // the returned sum leaves the range and the caller computes err_sumsq instead.
+// The larger magnitude by v_max_f64, which drops a NaN u.  u is NaN only if uprev is not
+// finite or one of the k_j in it is Inf or NaN: the sum of b_j k_j is a chain of fused
+// operations, which overflows to an Inf that a later finite term leaves as it is.  With
+// uprev Inf the quotient is NaN, and every k_j of u also has a nonzero weight in e, so
+// in each case the sum leaves the range.
 template <class T, class R>
 __device__ __forceinline__ T err_sumsq_in(const T (&e)[R::N], const T (&uprev)[R::N],
                                           const T (&u)[R::N], T abstol, T reltol) {
@@ -401,8 +426,7 @@ __device__ __forceinline__ T err_sumsq_in(const T (&e)[R::N], const T (&uprev)[R
   T s = T(0);
 #pragma unroll
   for (int c = 0; c < R::N; ++c) {
-    const T au = fabs(u[c]), ap = fabs(uprev[c]);
-    const T m = au < ap ? ap : au;
+    const T m = Ops<T>::max_abs(u[c], uprev[c]);
     const T t = Ops<T>::div_in(e[c], fma(m, reltol, abstol));
     s = c == 0 ? t * t : s + t * t;
   }
@@ -424,53 +448,93 @@ struct NormLen {
 // dt / clamp((q11/qold^beta2)/gamma) share their three divisions, a reject
 // dividing q11 by 1 (exact), and EEst == 0 dividing inv_qmax by 1.  EEst^beta1 now
 // and EEst^beta2 (the next step's qold^beta2 when qold becomes EEst) share one
-// logarithm, returned in `lg`: same bits as two pow calls.
-//
-// IN: every division and the root go through Ops<T>::div_r / div_in / root_in,
-// valid when s is in [2^-700, 2^700] and dt <= 2^700.  Then EEst is in
-// [2^-351, 2^350], q11 in [2^-50, 2^49], qold^beta2 in [0.47, 1] (qold =
-// max(EEst, 1e-4) of an accepted step, EEst <= 1), q in [1/qmax, 1/qmin] and dt >=
-// the solver's dtmin (>= 1e-14): every numerator lies in [2^-700, 2^700] and every
-// divisor (len, qold^beta2 or 1, gamma, q) in [2^-60, 2^60], the range those need.
-// For other s (0, tiny, huge, Inf, NaN) the IEEE operations run instead and the
-// IN results are discarded; computing them is plain arithmetic (the logarithm's and
-// exponential's table indices are masked to the tables) on any input.
+// logarithm: same bits as two pow calls.
 template <class T>
 struct CtrlK {
-  T beta1, inv_qmax, inv_qmin, gamma, r_len, r_gamma;
+  T beta1, beta2, inv_qmax, inv_qmin, gamma, r_len, r_gamma;
 };
 template <class T>
 struct CtrlOut {
   T EEst, dtq;
-  typename Ops<T>::Log lg;
+  T pow2;                      // EEst^beta2, binary64
+  typename Ops<T>::Log lg;     // EEst's logarithm, binary32
+  // EEst^beta2, of an accepted step
+  template <class Tab>
+  __device__ __forceinline__ T qold_pow(T beta2, const Tab& tab) const {
+    if constexpr (sizeof(T) == 8) return pow2;
+    else return Ops<T>::pw_from(lg, beta2, tab);
+  }
 };
-template <class T>
-__device__ __forceinline__ bool ctrl_in_range(T s, T dt) {
-  if constexpr (!Ops<T>::kFast) return false;
-  else return s >= T(0x1p-700) && s <= T(0x1p700) && dt <= T(0x1p700);
-}
-template <class T, class R, bool IN, class Tab>
+template <class T, class R, class Tab>
 __device__ __forceinline__ CtrlOut<T> controller(T s, T dt, T qold_pow, const CtrlK<T>& k,
                                                  const Tab& tab) {
-  constexpr int L = NormLen<R>::value;
   CtrlOut<T> o;
-  T x;
-  if constexpr (!IN || NormLen<R>::pow2) x = Ops<T>::div(s, T(L));  // a power of 2: exact
-  else x = Ops<T>::div_r(s, T(L), k.r_len);
-  o.EEst = IN ? Ops<T>::root_in(x) : Ops<T>::root(x);
-  o.lg = Ops<T>::plog(o.EEst, tab);
-  const T q11 = Ops<T>::pw_from(o.lg, k.beta1, tab);
+  o.EEst = Ops<T>::root(Ops<T>::div(s, T(NormLen<R>::value)));
+  const typename Ops<T>::Log lg = Ops<T>::plog(o.EEst, tab);
+  const T q11 = Ops<T>::pw_from(lg, k.beta1, tab);
+  if constexpr (sizeof(T) == 8) o.pow2 = Ops<T>::pw_from(lg, k.beta2, tab);
+  else o.lg = lg;
   const bool accept = !(o.EEst > T(1));
   const bool zero = (o.EEst == T(0));
   const T num = (accept && zero) ? k.inv_qmax : q11;
   const T den = (accept && !zero) ? qold_pow : T(1);
-  const T qg = IN ? Ops<T>::div_r(Ops<T>::div_in(num, den), k.gamma, k.r_gamma)
-                  : Ops<T>::div(Ops<T>::div(num, den), k.gamma);
+  const T qg = Ops<T>::div(Ops<T>::div(num, den), k.gamma);
   // With EEst not NaN, q11 and qold^beta2 are finite or +Inf and qg is not NaN:
   // Julia's min (gpuatsit5.jl:287) reduces to one comparison select.
   const T q = accept ? sdeh_math::fast_max(k.inv_qmax, sdeh_math::fast_min(k.inv_qmin, qg))
                      : sdeh_math::fast_min(k.inv_qmin, qg);
-  o.dtq = IN ? Ops<T>::div_in(dt, q) : Ops<T>::div(dt, q);
+  o.dtq = Ops<T>::div(dt, q);
+  return o;
+}
+
+// The same in binary64 for s in [2^-700, 2^700) and dt < 2^700 (ctrl_in_range): every
+// division and the root go through Ops<T>::div_r / div_in / root_in, and EEst, neither 0
+// nor special, through the logarithm and power without special values.  EEst is in
+// [2^-351, 2^350], q11 in [2^-50, 2^49], qold^beta2 in [0.47, 1] (qold = max(EEst, 1e-4)
+// of an accepted step, EEst <= 1), q in [1/qmax, 1/qmin] and dt >= the solver's dtmin (>=
+// 1e-14): every numerator lies in [2^-700, 2^700] and every divisor (len, qold^beta2 or 1,
+// gamma, q) in [2^-60, 2^60], the range those need.  For other s (0, tiny, huge, Inf,
+// NaN) controller() runs instead and this result is discarded; computing it is plain
+// arithmetic (the logarithm's and exponential's table indices are masked to the tables)
+// on any input.
+// These kernels are bound by the vector instructions they issue (the 2^20 Lorenz ATsit5
+// ensemble's first pass ran at the issue rate), so this path was cut to what it needs:
+// no selects for EEst = 0 or special values, 32-bit range checks and bit handling, ldexp,
+// and one-instruction minima and maxima.  Lorenz, before / after: 2^20 ATsit5 988 / 932 us,
+// 2^22 ATsit5 over spans 4,170 / 4,000 us, 2^20 uneven AVern7 9,430 / 9,200 us, 1,024 ATsit5
+// 38.6 / 37.4 us.
+__device__ __forceinline__ unsigned hi_word(double x) {
+  return (unsigned)(sdeh_math::bits_of(x) >> 32);
+}
+template <class T>
+__device__ __forceinline__ bool ctrl_in_range(T s, T dt) {
+  if constexpr (!Ops<T>::kFast) return false;
+  else  // exponent fields: -700 .. 699 of s (positive), below 700 of dt (positive)
+    return hi_word(s) - 0x14300000u < 0x57800000u && hi_word(dt) < 0x6bb00000u;
+}
+template <class T, class R, class Tab>
+__device__ __forceinline__ CtrlOut<T> controller_in(T s, T dt, T qold_pow, const CtrlK<T>& k,
+                                                    const Tab& tab) {
+  static_assert(sizeof(T) == 8, "binary64");
+  CtrlOut<T> o;
+  T x;
+  if constexpr (NormLen<R>::pow2) x = Ops<T>::div(s, T(NormLen<R>::value));  // exact
+  else x = Ops<T>::div_r(s, T(NormLen<R>::value), k.r_len);
+  o.EEst = Ops<T>::root_in(x);
+  T lh, ll;
+  sdeh_math::log_in_dd(o.EEst, &lh, &ll, tab);
+  const T q11 = sdeh_math::pow_in(lh, ll, k.beta1, tab);
+  o.pow2 = sdeh_math::pow_in(lh, ll, k.beta2, tab);
+  const bool accept = o.EEst <= T(1);
+  const T den = accept ? qold_pow : T(1);
+  const T qg = Ops<T>::div_r(Ops<T>::div_in(q11, den), k.gamma, k.r_gamma);
+  // max(inv_qmax, .) on accept only: on reject against a subnormal (inv_qmax's low word),
+  // which every quotient here exceeds
+  const uint64_t lob = sdeh_math::bits_of(k.inv_qmax);
+  const T lo = sdeh_math::double_of((uint64_t)(accept ? (unsigned)(lob >> 32) : 0u) << 32 |
+                                    (lob & 0xffffffffull));
+  const T q = Ops<T>::max_abs(lo, Ops<T>::min_abs(k.inv_qmin, qg));
+  o.dtq = Ops<T>::div_in(dt, q);
   return o;
 }
 
@@ -1300,7 +1364,7 @@ __device__ __forceinline__ void adaptive_body_wave(const sdeh_kargs& a) {
   const T qoldinit_pow = Ops<T>::pw(qoldinit, beta2);
   const auto tab = pow_tables<sizeof(T) == 8>();
   const T abstol = (T)a.abstol, reltol = (T)a.reltol;
-  const CtrlK<T> ck{beta1, inv_qmax, inv_qmin, gamma, Ops<T>::rcp_nr(T(NormLen<R>::value)),
+  const CtrlK<T> ck{beta1, beta2, inv_qmax, inv_qmin, gamma, Ops<T>::rcp_nr(T(NormLen<R>::value)),
                     Ops<T>::rcp_nr(gamma)};
   const T* ps = (const T*)a.ps;
   const int64_t n = a.n;
@@ -1314,7 +1378,7 @@ __device__ __forceinline__ void adaptive_body_wave(const sdeh_kargs& a) {
   for (int c = 0; c < P; ++c) pl[c] = T(0);
   R::template init_lane<T>(pl, ps);  // the wave-wide operands, for every lane
   double t = 0.0, tf = 0.0;
-  T dt = T(1), qold = qoldinit, qold_pow = qoldinit_pow;
+  T dt = T(1), qold_pow = qoldinit_pow;
   int32_t nacc = 0, nrej = 0, cur = 0;
   StepSink<T, N> sk{};
   double ts_next = 0.0;  // save_time(cur)
@@ -1359,7 +1423,6 @@ __device__ __forceinline__ void adaptive_body_wave(const sdeh_kargs& a) {
       t = a.tspan ? a.tspan[traj] : a.t0;
       tf = a.tspan ? a.tspan[n + traj] : a.tf;
       dt = (T)(a.dt0 ? a.dt0[traj] : a.dt);
-      qold = qoldinit;
       qold_pow = qoldinit_pow;
       nacc = nrej = 0;
       attempts = 0;
@@ -1418,12 +1481,11 @@ __device__ __forceinline__ void adaptive_body_wave(const sdeh_kargs& a) {
     const T ssq = err_sumsq<T, R, NWL>(err, uprev, u, abstol, reltol);
     CtrlOut<T> co;
     if constexpr (Ops<T>::kFast) {
-      co = controller<T, R, true>(ssq, dt, qold_pow, ck, tab);
-      if (run && !ctrl_in_range(ssq, dt)) co = controller<T, R, false>(ssq, dt, qold_pow, ck, tab);
+      co = controller_in<T, R>(ssq, dt, qold_pow, ck, tab);
+      if (run && !ctrl_in_range(ssq, dt)) co = controller<T, R>(ssq, dt, qold_pow, ck, tab);
     } else {
-      co = controller<T, R, false>(ssq, dt, qold_pow, ck, tab);
+      co = controller<T, R>(ssq, dt, qold_pow, ck, tab);
     }
-    const T EEst = co.EEst;
 
     // ---- PI controller: accept/reject (gpuatsit5.jl:279-299, gpuvern7.jl:406-426,
     // gpuvern9.jl:575-595) ----
@@ -1432,17 +1494,17 @@ __device__ __forceinline__ void adaptive_body_wave(const sdeh_kargs& a) {
     T dtold = T(0);
     if (run) {
       ++attempts;
-      if (EEst != EEst) {
+      if (co.EEst != co.EEst) {
         ret = RET_NAN;
-      } else if (EEst > T(1)) {
+      } else if (co.EEst > T(1)) {
         dt = co.dtq;
         ++nrej;
       } else {
-        qold = sdeh_math::fast_max(EEst, qoldinit);  // jl_max: EEst >= 0, not NaN
-        qold_pow = (qold == EEst) ? Ops<T>::pw_from(co.lg, beta2, tab) : qoldinit_pow;
+        // qold = max(EEst, qoldinit) (EEst >= 0, not NaN), kept as its power
+        qold_pow = qoldinit > co.EEst ? qoldinit_pow : co.qold_pow(beta2, tab);
         dtold = dt;
         const double rem = tf - t - (double)dtold;
-        dt = (T)sdeh_math::fast_min((double)fabs(co.dtq), fabs(rem));
+        dt = (T)Ops<T>::min_abs((double)co.dtq, rem);
         told = t;
         t = (rem < SNAP) ? tf : t + (double)dtold;
         ++nacc;
@@ -1632,7 +1694,7 @@ __device__ __forceinline__ void adaptive_body(const sdeh_kargs& a) {
   const auto tab = pow_tables<sizeof(T) == 8 && SAVE != SAVE_RUNS>();
   constexpr bool PIN = sizeof(T) == 8 && SAVE == SAVE_END;
   const T abstol = in_vgpr_if<PIN>((T)a.abstol), reltol = in_vgpr_if<PIN>((T)a.reltol);
-  const CtrlK<T> ck{beta1, inv_qmax, inv_qmin, gamma, Ops<T>::rcp_nr(T(NormLen<R>::value)),
+  const CtrlK<T> ck{beta1, beta2, inv_qmax, inv_qmin, gamma, Ops<T>::rcp_nr(T(NormLen<R>::value)),
                     Ops<T>::rcp_nr(gamma)};
   const T* ps = (const T*)a.ps;
   const int64_t n = a.n;
@@ -1640,7 +1702,7 @@ __device__ __forceinline__ void adaptive_body(const sdeh_kargs& a) {
   // Lane state.
   T uprev[N], comp[N], fsal[N], pl[P];
   double t = 0.0, tf = 0.0;
-  T dt = T(0), qold = T(0), qold_pow = T(0);
+  T dt = T(0), qold_pow = T(0);
   int32_t nacc = 0, nrej = 0, cur = 0;
   constexpr bool RUNS = SAVE == SAVE_RUNS, STEPS = RUNS || SAVE == SAVE_STEPS;
   static_assert(!RUNS || PkWave<T, R>::value, "runs of a small state");
@@ -1716,7 +1778,6 @@ __device__ __forceinline__ void adaptive_body(const sdeh_kargs& a) {
       fresh = false;
       note_visit(a, traj);
       Park::load(a, traj, uprev, fsal, comp, pl, t, tf, dt, qold_pow, nacc, nrej);
-      qold = qoldinit;  // written before it is read again
       attempts = (int64_t)nacc + nrej;
       cur = 0;
     }
@@ -1730,7 +1791,6 @@ __device__ __forceinline__ void adaptive_body(const sdeh_kargs& a) {
       t = a.tspan ? a.tspan[traj] : a.t0;
       tf = a.tspan ? a.tspan[n + traj] : a.tf;
       dt = (T)(a.dt0 ? a.dt0[traj] : a.dt);
-      qold = qoldinit;
       qold_pow = qoldinit_pow;
       nacc = nrej = 0;
       attempts = 0;
@@ -1797,35 +1857,29 @@ __device__ __forceinline__ void adaptive_body(const sdeh_kargs& a) {
         else ssq = err_sumsq<T, R>(err, uprev, u, abstol, reltol);
         const bool in = ctrl_in_range(ssq, dt);
         if (!in && a.err_bare) ssq = err_sumsq<T, R>(err, uprev, u, abstol, reltol);
-        co = controller<T, R, true>(ssq, dt, qold_pow, ck, tab);
-        if (!in) co = controller<T, R, false>(ssq, dt, qold_pow, ck, tab);
+        co = controller_in<T, R>(ssq, dt, qold_pow, ck, tab);
+        if (!in) co = controller<T, R>(ssq, dt, qold_pow, ck, tab);
       } else if constexpr (Ops<T>::kFast) {
         const T ssq = err_sumsq<T, R>(err, uprev, u, abstol, reltol);
-        co = controller<T, R, true>(ssq, dt, qold_pow, ck, tab);
-        if (!ctrl_in_range(ssq, dt)) co = controller<T, R, false>(ssq, dt, qold_pow, ck, tab);
+        co = controller_in<T, R>(ssq, dt, qold_pow, ck, tab);
+        if (!ctrl_in_range(ssq, dt)) co = controller<T, R>(ssq, dt, qold_pow, ck, tab);
       } else {
         const T ssq = err_sumsq<T, R>(err, uprev, u, abstol, reltol);
-        co = controller<T, R, false>(ssq, dt, qold_pow, ck, tab);
+        co = controller<T, R>(ssq, dt, qold_pow, ck, tab);
       }
-      const T EEst = co.EEst;
-      if (EEst != EEst) {
-        ret = RET_NAN;
-      } else {
-        // ---- PI controller: accept/reject (gpuatsit5.jl:279-299,
-        // gpuvern7.jl:406-426, gpuvern9.jl:575-595) ----
-        const bool accept = !(EEst > T(1));
-        const T dtq = co.dtq;
-        if (!accept) {
-          dt = dtq;
-          ++nrej;
-        } else {
-          qold = sdeh_math::fast_max(EEst, qoldinit);  // jl_max: EEst >= 0, not NaN
-          qold_pow = (qold == EEst) ? Ops<T>::pw_from(co.lg, beta2, tab) : qoldinit_pow;
-          const T dtold = dt;
+      // ---- PI controller: accept/reject (gpuatsit5.jl:279-299, gpuvern7.jl:406-426,
+      // gpuvern9.jl:575-595).  The accepted step's block stands first, for what it
+      // carries to the next attempt to stay in place. ----
+      {
+        const T dtold = dt;
+        dt = co.dtq;
+        if (co.EEst <= T(1)) {
+          // qold = max(EEst, qoldinit) (EEst >= 0, not NaN), kept as its power
+          qold_pow = qoldinit > co.EEst ? qoldinit_pow : co.qold_pow(beta2, tab);
           const double rem = tf - t - (double)dtold;
           // Julia's min: neither argument is NaN here (dtq is dt / q with q in
-          // [1/qmax, 1/qmin]; t and tf are finite or tf = +Inf), so one select.
-          dt = (T)sdeh_math::fast_min((double)fabs(dtq), fabs(rem));
+          // [1/qmax, 1/qmin]; t and tf are finite or tf = +Inf), so one minimum.
+          dt = (T)Ops<T>::min_abs((double)co.dtq, rem);
           const double told = t;
           t = (rem < SNAP) ? tf : t + (double)dtold;
           ++nacc;
@@ -1875,6 +1929,10 @@ __device__ __forceinline__ void adaptive_body(const sdeh_kargs& a) {
           if constexpr (ALG == ALG_ATSIT5) copyv(fsal, k7);
           if constexpr (KAHAN) copyv(comp, comp_new);
           if (!(t < tf)) ret = RET_DEFAULT;
+        } else if (co.EEst > T(1)) {
+          ++nrej;
+        } else {
+          ret = RET_NAN;
         }
       }
     }
@@ -1938,7 +1996,7 @@ __device__ __forceinline__ void adaptive_body_multi(const sdeh_kargs& a) {
   const T qoldinit_pow = Ops<T>::pw(qoldinit, beta2);
   const auto tab = pow_tables<sizeof(T) == 8>();
   const T abstol = (T)a.abstol, reltol = (T)a.reltol;
-  const CtrlK<T> ck{beta1, inv_qmax, inv_qmin, gamma, Ops<T>::rcp_nr(T(NormLen<R>::value)),
+  const CtrlK<T> ck{beta1, beta2, inv_qmax, inv_qmin, gamma, Ops<T>::rcp_nr(T(NormLen<R>::value)),
                     Ops<T>::rcp_nr(gamma)};
   const T* ps = (const T*)a.ps;
   const int64_t n = a.n;
@@ -2050,34 +2108,32 @@ __device__ __forceinline__ void adaptive_body_multi(const sdeh_kargs& a) {
 #pragma unroll
       for (int c = 0; c < N; ++c) err[k][c] = dt[k] * err[k][c];
       ssq[k] = err_sumsq<T, R>(err[k], uprev[k], u[k], abstol, reltol);
-      if constexpr (Ops<T>::kFast) co[k] = controller<T, R, true>(ssq[k], dt[k], qold_pow[k], ck, tab);
-      else co[k] = controller<T, R, false>(ssq[k], dt[k], qold_pow[k], ck, tab);
+      if constexpr (Ops<T>::kFast) co[k] = controller_in<T, R>(ssq[k], dt[k], qold_pow[k], ck, tab);
+      else co[k] = controller<T, R>(ssq[k], dt[k], qold_pow[k], ck, tab);
     }
     if constexpr (Ops<T>::kFast) {
 #pragma unroll
       for (int k = 0; k < TPL; ++k)  // the IEEE controller again where the check fails
         if (go[k] && !ctrl_in_range(ssq[k], dt[k]))
-          co[k] = controller<T, R, false>(ssq[k], dt[k], qold_pow[k], ck, tab);
+          co[k] = controller<T, R>(ssq[k], dt[k], qold_pow[k], ck, tab);
     }
     // ---- each attempting slot's decision (gpuatsit5.jl:279-299, gpuvern7.jl:406-426) ----
 #pragma unroll
     for (int k = 0; k < TPL; ++k) {
       if (!go[k]) continue;
-      const T EEst = co[k].EEst;
-      if (EEst != EEst) {
+      if (co[k].EEst != co[k].EEst) {
         ret[k] = RET_NAN;
         continue;
       }
-      if (EEst > T(1)) {
+      if (co[k].EEst > T(1)) {
         dt[k] = co[k].dtq;
         ++nrej[k];
         continue;
       }
-      const T qold = sdeh_math::fast_max(EEst, qoldinit);
-      qold_pow[k] = (qold == EEst) ? Ops<T>::pw_from(co[k].lg, beta2, tab) : qoldinit_pow;
+      qold_pow[k] = qoldinit > co[k].EEst ? qoldinit_pow : co[k].qold_pow(beta2, tab);
       const T dtold = dt[k];
       const double rem = tf[k] - t[k] - (double)dtold;
-      dt[k] = (T)sdeh_math::fast_min((double)fabs(co[k].dtq), fabs(rem));
+      dt[k] = (T)Ops<T>::min_abs((double)co[k].dtq, rem);
       t[k] = (rem < SNAP) ? tf[k] : t[k] + (double)dtold;
       ++nacc[k];
       copyv(uprev[k], u[k]);

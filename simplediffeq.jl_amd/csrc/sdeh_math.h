@@ -112,15 +112,11 @@ struct ConstTab {
   }
 };
 
-template <class Tab = ConstTab>
-SDEH_HD inline void log_norm_dd(double xs, int kadj, double* hi, double* lo,
-                                const Tab& tab = Tab()) {
+// The logarithm from its reduction: x = 2^k z, subinterval i of z.
+template <class Tab>
+SDEH_HD inline void log_reduced_dd(int i, int k, double z, double* hi, double* lo,
+                                   const Tab& tab) {
   using namespace sdeh_powtab;
-  const uint64_t ix = bits_of(xs);
-  const uint64_t tmp = ix - LOG_OFF;
-  const int i = (int)((tmp >> LOG_SHIFT) & (uint64_t)LOG_MASK);
-  const int k = (int)((int64_t)tmp >> 52) - kadj;
-  const double z = double_of(ix - (tmp & 0xfff0000000000000ULL));
   double invc, lh, ll;
   tab.log_row(i, &invc, &lh, &ll);
   const double r = fma(z, invc, -1.0);  // exact
@@ -153,6 +149,18 @@ SDEH_HD inline void log_norm_dd(double xs, int kadj, double* hi, double* lo,
   const double y = h + t;
   *hi = y;
   *lo = (h - y) + t;
+}
+
+template <class Tab = ConstTab>
+SDEH_HD inline void log_norm_dd(double xs, int kadj, double* hi, double* lo,
+                                const Tab& tab = Tab()) {
+  using namespace sdeh_powtab;
+  const uint64_t ix = bits_of(xs);
+  const uint64_t tmp = ix - LOG_OFF;
+  const int i = (int)((tmp >> LOG_SHIFT) & (uint64_t)LOG_MASK);
+  const int k = (int)((int64_t)tmp >> 52) - kadj;
+  const double z = double_of(ix - (tmp & 0xfff0000000000000ULL));
+  log_reduced_dd(i, k, z, hi, lo, tab);
 }
 
 SDEH_HD inline void log_pos_dd(double x, double* hi, double* lo) {
@@ -262,6 +270,32 @@ SDEH_HD inline double pow_from_ctrl(const PowLog& l, double y, const Tab& tab = 
   const double res = exp_core(ph, pl, &m, tab);
   const double v = res * double_of((uint64_t)(m + 1023) << 52);
   return l.is_special ? l.special : v;
+}
+
+// log_norm_dd of a normal finite x > 0, its bit pattern taken apart in 32-bit words (the
+// same index, exponent and z: LOG_OFF's low word is 0): the controller's logarithm where
+// its argument is known to be in range.
+template <class Tab>
+SDEH_HD inline void log_in_dd(double x, double* hi, double* lo, const Tab& tab) {
+  using namespace sdeh_powtab;
+  static_assert((LOG_OFF & 0xffffffffULL) == 0 && LOG_SHIFT >= 32, "32-bit words");
+  const uint64_t ix = bits_of(x);
+  const uint32_t xh = (uint32_t)(ix >> 32), th = xh - (uint32_t)(LOG_OFF >> 32);
+  const int i = (int)((th >> (LOG_SHIFT - 32)) & (uint32_t)LOG_MASK);
+  const int k = (int)th >> 20;
+  const double z = double_of((uint64_t)(xh - (th & 0xfff00000u)) << 32 | (ix & 0xffffffffULL));
+  log_reduced_dd(i, k, z, hi, lo, tab);
+}
+
+// pow_from_ctrl of log_in_dd's result: no special values, and 2^m by ldexp (the result is
+// normal, so the scaling is exact and the bits are the same).
+template <class Tab>
+SDEH_HD inline double pow_in(double hi, double lo, double y, const Tab& tab) {
+  const double ph = y * hi;
+  const double pl = fma(y, hi, -ph) + y * lo;
+  int m;
+  const double res = exp_core(ph, pl, &m, tab);
+  return __builtin_ldexp(res, m);
 }
 
 }  // namespace sdeh_math
