@@ -936,6 +936,36 @@ __device__ __forceinline__ void store_save(const sdeh_kargs& a, void* base, int6
   for (int c = 0; c < R::N; ++c) o[comp_idx<R>(c)] = u[c];
 }
 
+// This lane's place in row `row` of a saved-state output, the step from a row to the next
+// and the store of its components there, for the wave layout's runs of rows: AVern9's kernel
+// is short of registers, kept the trajectory's base address in scratch memory and reloaded
+// it for each row, and a reload waits for the stores of the rows before it (GLV-16, 2^17
+// trajectories, 256 points: 7,405 us so, 7,235 us with the place advanced row by row).  (The
+// one-lane kernels keep store_save: there the compiler merges a row's components into wide
+// stores, which it does not do here.)
+template <class T, class R>
+__device__ __forceinline__ T* save_row(const sdeh_kargs& a, void* base, int64_t row, int64_t rows,
+                                       int64_t traj) {
+  constexpr int FULL = R::N * R::G;
+  asm volatile("" : "+v"(traj));  // computed here, not kept from the trajectory's start
+  return (T*)base + (a.traj_major ? (traj * rows + row) * FULL + comp_idx<R>(0)
+                                  : (row * FULL + comp_idx<R>(0)) * a.n + traj);
+}
+template <class T, class R>
+__device__ __forceinline__ T* next_row(const sdeh_kargs& a, T* at) {
+  constexpr int FULL = R::N * R::G;
+  return at + (a.traj_major ? (int64_t)FULL : FULL * a.n);
+}
+template <class T, class R>
+__device__ __forceinline__ void store_row(const sdeh_kargs& a, T* at, const T (&u)[R::N]) {
+#pragma unroll
+  for (int c = 0; c < R::N; ++c) {
+    const int d = IsWave<R>::value ? R::G * c : c;
+    if (a.traj_major) at[d] = u[c];
+    else at[d * a.n] = u[c];
+  }
+}
+
 // saveat: NaN in the rows a trajectory ended before (from `row` on), written when it
 // ends.  Filling the whole output beforehand moved every byte of it twice: GLV-16, 2^17
 // trajectories, 256 points, the fill alone took 404 us of 1,437 in binary32 (2.1 GB) and
@@ -1557,6 +1587,11 @@ __device__ __forceinline__ void adaptive_body_wave(const sdeh_kargs& a) {
         const bool saves = stepped && cur < a.n_saveat && ts_next <= t;
         if (__ballot(saves) != 0ull) {
           if constexpr (V9) {
+            // u is not needed before the step is done: it waits in LDS rather than in the
+            // registers that the extra stages' vectors need (7,235 to 7,155 us as above)
+            __shared__ T upark[256 * N];
+#pragma unroll
+            for (int c = 0; c < N; ++c) upark[threadIdx.x + 256 * c] = u[c];
             T x[10][N];
             vern9_extra<T, R>(uprev, S9, x, pl, ps, told, dtold);  // told + c*dtold
             if (saves) {
@@ -1566,6 +1601,7 @@ __device__ __forceinline__ void adaptive_body_wave(const sdeh_kargs& a) {
               // point in order.  Same values as vern9_dense point by point.
               constexpr int PB = R::G;
               T* wl = wave_lds<T, NWL>() + (lane & (SLOTS - 1)) * DWS;
+              T* row = save_row<T, R>(a, a.u_saveat, cur, a.n_saveat, traj);
               const int q = lane_comp<R>();
               while (cur < a.n_saveat && ts_next <= t) {
                 const int64_t pq = cur + q;
@@ -1584,12 +1620,15 @@ __device__ __forceinline__ void adaptive_body_wave(const sdeh_kargs& a) {
                   const T(&wm)[V9W] = *reinterpret_cast<const T(*)[V9W]>(wl + m * V9W);
                   T o[N];
                   vern9_combine(o, uprev, dtold, wm, S9, x);
-                  store_save<T, R>(a, a.u_saveat, cur, a.n_saveat, traj, o);
+                  store_row<T, R>(a, row, o);
+                  row = next_row<T, R>(a, row);
                   ++cur;
                   ts_next = saves_at.at(a, cur);
                 }
               }
             }
+#pragma unroll
+            for (int c = 0; c < N; ++c) u[c] = upark[threadIdx.x + 256 * c];
           } else {
             T x[6][N];
             // Quirk (gpuvern7.jl:449): stage times from the post-step t.
