@@ -593,13 +593,11 @@ __device__ __forceinline__ void tsit5_stages(const T (&uprev)[R::N], const T (&k
   R::f(k7, u, p, ps, t + (double)dt);
 }
 
-// Tsit5 dense output (tsit5.jl:385-399 weights) at θ over (uprev, h).
-template <class T, int N>
-__device__ __forceinline__ void tsit5_dense(T (&out)[N], const T (&uprev)[N], T h, T th,
-                                            const T (&k1)[N], const T (&k2)[N],
-                                            const T (&k3)[N], const T (&k4)[N],
-                                            const T (&k5)[N], const T (&k6)[N],
-                                            const T (&k7)[N]) {
+// Tsit5 dense output (tsit5.jl:385-399): the 7 weights of θ, then out = uprev + h * (w_1 k1 +
+// ... + w_7 k7).
+constexpr int T5W = 7;
+template <class T>
+__device__ __forceinline__ void tsit5_weights(T th, T (&w)[T5W]) {
   const T r1[4] = {TS(r11), TS(r12), TS(r13), TS(r14)};
   const T r2[3] = {TS(r22), TS(r23), TS(r24)};
   const T r3[3] = {TS(r32), TS(r33), TS(r34)};
@@ -607,8 +605,19 @@ __device__ __forceinline__ void tsit5_dense(T (&out)[N], const T (&uprev)[N], T 
   const T r5[3] = {TS(r52), TS(r53), TS(r54)};
   const T r6[3] = {TS(r62), TS(r63), TS(r64)};
   const T r7[3] = {TS(r72), TS(r73), TS(r74)};
-  comb(out, uprev, h, poly1(th, r1), k1, poly2(th, r2), k2, poly2(th, r3), k3, poly2(th, r4),
-       k4, poly2(th, r5), k5, poly2(th, r6), k6, poly2(th, r7), k7);
+  w[0] = poly1(th, r1);
+  w[1] = poly2(th, r2); w[2] = poly2(th, r3); w[3] = poly2(th, r4);
+  w[4] = poly2(th, r5); w[5] = poly2(th, r6); w[6] = poly2(th, r7);
+}
+template <class T, int N>
+__device__ __forceinline__ void tsit5_dense(T (&out)[N], const T (&uprev)[N], T h, T th,
+                                            const T (&k1)[N], const T (&k2)[N],
+                                            const T (&k3)[N], const T (&k4)[N],
+                                            const T (&k5)[N], const T (&k6)[N],
+                                            const T (&k7)[N]) {
+  T w[T5W];
+  tsit5_weights(th, w);
+  comb(out, uprev, h, w[0], k1, w[1], k2, w[2], k3, w[3], k4, w[4], k5, w[5], k6, w[6], k7);
 }
 #undef TS
 
@@ -943,12 +952,54 @@ __device__ __forceinline__ void store_save(const sdeh_kargs& a, void* base, int6
 // trajectories, 256 points: 7,405 us so, 7,235 us with the place advanced row by row).  (The
 // one-lane kernels keep store_save: there the compiler merges a row's components into wide
 // stores, which it does not do here.)
+//
+// Trajectory-major binary32 rows of four lanes with four components each are transposed:
+// lane q, which holds components q, q + 4, q + 8, q + 12, gets 4q .. 4q + 3, stored at
+// once, so that one store instruction writes a trajectory's 64-byte row end to end: with
+// shared weights 1,005 to 850 us for GLV-16 ATsit5, 2^17 trajectories, 256 points.  (binary64
+// rows, whose stores already write 32 bytes in a piece, lost by it: AVern9 7,150 / 7,250 us.)
+template <class T, class R>
+struct RowTr {  // the row's transpose: 4 x 4 over lanes 16 apart
+  static constexpr bool value = sizeof(T) == 4 && IsWave<R>::value && R::G == 4 && R::N == 4;
+};
+__device__ __forceinline__ void transpose4(unsigned (&r)[4]) {
+  const auto a = __builtin_amdgcn_permlane16_swap(r[0], r[1], false, false);
+  const auto b = __builtin_amdgcn_permlane16_swap(r[2], r[3], false, false);
+  const auto c = __builtin_amdgcn_permlane32_swap(a[0], b[0], false, false);
+  const auto d = __builtin_amdgcn_permlane32_swap(a[1], b[1], false, false);
+  r[0] = c[0];
+  r[1] = d[0];
+  r[2] = c[1];
+  r[3] = d[1];
+}
+__device__ __forceinline__ void transpose4(float (&u)[4]) {
+  unsigned r[4];
+#pragma unroll
+  for (int c = 0; c < 4; ++c) r[c] = __builtin_bit_cast(unsigned, u[c]);
+  transpose4(r);
+#pragma unroll
+  for (int c = 0; c < 4; ++c) u[c] = __builtin_bit_cast(float, r[c]);
+}
+__device__ __forceinline__ void transpose4(double (&u)[4]) {
+  unsigned lo[4], hi[4];
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    const uint64_t b = __builtin_bit_cast(uint64_t, u[c]);
+    lo[c] = (unsigned)b;
+    hi[c] = (unsigned)(b >> 32);
+  }
+  transpose4(lo);
+  transpose4(hi);
+#pragma unroll
+  for (int c = 0; c < 4; ++c) u[c] = __builtin_bit_cast(double, (uint64_t)hi[c] << 32 | lo[c]);
+}
 template <class T, class R>
 __device__ __forceinline__ T* save_row(const sdeh_kargs& a, void* base, int64_t row, int64_t rows,
                                        int64_t traj) {
   constexpr int FULL = R::N * R::G;
   asm volatile("" : "+v"(traj));  // computed here, not kept from the trajectory's start
-  return (T*)base + (a.traj_major ? (traj * rows + row) * FULL + comp_idx<R>(0)
+  const int c0 = RowTr<T, R>::value ? lane_comp<R>() * R::N : comp_idx<R>(0);
+  return (T*)base + (a.traj_major ? (traj * rows + row) * FULL + c0
                                   : (row * FULL + comp_idx<R>(0)) * a.n + traj);
 }
 template <class T, class R>
@@ -958,6 +1009,15 @@ __device__ __forceinline__ T* next_row(const sdeh_kargs& a, T* at) {
 }
 template <class T, class R>
 __device__ __forceinline__ void store_row(const sdeh_kargs& a, T* at, const T (&u)[R::N]) {
+  if (RowTr<T, R>::value && a.traj_major) {
+    T w[R::N];
+#pragma unroll
+    for (int c = 0; c < R::N; ++c) w[c] = u[c];
+    if constexpr (RowTr<T, R>::value) transpose4(w);
+#pragma unroll
+    for (int c = 0; c < R::N; ++c) at[c] = w[c];
+    return;
+  }
 #pragma unroll
   for (int c = 0; c < R::N; ++c) {
     const int d = IsWave<R>::value ? R::G * c : c;
@@ -975,7 +1035,12 @@ __device__ __forceinline__ void save_unreached(const sdeh_kargs& a, int64_t row,
   T x[R::N];
 #pragma unroll
   for (int c = 0; c < R::N; ++c) x[c] = (T)__builtin_nan("");
-  for (; row < a.n_saveat; ++row) store_save<T, R>(a, a.u_saveat, row, a.n_saveat, traj, x);
+  if constexpr (RowTr<T, R>::value) {
+    T* at = save_row<T, R>(a, a.u_saveat, row, a.n_saveat, traj);
+    for (; row < a.n_saveat; ++row, at = next_row<T, R>(a, at)) store_row<T, R>(a, at, x);
+  } else {
+    for (; row < a.n_saveat; ++row) store_save<T, R>(a, a.u_saveat, row, a.n_saveat, traj, x);
+  }
 }
 
 __device__ __forceinline__ void store_save_time(const sdeh_kargs& a, int64_t row, int64_t traj,
@@ -1387,6 +1452,23 @@ struct SaveTimes<false> {
   __device__ static SaveTimes init(const sdeh_kargs&) { return {}; }
 };
 
+// Dense output in the wave layout: the weights depend on the point only, so the G lanes of
+// a trajectory take G of its points at a time, lane q the weights of point cur + q, and
+// share them through LDS; every lane then forms its components of each point in order.
+// Same values as point by point.  `at`: this lane's place in its trajectory's share.
+// (ATsit5, GLV-16 binary32, shared / each lane its own weights: 2^17 trajectories, 256 points
+// 880 / 970 us; 1,024 trajectories, where the exchange's latency shows, 236 / 228.)
+template <class T, int NW>
+__device__ __forceinline__ void share_weights(T* at, const T (&w)[NW]) {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();  // the previous batch's reads are done
+#pragma unroll
+  for (int i = 0; i < NW; ++i) at[i] = w[i];
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // ---------------------------------------------------------------------------
 // Adaptive solvers: ATsit5, AVern7, AVern9.
 // ---------------------------------------------------------------------------
@@ -1408,9 +1490,9 @@ __device__ __forceinline__ void adaptive_body_wave(const sdeh_kargs& a) {
   // dense-output weights of R::G points per trajectory.  Each trajectory's share is
   // padded to an odd number of values (DWS) so that the wave's trajectories read
   // their weights from different banks.
-  constexpr int DWS = R::G * V9W + 1;
+  constexpr int NW = V9 ? V9W : T5W, DWS = R::G * NW + 1;
   constexpr int NWG = SLOTS * wave_slot_stride<T, R>();
-  constexpr int NWL = (V9 && SAVE == SAVE_AT && SLOTS * DWS > NWG) ? SLOTS * DWS : NWG;
+  constexpr int NWL = ((V9 || ALG == ALG_ATSIT5) && SAVE == SAVE_AT && SLOTS * DWS > NWG) ? SLOTS * DWS : NWG;
   constexpr double DTMIN = V9 ? (double)1.0e-7f : 1.0e-14;  // gpuvern9.jl:466
   constexpr double SNAP = DTMIN;                            // gpuvern9.jl:591
   // build_adaptive_controller_cache(T), src/SimpleDiffEq.jl:67-77
@@ -1570,15 +1652,27 @@ __device__ __forceinline__ void adaptive_body_wave(const sdeh_kargs& a) {
     }
     if constexpr (SAVE == SAVE_AT) {
       if constexpr (ALG == ALG_ATSIT5) {  // gpuatsit5.jl:305-316
-        if (stepped) {
+        const bool saves = stepped && cur < a.n_saveat && ts_next <= t;
+        if (saves) {
+          T* wl = wave_lds<T, NWL>() + (lane & (SLOTS - 1)) * DWS;
+          T* row = save_row<T, R>(a, a.u_saveat, cur, a.n_saveat, traj);
+          const int q = lane_comp<R>();
           while (cur < a.n_saveat && ts_next <= t) {
-            const double ts_after = saves_at.at(a, cur + 1);
-            const T th = (T)((ts_next - told) / (double)dtold);
-            T o[N];
-            tsit5_dense(o, uprev, dtold, th, fsal, k2, k3, k4, k5, k6, k7);
-            store_save<T, R>(a, a.u_saveat, cur, a.n_saveat, traj, o);
-            ++cur;
-            ts_next = ts_after;
+            const int64_t pq = cur + q;
+            const double tq = pq < a.n_saveat ? saves_at.at(a, pq) : ts_next;
+            T w[NW];
+            tsit5_weights((T)((tq - told) / (double)dtold), w);
+            share_weights<T, NW>(wl + q * NW, w);
+            for (int m = 0; m < R::G && cur < a.n_saveat && ts_next <= t; ++m) {
+              const T(&wm)[NW] = *reinterpret_cast<const T(*)[NW]>(wl + m * NW);
+              T o[N];
+              comb(o, uprev, dtold, wm[0], fsal, wm[1], k2, wm[2], k3, wm[3], k4, wm[4], k5, wm[5],
+                   k6, wm[6], k7);
+              store_row<T, R>(a, row, o);
+              row = next_row<T, R>(a, row);
+              ++cur;
+              ts_next = saves_at.at(a, cur);
+            }
           }
         }
       } else {
@@ -1595,29 +1689,18 @@ __device__ __forceinline__ void adaptive_body_wave(const sdeh_kargs& a) {
             T x[10][N];
             vern9_extra<T, R>(uprev, S9, x, pl, ps, told, dtold);  // told + c*dtold
             if (saves) {
-              // The weights depend on the point only: the G lanes of a trajectory take
-              // G of its points at a time, lane q the weights of point cur + q, and
-              // share them through LDS; every lane then forms its components of each
-              // point in order.  Same values as vern9_dense point by point.
-              constexpr int PB = R::G;
               T* wl = wave_lds<T, NWL>() + (lane & (SLOTS - 1)) * DWS;
               T* row = save_row<T, R>(a, a.u_saveat, cur, a.n_saveat, traj);
               const int q = lane_comp<R>();
               while (cur < a.n_saveat && ts_next <= t) {
                 const int64_t pq = cur + q;
                 const double tq = pq < a.n_saveat ? saves_at.at(a, pq) : ts_next;
-                T w[V9W];
+                T w[NW];
                 vern9_weights((T)((tq - told) / (double)dtold), w);
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                __builtin_amdgcn_wave_barrier();  // the previous batch's reads are done
-#pragma unroll
-                for (int i = 0; i < V9W; ++i) wl[q * V9W + i] = w[i];
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                __builtin_amdgcn_wave_barrier();
-                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-                for (int m = 0; m < PB && cur < a.n_saveat && ts_next <= t; ++m) {
+                share_weights<T, NW>(wl + q * NW, w);
+                for (int m = 0; m < R::G && cur < a.n_saveat && ts_next <= t; ++m) {
                   // the weights are read from LDS where the combination uses them
-                  const T(&wm)[V9W] = *reinterpret_cast<const T(*)[V9W]>(wl + m * V9W);
+                  const T(&wm)[NW] = *reinterpret_cast<const T(*)[NW]>(wl + m * NW);
                   T o[N];
                   vern9_combine(o, uprev, dtold, wm, S9, x);
                   store_row<T, R>(a, row, o);

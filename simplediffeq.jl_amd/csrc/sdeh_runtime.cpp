@@ -380,8 +380,7 @@ int user_kernel(sdeh_ctx* c, int64_t rhs, int alg, int dtype, int save, int kaha
 // in the 16-lane group layout, 10.8 ms in the 4-lane matrix-core layout; endpoint
 // only 4.35 / 2.86 ms.  binary32 ATsit5 fits one lane's registers and runs 1.6x
 // faster there than in the group layout, which repeats the controller on all 16
-// lanes, and 1.5x faster than in the matrix-core layout (1.49 against 2.24 ms with
-// 256 saveat points), which it takes on request only.)
+// lanes; auto_lanes says where it takes the matrix-core layout.)
 int resolve_kernel(sdeh_ctx* c, int64_t rhs, int alg, int dtype, int save, int kahan,
                    int lanes, KernelRef* out, int waves = 0, int tpl = 1) {
   out->waves = 0;
@@ -451,6 +450,25 @@ int resolve_kernel(sdeh_ctx* c, int64_t rhs, int alg, int dtype, int save, int k
     return fail(c, SDEH_E_INVALID, "registered right-hand sides run one lane per trajectory");
   out->lanes = 1;
   return user_kernel(c, rhs, alg, dtype, save, kahan, out, waves, tpl);
+}
+
+// The lanes that `lanes` = 0 stands for: in binary32 the matrix-core layout too, where it has
+// a kernel and nothing that only one lane per trajectory offers is asked for.  Both layouts
+// give the same bits.  One lane | matrix-core layout, GLV-16 ATsit5, tolerances 1e-6 (us):
+//   n             endpoint        11 points       256 points, trajectory-major
+//      1,024     367 |   115     400 |   144     570 |   236
+//    131,072     650 |   450     648 |   528     955 |   880
+//    524,288   1,840 | 1,400   2,037 | 1,733
+// (f32 matrix products run at twice the vector rate and beside it, a wave holds a quarter of
+// the trajectories, and the kernel's 107 registers leave four waves per SIMD instead of two.)
+// An ensemble of at most 64, one wave either way, stays on one lane.
+int auto_lanes(const sdeh_solve_desc* d, int save, int kahan) {
+  if (d->lanes != 0 || d->dtype != SDEH_F32 || d->n_traj <= 64 || d->waves || d->per_lane ||
+      d->schedule == SDEH_SCHED_STAGED)
+    return d->lanes;
+  const Builtin* b = find_builtin(d->rhs);
+  return b && b->mgroup > 1 && b->mgroup_lookup(d->dtype, d->alg, save, kahan, 0, 1) ? b->mgroup
+                                                                                     : 0;
 }
 
 hipError_t launch(const KernelRef& k, int grid, int block, sdeh_kargs* a, hipStream_t s) {
@@ -737,7 +755,8 @@ int plan_solve(sdeh_ctx* c, const sdeh_solve_desc* d, const sdeh_io* io, Plan* p
     a.g_start = g.start;
     a.g_step = g.step;
   }
-  r = resolve_kernel(c, d->rhs, d->alg, d->dtype, pl->save, pl->kahan, d->lanes, &pl->k);
+  r = resolve_kernel(c, d->rhs, d->alg, d->dtype, pl->save, pl->kahan,
+                     auto_lanes(d, pl->save, pl->kahan), &pl->k);
   if (r) return r;
   if (pl->packed && adaptive) {  // the counting pass: the endpoint kernel, same layout
     r = resolve_kernel(c, d->rhs, d->alg, d->dtype, SAVE_END, pl->kahan, pl->k.lanes,
