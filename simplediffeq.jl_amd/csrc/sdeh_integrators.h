@@ -1064,16 +1064,15 @@ __device__ __forceinline__ unsigned lane_rank(unsigned long long mask) {
 // would otherwise write back partly filled).
 //
 // The SAVE_RUNS kernels (adaptive solvers, small states; the host takes them for ensembles
-// beyond what fits the GPU at once) hold their rows in LDS and the wave writes them
-// together (flush_wave), run by run: a run is PK_ROWS output rows
-// that start at a multiple of PK_ROWS, so its 96 bytes of state and 32 of time (three
-// binary64 components) begin on 32-byte boundaries.  What costs is lines written in part:
-// runs of 96 bytes anywhere go to HBM at 0.96 TB/s, on 32-byte boundaries at 1.4, whole
-// 128-byte lines at 5.1.  Saving pass of the 2^20 Lorenz ATsit5 ensemble (67 M rows): each
-// lane storing its rows from registers 1,717 us, the wave storing unaligned runs 1,708,
-// aligned runs 1,440 (870 with the stores left out).  Small ensembles keep the registers:
-// a lone wave per SIMD waits for the flush's LDS round trips (1,024 trajectories 382
-// against 431 us).  Eight-row runs leave room for two waves per SIMD: 1,618 us.
+// beyond what fits the GPU at once) collect each trajectory's u rows and times in LDS by
+// 64-byte sectors of the output, and the wave writes the sectors that its lanes have filled
+// together (flush_sectors), eight lanes a sector.  What costs is sectors written in part: runs
+// of 96 bytes anywhere go to HBM at 0.96 TB/s, on 32-byte boundaries at 1.4, whole 64-byte
+// sectors at 3.3 and 128-byte lines at 5.1.  Saving pass of the 2^20 Lorenz ATsit5 ensemble
+// (67 M rows): each lane storing its rows from registers 1,717 us, the wave storing runs of
+// four rows 1,708 unaligned and 1,440 at 32 bytes, sectors 1,200 (870 with the stores left
+// out).  Small ensembles keep the registers: a lone wave per SIMD waits for the flush's LDS
+// round trips (1,024 trajectories 382 against 431 us with runs of four rows).
 #ifndef SDEH_PK_ROWS
 #define SDEH_PK_ROWS 4
 #endif
@@ -1081,30 +1080,35 @@ constexpr int PK_ROWS = SDEH_PK_ROWS;
 static_assert(PK_ROWS >= 2 && PK_ROWS <= 4 && (PK_ROWS & (PK_ROWS - 1)) == 0, "2 or 4 rows");
 
 // Whether packed rows go through LDS: one lane per trajectory and at most 32 bytes of
-// state, so that four waves' rows take at most a quarter of a CU's LDS for the states up
-// to three binary64 components (four waves per SIMD, as the registers allow).
+// state, so that a row reaches past the end of one sector at most.  Four waves' sectors and
+// lists with the pow tables take a quarter of a CU's LDS to the byte (four waves per SIMD,
+// as the registers allow; with room for both kinds of sectors in every list the tables did
+// not fit: 2,320 against 2,290 us for the whole solve).
 template <class T, class R>
 struct PkWave {
   static constexpr bool value = R::G == 1 && R::N * sizeof(T) <= 32;
 };
 
-// One wave's rows in LDS.  Row `row` of the output goes to slot row % PK_ROWS of its
-// lane: u [lane][slot][component], t [lane][slot], the lanes an odd number of elements
-// apart (conflict-free for the lanes' own writes); list: the flush's runs.
-template <class T, int N>
+// One wave's sectors in LDS: each lane's current sector of the u output and of the times, as
+// eight 64-bit words, word w of lane l at 8 l + (w ^ l % 8) (lanes at the same word fall in
+// different banks); the flush's list: each sector's address in the output, and its place
+// here (byte offset of word 0) with a mask of its 4-byte pieces to write above it.
 struct PkBuf {
-  static constexpr int US = PK_ROWS * N + 1 - (PK_ROWS * N) % 2, TS = PK_ROWS + 1;
-  // lanes that write one run: PK_ROWS * N of u and PK_ROWS of t, in a power of two
-  static constexpr int NEED = PK_ROWS * (N + 1);
-  static constexpr int LANES = NEED <= 8 ? 8 : NEED <= 16 ? 16 : NEED <= 32 ? 32 : 64;
-  static_assert(NEED <= 64, "a run fits the wave");
-  double t[64 * TS];
-  uint64_t list[64];
-  T u[64 * US];
+  uint64_t w[2][64 * 8];  // u, t
+  uint64_t at[64];
+  unsigned place[64];
+  // element e of lane l's sector of u
+  template <class T>
+  __device__ __forceinline__ T& u(unsigned l, unsigned e) {
+    if constexpr (sizeof(T) == 8) return ((T*)w[0])[8 * l + (e ^ (l & 7u))];
+    else return ((T*)w[0])[16 * l + 2 * ((e >> 1) ^ (l & 7u)) + (e & 1u)];
+  }
+  __device__ __forceinline__ double& t(unsigned l, unsigned e) {
+    return ((double*)w[1])[8 * l + (e ^ (l & 7u))];
+  }
 };
-template <class T, int N>
-__device__ __forceinline__ PkBuf<T, N>& pk_buf() {
-  __shared__ PkBuf<T, N> buf[4];  // blocks of at most 256 threads
+__device__ __forceinline__ PkBuf& pk_buf() {
+  __shared__ PkBuf buf[4];  // blocks of at most 256 threads
   return buf[threadIdx.x >> 6];
 }
 
@@ -1114,7 +1118,9 @@ struct StepSink {
   int32_t lim;   // rows available (packed) or max_saves
   int32_t n;     // points offered
   int32_t kept;  // points stored (written or held back)
-  int32_t held;  // packed: rows held back, in LDS or the last `held` of bt/bu
+  int32_t held;  // packed: rows held back, the last `held` of bt/bu; SAVE_RUNS: HELD flags
+  uint64_t ua;   // SAVE_RUNS: addresses of the next row in u and in the times
+  uint64_t ta;
   double bt[PK_ROWS];
   T bu[PK_ROWS][N];
 };
@@ -1126,6 +1132,8 @@ __device__ __forceinline__ void sink_start(const sdeh_kargs& a, StepSink<T, N>& 
   if (a.packed) {
     s.base = a.steps_off[traj];
     s.lim = a.n_steps[traj];
+    s.ua = (uint64_t)a.u_steps + (uint64_t)s.base * (R::N * R::G * sizeof(T));
+    s.ta = (uint64_t)a.t_steps + (uint64_t)s.base * 8u;
   } else {
     s.base = 0;
     s.lim = a.max_saves;
@@ -1151,80 +1159,92 @@ __device__ __forceinline__ void flush_steps(const sdeh_kargs& a, StepSink<T, R::
   s.held = 0;
 }
 
-// Packed, rows in LDS: write the rows of the lanes flagged in `mine` (each at least one,
-// all of one aligned run of PK_ROWS rows), called by the whole wave.  The flagged lanes
-// list their runs; PkBuf::LANES consecutive lanes write one run, each lane always the same
-// element of u or t, so a run needs one list entry and one value read per lane.
-template <class T, class R>
-__device__ __forceinline__ void flush_wave(const sdeh_kargs& a, StepSink<T, R::N>& s, bool mine) {
-  constexpr int N = R::N;
-  typedef PkBuf<T, N> B;
-  constexpr unsigned PER = 64 / B::LANES;  // runs per pass
-  B& b = pk_buf<T, N>();
-  const unsigned long long mask = __ballot(mine);
-  const unsigned runs = (unsigned)__popcll(mask), l = (unsigned)__lane_id();
-  if (mine) {
-    const uint64_t end = (uint64_t)(s.base + s.kept);  // rows [end - held, end)
-    const uint64_t run = (end - 1) / PK_ROWS;
-    const uint64_t lo = (end - (uint64_t)s.held) - run * PK_ROWS, hi = end - run * PK_ROWS;
-    b.list[lane_rank(mask)] = run << 12 | l << 6 | lo << 3 | hi;
-    s.held = 0;
-  }
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  // this lane's element of a run: where it lies in a lane's LDS rows and in the output
-  const unsigned e = l % B::LANES;
-  const bool is_u = e < (unsigned)(PK_ROWS * N), is_t = !is_u && e < (unsigned)B::NEED;
-  const unsigned slot = is_u ? e / N : e - PK_ROWS * N;
-  const T* const lu = b.u + e;
-  const double* const lt = b.t + (is_t ? slot : 0);
-  T* const gu = (T*)a.u_steps + e;
-  double* const gt = a.t_steps + slot;
-  // four passes at a time, so that their LDS reads are in flight together (a lone wave
-  // otherwise waits for each: 2.8 us for 64 runs)
-  constexpr int Q = 4;
-  for (unsigned r0 = l / B::LANES; r0 < runs; r0 += Q * PER) {
-    uint64_t d[Q];
-#pragma unroll
-    for (int j = 0; j < Q; ++j) {
-      const unsigned r = r0 + j * PER;
-      d[j] = b.list[r < runs ? r : r0];
-      if (r >= runs) d[j] &= ~uint64_t(7);  // no rows
+// SAVE_RUNS: what a lane holds in LDS.  A row that fills or crosses the end of its sector of u
+// leaves that sector to be written (HELD_U) before its elements past the end, which flush_full
+// takes from the state, which is still that row's.  From HELD_LU and HELD_LT on: the first
+// 4-byte piece of the current sectors that is the trajectory's own.
+enum { HELD_U = 1, HELD_T = 2, HELD_PART = 4, HELD_LU = 8, HELD_LT = 12 };
+
+// Write sectors from LDS, called by the whole wave: FULL, the filled sectors of the lanes
+// with HELD_U or HELD_T; otherwise the begun sectors of the lanes flagged in `mine`.
+template <class T, class R, bool FULL>
+__device__ __forceinline__ void flush_sectors(const sdeh_kargs& a, const StepSink<T, R::N>& s,
+                                              bool mine) {
+  PkBuf& b = pk_buf();
+  const unsigned l = (unsigned)__lane_id();
+  const unsigned pu = ((unsigned)s.ua & 63u) >> 2, pt = ((unsigned)s.ta & 63u) >> 2;
+  const bool fu = FULL ? (s.held & HELD_U) != 0 : mine && pu != 0;
+  const bool ft = FULL ? (s.held & HELD_T) != 0 : mine && pt != 0;
+  const unsigned long long mu = __ballot(fu), mt = __ballot(ft);
+  const unsigned home = 64u * l + 8u * (l & 7u);  // word 0 of this lane's sector of u
+  const unsigned w = l & 7u, w8 = 8u * w;
+  // the list holds a wave's sectors of one kind, as a rule those of both
+  const bool once = __popcll(mu) + __popcll(mt) <= 64;
+  for (int go = once ? 1 : 0; go < 2; ++go) {
+    const unsigned long long gu = go == 0 || once ? mu : 0ull, gt = go == 1 ? mt : 0ull;
+    const unsigned nu = (unsigned)__popcll(gu), cnt = nu + (unsigned)__popcll(gt);
+    if (fu && gu != 0ull) {
+      const unsigned k = lane_rank(mu), lo = (unsigned)(s.held >> HELD_LU) & 15u;
+      b.at[k] = (s.ua & ~63ull) - (FULL ? 64u : 0u);
+      b.place[k] = home | ((FULL ? 0xffffu : (1u << pu) - 1u) >> lo << lo) << 16;
     }
-    if constexpr (sizeof(T) == 8) {  // u and t alike: one read and one store per lane
-      const T* const lp = is_u ? lu : (const T*)lt;
-      T* const gp = is_u ? gu : (T*)gt;
-      const unsigned ls = is_u ? B::US : B::TS, gs = is_u ? PK_ROWS * N : PK_ROWS;
-      T v[Q];
+    if (ft && gt != 0ull) {
+      const unsigned k = nu + lane_rank(mt), lo = (unsigned)(s.held >> HELD_LT) & 15u;
+      b.at[k] = (s.ta & ~63ull) - (FULL ? 64u : 0u);
+      b.place[k] = home | 4096u | ((FULL ? 0xffffu : (1u << pt) - 1u) >> lo << lo) << 16;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    // two passes at a time, so that their LDS reads are in flight together
+    constexpr unsigned Q = 2;
+    for (unsigned r0 = l >> 3; r0 < cnt; r0 += 8 * Q) {
+      uint64_t at[Q], v[Q];
+      unsigned pl[Q];
 #pragma unroll
-      for (int j = 0; j < Q; ++j) v[j] = lp[((unsigned)(d[j] >> 6) & 63u) * ls];
-#pragma unroll
-      for (int j = 0; j < Q; ++j)
-        if (slot >= ((unsigned)(d[j] >> 3) & 7u) && slot < ((unsigned)d[j] & 7u))
-          gp[(d[j] >> 12) * gs] = v[j];
-    } else {
-      T vu[Q];
-      double vt[Q];
-#pragma unroll
-      for (int j = 0; j < Q; ++j) {
-        const unsigned src = (unsigned)(d[j] >> 6) & 63u;
-        if (is_u) vu[j] = lu[src * B::US];
-        else vt[j] = lt[src * B::TS];
+      for (unsigned j = 0; j < Q; ++j) {  // (entries past cnt are read, but not used)
+        at[j] = b.at[(r0 + 8 * j) & 63u] | w8;
+        pl[j] = b.place[(r0 + 8 * j) & 63u];
       }
 #pragma unroll
-      for (int j = 0; j < Q; ++j)
-        if (slot >= ((unsigned)(d[j] >> 3) & 7u) && slot < ((unsigned)d[j] & 7u)) {
-          if (is_u) gu[(d[j] >> 12) * (PK_ROWS * N)] = vu[j];
-          else gt[(d[j] >> 12) * PK_ROWS] = vt[j];
+      for (unsigned j = 0; j < Q; ++j)
+        v[j] = *(const uint64_t*)((const char*)b.w + ((pl[j] & 0x1ff8u) ^ w8));
+#pragma unroll
+      for (unsigned j = 0; j < Q; ++j) {
+        const unsigned m = r0 + 8 * j < cnt ? pl[j] >> (16u + 2u * w) & 3u : 0u;
+        if (m == 3u) *(uint64_t*)at[j] = v[j];
+        if (sizeof(T) == 4) {
+          if (m == 1u) *(uint32_t*)at[j] = (uint32_t)v[j];
+          if (m == 2u) *(uint32_t*)(at[j] + 4) = (uint32_t)(v[j] >> 32);
         }
+      }
     }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();  // the reads are done before the next writes
   }
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();  // the reads are done before a lane writes its next row
 }
 
-// RUNS: rows go to LDS, and the caller calls flush_wave at the end of each aligned run.
+// The filled sectors of the wave's lanes, then the elements of the last row past the end of
+// its sector, from the state u.
+template <class T, class R>
+__device__ __forceinline__ void flush_full(const sdeh_kargs& a, StepSink<T, R::N>& s,
+                                           const T (&u)[R::N]) {
+  constexpr unsigned SE = 64 / sizeof(T);
+  flush_sectors<T, R, true>(a, s, false);
+  if (s.held & HELD_U) {
+    PkBuf& b = pk_buf();
+    const unsigned l = (unsigned)__lane_id();
+    const unsigned past = ((unsigned)s.ua & 63u) / (unsigned)sizeof(T);  // elements past the end
+#pragma unroll
+    for (int c = 1; c < R::N; ++c) {
+      const unsigned e = past - (unsigned)(R::N - c);
+      if (e < SE) b.u<T>(l, e) = u[c];
+    }
+    s.held &= ~(HELD_U | 15 << HELD_LU);
+  }
+  if (s.held & HELD_T) s.held &= ~(HELD_T | 15 << HELD_LT);
+}
+
 template <class T, class R, bool RUNS = false>
 __device__ __forceinline__ void save_step(const sdeh_kargs& a, StepSink<T, R::N>& s,
                                           int64_t traj, double t, const T (&u)[R::N]) {
@@ -1232,22 +1252,36 @@ __device__ __forceinline__ void save_step(const sdeh_kargs& a, StepSink<T, R::N>
   ++s.n;
   if (s.kept >= s.lim) return;
   if constexpr (RUNS) {
-    PkBuf<T, R::N>& b = pk_buf<T, R::N>();
-    const int l = (int)__lane_id();
-    const int64_t row = s.base + s.kept;
-    const int slot = (int)row & (PK_ROWS - 1);
-    if (s.kept == 0 && slot == PK_ROWS - 1) {
-      // a first row that ends its run goes out at once: the step after it may come
-      // before the next flush
+    constexpr unsigned SE = 64 / sizeof(T);
+    PkBuf& b = pk_buf();
+    const unsigned l = (unsigned)__lane_id();
+    const unsigned su = ((unsigned)s.ua & 63u) / (unsigned)sizeof(T);
+    const unsigned st = ((unsigned)s.ta & 63u) / 8u;
+    const bool ends_u = su + (unsigned)R::N >= SE, ends_t = st == 7u;
+    if (s.kept == 0) {
+      // a first row's part of a sector that it ends goes out at once: the step after it may
+      // come before the next flush
 #pragma unroll
-      for (int c = 0; c < R::N; ++c) ((T*)a.u_steps)[row * R::N + c] = u[c];
-      a.t_steps[row] = t;
+      for (int c = 0; c < R::N; ++c) {
+        const unsigned e = su + (unsigned)c;
+        if (ends_u && e < SE) ((T*)s.ua)[c] = u[c];
+        else b.u<T>(l, e & (SE - 1)) = u[c];
+      }
+      if (ends_t) *(double*)s.ta = t;
+      else b.t(l, st) = t;
+      s.held = HELD_PART | (ends_u ? 0 : (int)(su * sizeof(T) / 4) << HELD_LU) |
+               (ends_t ? 0 : (int)(2u * st) << HELD_LT);
     } else {
 #pragma unroll
-      for (int c = 0; c < R::N; ++c) b.u[l * PkBuf<T, R::N>::US + slot * R::N + c] = u[c];
-      b.t[l * PkBuf<T, R::N>::TS + slot] = t;
-      ++s.held;
+      for (int c = 0; c < R::N; ++c) {
+        const unsigned e = su + (unsigned)c;
+        if (c == 0 || e < SE) b.u<T>(l, e) = u[c];
+      }
+      b.t(l, st) = t;
+      s.held |= (ends_u ? HELD_U : 0) | (ends_t ? HELD_T : 0);
     }
+    s.ua += R::N * sizeof(T);
+    s.ta += 8u;
     ++s.kept;
     return;
   }
@@ -1839,8 +1873,7 @@ __device__ __forceinline__ void adaptive_body(const sdeh_kargs& a) {
           gamma = T(9.0 / 10), qoldinit = T(1.0e-4);
   const T inv_qmax = T(1) / qmax, inv_qmin = T(1) / qmin;
   const T qoldinit_pow = Ops<T>::pw(qoldinit, beta2);
-  // (the runs' buffers leave no LDS for a fourth block of four waves)
-  const auto tab = pow_tables<sizeof(T) == 8 && SAVE != SAVE_RUNS>();
+  const auto tab = pow_tables<sizeof(T) == 8>();
   const auto saves_at = SaveTimes<SAVE == SAVE_AT>::init(a);
   constexpr bool PIN = sizeof(T) == 8 && SAVE == SAVE_END;
   const T abstol = in_vgpr_if<PIN>((T)a.abstol), reltol = in_vgpr_if<PIN>((T)a.reltol);
@@ -1855,7 +1888,7 @@ __device__ __forceinline__ void adaptive_body(const sdeh_kargs& a) {
   T dt = T(0), qold_pow = T(0);
   int32_t nacc = 0, nrej = 0, cur = 0;
   constexpr bool RUNS = SAVE == SAVE_RUNS, STEPS = RUNS || SAVE == SAVE_STEPS;
-  static_assert(!RUNS || PkWave<T, R>::value, "runs of a small state");
+  static_assert(!RUNS || PkWave<T, R>::value, "sectors of a small state");
   StepSink<T, N> sk{};
   double ts_next = 0.0;  // the save time of point cur
   int64_t attempts = 0, traj = -1;
@@ -1888,12 +1921,16 @@ __device__ __forceinline__ void adaptive_body(const sdeh_kargs& a) {
 
   for (;;) {
     if constexpr (RUNS) {
-      // Rows held in LDS: each lane's once they end an aligned run; those of ended
-      // trajectories before their lanes can take new ones, or at the wave's end.
-      const bool ends = a.persistent || __ballot(active) == 0ull;
-      const bool out = sk.held > 0 && (((sk.base + sk.kept) & (PK_ROWS - 1)) == 0 ||
-                                       (ends && !active));
-      if (__ballot(out) != 0ull) flush_wave<T, R>(a, sk, out);
+      // Sectors in LDS: each once it is full; the begun ones of ended trajectories
+      // before their lanes can take new ones, or at the wave's end.
+      if (__ballot((sk.held & (HELD_U | HELD_T)) != 0) != 0ull) flush_full<T, R>(a, sk, uprev);
+      if (a.persistent || __ballot(active) == 0ull) {
+        const bool out = !active && sk.held != 0;
+        if (__ballot(out) != 0ull) {
+          flush_sectors<T, R, false>(a, sk, out);
+          if (out) sk.held = 0;
+        }
+      }
     }
     if (a.persistent) {
       bool want = !active && lead;

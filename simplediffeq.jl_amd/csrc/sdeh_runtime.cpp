@@ -823,7 +823,7 @@ int plan_solve(sdeh_ctx* c, const sdeh_solve_desc* d, const sdeh_io* io, Plan* p
         sh.schedule = SDEH_SCHED_ONE_LAUNCH;
         sh.block = 256;
         pl->span = false;
-        // the kernel that writes its rows by runs, for states of at most 32 bytes
+        // the kernel that writes its rows by whole sectors, for states of at most 32 bytes
         KernelRef kr;
         if ((size_t)pl->n_state * pl->es <= 32 &&
             !resolve_kernel(c, d->rhs, d->alg, d->dtype, SAVE_RUNS, pl->kahan, 1, &kr))
@@ -1007,7 +1007,9 @@ int run_plan(sdeh_ctx* c, Plan& pl, hipStream_t s, unsigned long long* queue, bo
       if (st) return st;
     } else {
       if (a.persistent) HIPCHK(c, sdeh_util_zero_u64(queue, 1, s));
-      const bool runs = pl.pk_ranked && (pl.k_runs.aot || pl.k_runs.fn);
+      // (its kernel finds whole elements in the outputs' 64-byte sectors)
+      const bool runs = pl.pk_ranked && (pl.k_runs.aot || pl.k_runs.fn) &&
+                        (uintptr_t)a.u_steps % pl.es == 0 && (uintptr_t)a.t_steps % 8 == 0;
       HIPCHK(c, launch(runs ? pl.k_runs : pl.k, pl.shape.grid, pl.shape.block, &a, s));
     }
     if (timed) HIPCHK(c, hipEventRecord(c->ev1, s));

@@ -1,7 +1,7 @@
 """Packed save_everystep rows: states on both sides of the 32-byte rule, sizes around a wave
 and a block, both precisions, a trajectory left with part of its rows (against the
 trajectory-major rows, bit for bit); and, beyond what fits the GPU at once, the saving pass
-in the order of the counted attempts that writes aligned runs of four rows from LDS
+in the order of the counted attempts that writes whole sectors from LDS
 (against the persistent schedule, bit for bit)."""
 import numpy as np
 import pytest
@@ -87,7 +87,7 @@ def test_cut_in_the_middle_of_a_run(ctx, alg, short):
     (4, _abi.F64, _abi.ALG_ATSIT5, True, 3)])
 def test_ranked_saving_pass(n_state, dtype, alg, spans, cut):
     """Beyond what fits the GPU at once the saving pass takes the trajectories by their
-    counted attempts and writes run by run; everything is the persistent schedule's."""
+    counted attempts and writes sector by sector; everything is the persistent schedule's."""
     c = runtime.Context(0)
     rhs, n_param = _rhs(c, n_state)
     n = 600_001
