@@ -39,6 +39,7 @@ SDEH_HIDDEN const void* sdeh_aot_ExpDecay3(int, int, int, int, int, int);
 SDEH_HIDDEN const void* sdeh_aot_Affine1(int, int, int, int, int, int);
 SDEH_HIDDEN const void* sdeh_aot_Linear2(int, int, int, int, int, int);
 SDEH_HIDDEN hipError_t sdeh_util_fill_f64(double*, double, int64_t, hipStream_t);
+SDEH_HIDDEN hipError_t sdeh_util_transpose(const void*, void*, int64_t, int64_t, int, hipStream_t);
 SDEH_HIDDEN hipError_t sdeh_util_fill_f32(float*, float, int64_t, hipStream_t);
 SDEH_HIDDEN hipError_t sdeh_util_zero_u64(unsigned long long*, int, hipStream_t);
 SDEH_HIDDEN hipError_t sdeh_util_count(const int32_t*, const int32_t*, const int32_t*, int64_t,
@@ -564,6 +565,9 @@ struct Plan {
   // decreasing attempts, as counted, in one launch (see run_plan)
   bool pk_ranked = false;
   KernelRef k_runs;  // its kernel where it is not k
+  // point-major saveat output by way of trajectory-major rows in scratch (see row_scratch)
+  bool by_rows = false;
+  void* rows_out = nullptr;
   int64_t pk_cap = 0;
   int64_t* pk_off = nullptr;
   int64_t* pk_tiles = nullptr;
@@ -641,6 +645,7 @@ size_t staged_stride(const sdeh_solve_desc* d, const Plan& pl) {
 // Persistent layouts with several lanes per trajectory claim one wave's slots at a time
 // (GLV-16 ATsit5, 500,000: 2,972 against 3,491 us claiming 64).
 constexpr size_t kStagedBytes = size_t(1) << 30;
+
 Shape default_shape(sdeh_ctx* c, const Plan& pl, int dtype, int64_t n, bool sorted, bool planned,
                     bool can_stage) {
   Shape sh;
@@ -659,6 +664,31 @@ Shape default_shape(sdeh_ctx* c, const Plan& pl, int dtype, int64_t n, bool sort
     sh.schedule = SDEH_SCHED_PERSISTENT;
   }
   return sh;
+}
+
+// Whether point-major saveat output goes by way of trajectory-major rows in scratch and a
+// transpose.  The lanes of a wave reach a save point at different times, the further apart
+// the more points there are, so in the point-major layout each stores single elements,
+// lines apart; the memory-side cache (256 MB) still joins them into whole lines where the
+// output about fits it, and beyond that each goes to memory by itself.  The costlier a step,
+// the more of that hides behind it.  Stored in place | by way of rows (us):
+//   ATsit5  Lorenz binary64  150,001 x 101 points    679 |   677     524,288 x  50  1,126 | 1,154
+//                            262,144 x  80           917 |   814     524,288 x  30    898 |   953
+//                            262,144 x 101         1,166 |   928   1,048,576 x  30  1,551 | 1,745
+//                            262,144 x 200         2,857 | 1,561
+//           Lorenz binary32  262,144 x 101           845 |   607
+//           GLV-16 binary32  131,072 x 256         4,942 | 1,806     131,072 x  50    578 |   702
+//                  binary64   65,536 x 128         1,379 | 1,133     131,072 x  50  1,054 | 1,283
+//   AVern7  Lorenz           262,144 x 200         3,942 | 3,326     262,144 x 101  2,151 | 2,272
+//                            524,288 x 160         5,671 | 5,392
+//   AVern9  Lorenz           524,288 x 160         9,968 | 10,125
+//           GLV-16           131,072 x 120         5,535 | 5,806
+// (Fixed-step solvers reach a point with all lanes at once.)
+constexpr size_t kRowsFrom = size_t(300) << 20, kRowsTo = size_t(2) << 30;
+bool row_scratch(const sdeh_solve_desc* d, const Plan& pl, size_t bytes) {
+  const int64_t from = d->alg == SDEH_ALG_ATSIT5 ? 80 : d->alg == SDEH_ALG_AVERN7 ? 160 : 0;
+  return pl.save == SAVE_AT && from && d->n_saveat >= from &&
+         d->save_layout == SDEH_SAVE_POINT_MAJOR && bytes > kRowsFrom && bytes <= kRowsTo;
 }
 
 // Validate the descriptor and fill everything except the device pointers.
@@ -1012,6 +1042,9 @@ int run_plan(sdeh_ctx* c, Plan& pl, hipStream_t s, unsigned long long* queue, bo
                         (uintptr_t)a.u_steps % pl.es == 0 && (uintptr_t)a.t_steps % 8 == 0;
       HIPCHK(c, launch(runs ? pl.k_runs : pl.k, pl.shape.grid, pl.shape.block, &a, s));
     }
+    if (pl.by_rows)
+      HIPCHK(c, sdeh_util_transpose(a.u_saveat, pl.rows_out, a.n, a.n_saveat * pl.n_state,
+                                    (int)pl.es, s));
     if (timed) HIPCHK(c, hipEventRecord(c->ev1, s));
   }
   return SDEH_OK;
@@ -1177,6 +1210,7 @@ int solve_impl(sdeh_ctx* c, const sdeh_solve_desc* d, const sdeh_io* io, int32_t
     pl.shape.schedule = SDEH_SCHED_PERSISTENT;
   }
 
+  pl.by_rows = !host && row_scratch(d, pl, sz.u_saveat);
   // Device layout: saveat copy + (host mode) all buffers + counters always.
   const bool own_counts = !io->naccept || !io->nreject || host;
   auto scratch_need = [&]() {
@@ -1194,6 +1228,7 @@ int solve_impl(sdeh_ctx* c, const sdeh_solve_desc* d, const sdeh_io* io, int32_t
       if (host) need += round256(sz.pk_off);
     }
     if (pl.span) need += round256(sz.span_order) + 2 * round256(sz.span_hist);
+    if (pl.by_rows) need += round256(sz.u_saveat);
     if (pl.staged || pl.pk_ranked)
       need += round256(sz.st_rec) + round256(sz.st_key) + round256(sz.st_order) +
               round256(sz.st_hist);
@@ -1211,6 +1246,11 @@ int solve_impl(sdeh_ctx* c, const sdeh_solve_desc* d, const sdeh_io* io, int32_t
     pl.shape.schedule = SDEH_SCHED_PERSISTENT;
     c->err.clear();
     sz = sizes_of(d, io, pl);
+    r = ensure_arena(c, scratch_need());
+  }
+  if (r == SDEH_E_NOMEM && pl.by_rows) {  // no room for the rows: stored where they belong
+    pl.by_rows = false;
+    c->err.clear();
     r = ensure_arena(c, scratch_need());
   }
   if (r) return r;
@@ -1277,6 +1317,11 @@ int solve_impl(sdeh_ctx* c, const sdeh_solve_desc* d, const sdeh_io* io, int32_t
     a.u_steps = io->u_steps;
     a.t_steps = io->t_steps;
     a.n_steps = io->n_steps;
+  }
+  if (pl.by_rows && n > 0) {
+    pl.rows_out = a.u_saveat;
+    a.u_saveat = ar.take(sz.u_saveat);
+    a.traj_major = 1;
   }
   a.naccept = (!host && io->naccept) ? io->naccept : nullptr;
   a.nreject = (!host && io->nreject) ? io->nreject : nullptr;
