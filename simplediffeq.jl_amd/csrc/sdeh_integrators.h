@@ -560,35 +560,97 @@ __device__ __forceinline__ T poly2(T th, const T (&r)[NR]) {
 // `kahan` variants return the compensation of the u update.
 // ---------------------------------------------------------------------------
 
+// The stages' coefficients as immediates (Imm), which the compiler moves to scalar registers
+// before each use (two moves for each binary64 one), or the first of them held in scalar
+// registers for the kernel's life (Held: as many as the registers hold beside a save mode's
+// pointers).  A lone wave waits for each move: Lorenz, 100 fixed steps, 1,024 trajectories,
+// immediates / held: Tsit5 46 / 32 us, Vern7 70 / 52, Vern9 125 / 97; 2^20 trajectories 457 /
+// 440, 698 / 686, 1,262 / 1,235.
+#define SDEH_TSIT5_HELD(X)                                                                      \
+  X(a21) X(a31) X(a32) X(a41) X(a42) X(a43) X(a51) X(a52) X(a53) X(a54) X(a61) X(a62) X(a63)    \
+  X(a64) X(a65) X(a71) X(a72) X(a73) X(a74) X(a75) X(a76)
+#define SDEH_TSIT5_REST(X)
+#define SDEH_VERN7_HELD(X)                                                                      \
+  X(a021) X(a031) X(a032) X(a041) X(a043) X(a051) X(a053) X(a054) X(a061) X(a063) X(a064)       \
+  X(a065) X(a071) X(a073) X(a074) X(a075) X(a076) X(a081) X(a083) X(a084) X(a085)
+#define SDEH_VERN7_REST(X)                                                                      \
+  X(a086) X(a087) X(a091) X(a093) X(a094) X(a095) X(a096) X(a097) X(a098) X(b1) X(b4) X(b5)     \
+  X(b6) X(b7) X(b8) X(b9)
+#define SDEH_VERN9_HELD(X)                                                                      \
+  X(a0201) X(a0301) X(a0302) X(a0401) X(a0403) X(a0501) X(a0503) X(a0504) X(a0601) X(a0604)     \
+  X(a0605) X(a0701) X(a0704) X(a0705) X(a0706) X(a0801) X(a0806) X(a0807) X(a0901) X(a0906)     \
+  X(a0907)
+#define SDEH_VERN9_REST(X)                                                                      \
+  X(a0908) X(a1001) X(a1006) X(a1007) X(a1008) X(a1009) X(a1101) X(a1106) X(a1107) X(a1108)     \
+  X(a1109) X(a1110) X(a1201) X(a1206) X(a1207) X(a1208) X(a1209) X(a1210) X(a1211) X(a1301)     \
+  X(a1306) X(a1307) X(a1308) X(a1309) X(a1310) X(a1311) X(a1312) X(a1401) X(a1406) X(a1407)     \
+  X(a1408) X(a1409) X(a1410) X(a1411) X(a1412) X(a1413) X(a1501) X(a1506) X(a1507) X(a1508)     \
+  X(a1509) X(a1510) X(a1511) X(a1512) X(a1513) X(a1514) X(b1) X(b8) X(b9) X(b10) X(b11)         \
+  X(b12) X(b13) X(b14) X(b15)
+template <class X>
+__device__ __forceinline__ X in_sgpr(X x) {
+  asm volatile("" : "+s"(x));
+  return x;
+}
+#define SDEH_IMM(n) T n = T(TAB::n);
+#define SDEH_HOLD(n) k.n = in_sgpr(k.n);
+#define SDEH_COEFS(NAME, LIST)                          \
+  template <class T>                                    \
+  struct NAME##Imm {                                    \
+    SDEH_##LIST##_HELD(SDEH_IMM) SDEH_##LIST##_REST(SDEH_IMM)  \
+    __device__ static NAME##Imm init() { return {}; }   \
+  };                                                    \
+  template <class T>                                    \
+  struct NAME##Held {                                   \
+    SDEH_##LIST##_HELD(SDEH_IMM) SDEH_##LIST##_REST(SDEH_IMM) \
+    __device__ static NAME##Held init() {               \
+      NAME##Held k;                                     \
+      SDEH_##LIST##_HELD(SDEH_HOLD)                     \
+      return k;                                         \
+    }                                                   \
+  };
+#define TAB sdeh_tab::tsit5
+SDEH_COEFS(Ts, TSIT5)
+#undef TAB
+#define TAB sdeh_tab::vern7
+SDEH_COEFS(V7C, VERN7)
+#undef TAB
+#define TAB sdeh_tab::vern9
+SDEH_COEFS(V9C, VERN9)
+#undef TAB
+#undef SDEH_COEFS
+#undef SDEH_HOLD
+#undef SDEH_IMM
+
 #define TS(x) T(sdeh_tab::tsit5::x)
 
 // Tsit5 stages k2..k7 from k1 (FSAL); gpuatsit5.jl:99-110 / 258-270.
-template <class T, class R, bool KAHAN>
+template <class T, class R, bool KAHAN, class C = TsImm<T>>
 __device__ __forceinline__ void tsit5_stages(const T (&uprev)[R::N], const T (&k1)[R::N],
                                              T (&k2)[R::N], T (&k3)[R::N], T (&k4)[R::N],
                                              T (&k5)[R::N], T (&k6)[R::N], T (&k7)[R::N],
                                              T (&u)[R::N], const T (&comp)[R::N],
                                              T (&comp_new)[R::N], const T* p, const T* ps,
-                                             double t, T dt) {
+                                             double t, T dt, const C& co = C()) {
   constexpr int N = R::N;
   T tmp[N];
-  comb1(tmp, uprev, dt * TS(a21), k1);
+  comb1(tmp, uprev, dt * co.a21, k1);
   R::f(k2, tmp, p, ps, stage_t(t, (double)TS(c1), (double)dt));
-  comb(tmp, uprev, dt, TS(a31), k1, TS(a32), k2);
+  comb(tmp, uprev, dt, co.a31, k1, co.a32, k2);
   R::f(k3, tmp, p, ps, stage_t(t, (double)TS(c2), (double)dt));
-  comb(tmp, uprev, dt, TS(a41), k1, TS(a42), k2, TS(a43), k3);
+  comb(tmp, uprev, dt, co.a41, k1, co.a42, k2, co.a43, k3);
   R::f(k4, tmp, p, ps, stage_t(t, (double)TS(c3), (double)dt));
-  comb(tmp, uprev, dt, TS(a51), k1, TS(a52), k2, TS(a53), k3, TS(a54), k4);
+  comb(tmp, uprev, dt, co.a51, k1, co.a52, k2, co.a53, k3, co.a54, k4);
   R::f(k5, tmp, p, ps, stage_t(t, (double)TS(c4), (double)dt));
-  comb(tmp, uprev, dt, TS(a61), k1, TS(a62), k2, TS(a63), k3, TS(a64), k4, TS(a65), k5);
+  comb(tmp, uprev, dt, co.a61, k1, co.a62, k2, co.a63, k3, co.a64, k4, co.a65, k5);
   R::f(k6, tmp, p, ps, t + (double)dt);
   if constexpr (KAHAN) {
     T acc[N];
-    lsum(acc, TS(a71), k1, TS(a72), k2, TS(a73), k3, TS(a74), k4, TS(a75), k5, TS(a76), k6);
+    lsum(acc, co.a71, k1, co.a72, k2, co.a73, k3, co.a74, k4, co.a75, k5, co.a76, k6);
     kahan_update(u, comp_new, uprev, comp, dt, acc);
   } else {
-    comb(u, uprev, dt, TS(a71), k1, TS(a72), k2, TS(a73), k3, TS(a74), k4, TS(a75), k5,
-         TS(a76), k6);
+    comb(u, uprev, dt, co.a71, k1, co.a72, k2, co.a73, k3, co.a74, k4, co.a75, k5,
+         co.a76, k6);
   }
   R::f(k7, u, p, ps, t + (double)dt);
 }
@@ -632,32 +694,32 @@ struct V7K {
 
 // Verner 7 stages k1..k9 (+k10, error) and u; gpuvern7.jl:104-136 / 360-402.
 // Returns the embedded error accumulator in err (adaptive only).
-template <class T, class R, bool ADAPT, bool KAHAN>
+template <class T, class R, bool ADAPT, bool KAHAN, class C = V7CImm<T>>
 __device__ __forceinline__ void vern7_stages(const T (&uprev)[R::N], V7K<T, R::N>& K,
                                              T (&u)[R::N], T (&err)[R::N],
                                              const T (&comp)[R::N], T (&comp_new)[R::N],
-                                             const T* p, const T* ps, double t, T dt) {
+                                             const T* p, const T* ps, double t, T dt, const C& co = C()) {
   constexpr int N = R::N;
   T tmp[N], k2[N], k3[N];
   R::f(K.k1, uprev, p, ps, t);
-  comb1(tmp, uprev, dt * V7(a021), K.k1);
+  comb1(tmp, uprev, dt * co.a021, K.k1);
   R::f(k2, tmp, p, ps, stage_t(t, (double)V7(c2), (double)dt));
-  comb(tmp, uprev, dt, V7(a031), K.k1, V7(a032), k2);
+  comb(tmp, uprev, dt, co.a031, K.k1, co.a032, k2);
   R::f(k3, tmp, p, ps, stage_t(t, (double)V7(c3), (double)dt));
-  comb(tmp, uprev, dt, V7(a041), K.k1, V7(a043), k3);
+  comb(tmp, uprev, dt, co.a041, K.k1, co.a043, k3);
   R::f(K.k4, tmp, p, ps, stage_t(t, (double)V7(c4), (double)dt));
-  comb(tmp, uprev, dt, V7(a051), K.k1, V7(a053), k3, V7(a054), K.k4);
+  comb(tmp, uprev, dt, co.a051, K.k1, co.a053, k3, co.a054, K.k4);
   R::f(K.k5, tmp, p, ps, stage_t(t, (double)V7(c5), (double)dt));
-  comb(tmp, uprev, dt, V7(a061), K.k1, V7(a063), k3, V7(a064), K.k4, V7(a065), K.k5);
+  comb(tmp, uprev, dt, co.a061, K.k1, co.a063, k3, co.a064, K.k4, co.a065, K.k5);
   R::f(K.k6, tmp, p, ps, stage_t(t, (double)V7(c6), (double)dt));
-  comb(tmp, uprev, dt, V7(a071), K.k1, V7(a073), k3, V7(a074), K.k4, V7(a075), K.k5, V7(a076),
+  comb(tmp, uprev, dt, co.a071, K.k1, co.a073, k3, co.a074, K.k4, co.a075, K.k5, co.a076,
        K.k6);
   R::f(K.k7, tmp, p, ps, stage_t(t, (double)V7(c7), (double)dt));
-  comb(tmp, uprev, dt, V7(a081), K.k1, V7(a083), k3, V7(a084), K.k4, V7(a085), K.k5, V7(a086),
-       K.k6, V7(a087), K.k7);
+  comb(tmp, uprev, dt, co.a081, K.k1, co.a083, k3, co.a084, K.k4, co.a085, K.k5, co.a086,
+       K.k6, co.a087, K.k7);
   R::f(K.k8, tmp, p, ps, stage_t(t, (double)V7(c8), (double)dt));
-  comb(tmp, uprev, dt, V7(a091), K.k1, V7(a093), k3, V7(a094), K.k4, V7(a095), K.k5, V7(a096),
-       K.k6, V7(a097), K.k7, V7(a098), K.k8);
+  comb(tmp, uprev, dt, co.a091, K.k1, co.a093, k3, co.a094, K.k4, co.a095, K.k5, co.a096,
+       K.k6, co.a097, K.k7, co.a098, K.k8);
   T k10[N];
   if constexpr (ADAPT) {
     T g10[N];
@@ -670,12 +732,12 @@ __device__ __forceinline__ void vern7_stages(const T (&uprev)[R::N], V7K<T, R::N
   }
   if constexpr (KAHAN) {
     T acc[N];
-    lsum(acc, V7(b1), K.k1, V7(b4), K.k4, V7(b5), K.k5, V7(b6), K.k6, V7(b7), K.k7, V7(b8),
-         K.k8, V7(b9), K.k9);
+    lsum(acc, co.b1, K.k1, co.b4, K.k4, co.b5, K.k5, co.b6, K.k6, co.b7, K.k7, co.b8,
+         K.k8, co.b9, K.k9);
     kahan_update(u, comp_new, uprev, comp, dt, acc);
   } else {
-    comb(u, uprev, dt, V7(b1), K.k1, V7(b4), K.k4, V7(b5), K.k5, V7(b6), K.k6, V7(b7), K.k7,
-         V7(b8), K.k8, V7(b9), K.k9);
+    comb(u, uprev, dt, co.b1, K.k1, co.b4, K.k4, co.b5, K.k5, co.b6, K.k6, co.b7, K.k7,
+         co.b8, K.k8, co.b9, K.k9);
   }
   if constexpr (ADAPT) {
     lsum(err, V7(btilde1), K.k1, V7(btilde4), K.k4, V7(btilde5), K.k5, V7(btilde6), K.k6,
@@ -749,31 +811,31 @@ struct V9S {
 // On return `S` holds the dense-output slots: k1, k8..k15 (renamed as at
 // gpuvern9.jl:564-573) or, when `alias_quirk`, k1..k9 (the fixed solver's
 // unrenamed variables, gpuvern9.jl:216-331).
-template <class T, class R, bool ADAPT, bool KAHAN, bool KEEP>
+template <class T, class R, bool ADAPT, bool KAHAN, bool KEEP, class C = V9CImm<T>>
 __device__ __forceinline__ void vern9_stages(const T (&uprev)[R::N], V9S<T, R::N>& S,
                                              T (&u)[R::N], T (&err)[R::N],
                                              const T (&comp)[R::N], T (&comp_new)[R::N],
                                              const T* p, const T* ps, double t, T dt,
-                                             bool alias_quirk) {
+                                             bool alias_quirk, const C& co = C()) {
   constexpr int N = R::N;
   T tmp[N], k1[N], k2[N], k3[N], k4[N], k5[N], k6[N], k7[N], k8[N], k9[N], k10[N], k11[N],
       k12[N], k13[N], k14[N], k15[N];
   R::f(k1, uprev, p, ps, t);
-  comb1(tmp, uprev, dt * V9(a0201), k1);
+  comb1(tmp, uprev, dt * co.a0201, k1);
   R::f(k2, tmp, p, ps, stage_t(t, (double)V9(c1), (double)dt));
-  comb(tmp, uprev, dt, V9(a0301), k1, V9(a0302), k2);
+  comb(tmp, uprev, dt, co.a0301, k1, co.a0302, k2);
   R::f(k3, tmp, p, ps, stage_t(t, (double)V9(c2), (double)dt));
-  comb(tmp, uprev, dt, V9(a0401), k1, V9(a0403), k3);
+  comb(tmp, uprev, dt, co.a0401, k1, co.a0403, k3);
   R::f(k4, tmp, p, ps, stage_t(t, (double)V9(c3), (double)dt));
-  comb(tmp, uprev, dt, V9(a0501), k1, V9(a0503), k3, V9(a0504), k4);
+  comb(tmp, uprev, dt, co.a0501, k1, co.a0503, k3, co.a0504, k4);
   R::f(k5, tmp, p, ps, stage_t(t, (double)V9(c4), (double)dt));
-  comb(tmp, uprev, dt, V9(a0601), k1, V9(a0604), k4, V9(a0605), k5);
+  comb(tmp, uprev, dt, co.a0601, k1, co.a0604, k4, co.a0605, k5);
   R::f(k6, tmp, p, ps, stage_t(t, (double)V9(c5), (double)dt));
-  comb(tmp, uprev, dt, V9(a0701), k1, V9(a0704), k4, V9(a0705), k5, V9(a0706), k6);
+  comb(tmp, uprev, dt, co.a0701, k1, co.a0704, k4, co.a0705, k5, co.a0706, k6);
   R::f(k7, tmp, p, ps, stage_t(t, (double)V9(c6), (double)dt));
-  comb(tmp, uprev, dt, V9(a0801), k1, V9(a0806), k6, V9(a0807), k7);
+  comb(tmp, uprev, dt, co.a0801, k1, co.a0806, k6, co.a0807, k7);
   R::f(k8, tmp, p, ps, stage_t(t, (double)V9(c7), (double)dt));
-  comb(tmp, uprev, dt, V9(a0901), k1, V9(a0906), k6, V9(a0907), k7, V9(a0908), k8);
+  comb(tmp, uprev, dt, co.a0901, k1, co.a0906, k6, co.a0907, k7, co.a0908, k8);
   R::f(k9, tmp, p, ps, stage_t(t, (double)V9(c8), (double)dt));
   if constexpr (KEEP) {
     if (alias_quirk) {
@@ -781,23 +843,23 @@ __device__ __forceinline__ void vern9_stages(const T (&uprev)[R::N], V9S<T, R::N
       copyv(S.s[5], k6); copyv(S.s[6], k7); copyv(S.s[7], k8); copyv(S.s[8], k9);
     }
   }
-  comb(tmp, uprev, dt, V9(a1001), k1, V9(a1006), k6, V9(a1007), k7, V9(a1008), k8, V9(a1009),
+  comb(tmp, uprev, dt, co.a1001, k1, co.a1006, k6, co.a1007, k7, co.a1008, k8, co.a1009,
        k9);
   R::f(k10, tmp, p, ps, stage_t(t, (double)V9(c9), (double)dt));
-  comb(tmp, uprev, dt, V9(a1101), k1, V9(a1106), k6, V9(a1107), k7, V9(a1108), k8, V9(a1109),
-       k9, V9(a1110), k10);
+  comb(tmp, uprev, dt, co.a1101, k1, co.a1106, k6, co.a1107, k7, co.a1108, k8, co.a1109,
+       k9, co.a1110, k10);
   R::f(k11, tmp, p, ps, stage_t(t, (double)V9(c10), (double)dt));
-  comb(tmp, uprev, dt, V9(a1201), k1, V9(a1206), k6, V9(a1207), k7, V9(a1208), k8, V9(a1209),
-       k9, V9(a1210), k10, V9(a1211), k11);
+  comb(tmp, uprev, dt, co.a1201, k1, co.a1206, k6, co.a1207, k7, co.a1208, k8, co.a1209,
+       k9, co.a1210, k10, co.a1211, k11);
   R::f(k12, tmp, p, ps, stage_t(t, (double)V9(c11), (double)dt));
-  comb(tmp, uprev, dt, V9(a1301), k1, V9(a1306), k6, V9(a1307), k7, V9(a1308), k8, V9(a1309),
-       k9, V9(a1310), k10, V9(a1311), k11, V9(a1312), k12);
+  comb(tmp, uprev, dt, co.a1301, k1, co.a1306, k6, co.a1307, k7, co.a1308, k8, co.a1309,
+       k9, co.a1310, k10, co.a1311, k11, co.a1312, k12);
   R::f(k13, tmp, p, ps, stage_t(t, (double)V9(c12), (double)dt));
-  comb(tmp, uprev, dt, V9(a1401), k1, V9(a1406), k6, V9(a1407), k7, V9(a1408), k8, V9(a1409),
-       k9, V9(a1410), k10, V9(a1411), k11, V9(a1412), k12, V9(a1413), k13);
+  comb(tmp, uprev, dt, co.a1401, k1, co.a1406, k6, co.a1407, k7, co.a1408, k8, co.a1409,
+       k9, co.a1410, k10, co.a1411, k11, co.a1412, k12, co.a1413, k13);
   R::f(k14, tmp, p, ps, stage_t(t, (double)V9(c13), (double)dt));
-  comb(tmp, uprev, dt, V9(a1501), k1, V9(a1506), k6, V9(a1507), k7, V9(a1508), k8, V9(a1509),
-       k9, V9(a1510), k10, V9(a1511), k11, V9(a1512), k12, V9(a1513), k13, V9(a1514), k14);
+  comb(tmp, uprev, dt, co.a1501, k1, co.a1506, k6, co.a1507, k7, co.a1508, k8, co.a1509,
+       k9, co.a1510, k10, co.a1511, k11, co.a1512, k12, co.a1513, k13, co.a1514, k14);
   T k16[N];
   if constexpr (ADAPT) {
     T g16[N];
@@ -810,12 +872,12 @@ __device__ __forceinline__ void vern9_stages(const T (&uprev)[R::N], V9S<T, R::N
   }
   if constexpr (KAHAN) {
     T acc[N];
-    lsum(acc, V9(b1), k1, V9(b8), k8, V9(b9), k9, V9(b10), k10, V9(b11), k11, V9(b12), k12,
-         V9(b13), k13, V9(b14), k14, V9(b15), k15);
+    lsum(acc, co.b1, k1, co.b8, k8, co.b9, k9, co.b10, k10, co.b11, k11, co.b12, k12,
+         co.b13, k13, co.b14, k14, co.b15, k15);
     kahan_update(u, comp_new, uprev, comp, dt, acc);
   } else {
-    comb(u, uprev, dt, V9(b1), k1, V9(b8), k8, V9(b9), k9, V9(b10), k10, V9(b11), k11, V9(b12),
-         k12, V9(b13), k13, V9(b14), k14, V9(b15), k15);
+    comb(u, uprev, dt, co.b1, k1, co.b8, k8, co.b9, k9, co.b10, k10, co.b11, k11, co.b12,
+         k12, co.b13, k13, co.b14, k14, co.b15, k15);
   }
   if constexpr (ADAPT) {
     lsum(err, V9(btilde1), k1, V9(btilde8), k8, V9(btilde9), k9, V9(btilde10), k10,
@@ -2355,6 +2417,26 @@ __device__ __forceinline__ double grid_elem(const sdeh_kargs& a, int64_t i) {
   return s + (e + lo);
 }
 
+// The coefficients of a solver's stages, held or not (none: an empty set).
+struct NoCoefs {
+  __device__ static NoCoefs init() { return {}; }
+};
+template <class T, int ALG, bool HELD>
+struct StageCoefs {
+  template <bool B, class X, class Y>
+  struct Pick { typedef X type; };
+  template <class X, class Y>
+  struct Pick<false, X, Y> { typedef Y type; };
+  static constexpr bool TS = ALG == ALG_TSIT5 || ALG == ALG_ATSIT5,
+                        V7 = ALG == ALG_VERN7 || ALG == ALG_AVERN7,
+                        V9 = ALG == ALG_VERN9 || ALG == ALG_AVERN9;
+  typedef typename Pick<HELD, TsHeld<T>, TsImm<T>>::type Tsit5;
+  typedef typename Pick<HELD, V7CHeld<T>, V7CImm<T>>::type Vern7;
+  typedef typename Pick<HELD, V9CHeld<T>, V9CImm<T>>::type Vern9;
+  typedef typename Pick<TS, Tsit5, typename Pick<V7, Vern7,
+                        typename Pick<V9, Vern9, NoCoefs>::type>::type>::type type;
+};
+
 template <class T, class R, int ALG, int SAVE>
 __device__ __forceinline__ void fixed_body(const sdeh_kargs& a) {
   static_assert(!IsWave<R>::value, "fixed-step solvers run the lane and group layouts");
@@ -2389,6 +2471,8 @@ __device__ __forceinline__ void fixed_body(const sdeh_kargs& a) {
   }
   if constexpr (SAVE == SAVE_STEPS) save_step<T, R>(a, sk, traj, t, u);
   T k7[N];
+  using Held = typename StageCoefs<T, ALG, (sizeof(T) == 8 && R::G == 1 && N <= 4)>::type;
+  const Held co = Held::init();
   if constexpr (ALG == ALG_TSIT5) R::f(k7, u, pl, ps, t);  // gpuatsit5.jl:86
   for (int64_t i = 1; i < a.g_len; ++i) {
     copyv(uprev, u);
@@ -2423,7 +2507,7 @@ __device__ __forceinline__ void fixed_body(const sdeh_kargs& a) {
     } else if constexpr (ALG == ALG_TSIT5) {
       T k1[N], k2[N], k3[N], k4[N], k5[N], k6[N];
       copyv(k1, k7);
-      tsit5_stages<T, R, false>(uprev, k1, k2, k3, k4, k5, k6, k7, u, zero, dummy, pl, ps, t, dt);
+      tsit5_stages<T, R, false>(uprev, k1, k2, k3, k4, k5, k6, k7, u, zero, dummy, pl, ps, t, dt, co);
       t += (double)dt;
       if constexpr (SAVE == SAVE_AT) {  // :116-127
         while (cur < a.n_saveat && ts_next <= t) {
@@ -2438,7 +2522,7 @@ __device__ __forceinline__ void fixed_body(const sdeh_kargs& a) {
       }
     } else if constexpr (ALG == ALG_VERN7) {
       V7K<T, N> K;
-      vern7_stages<T, R, false, false>(uprev, K, u, err, zero, dummy, pl, ps, t, dt);
+      vern7_stages<T, R, false, false>(uprev, K, u, err, zero, dummy, pl, ps, t, dt, co);
       const double told = t;
       t += (double)dt;  // gpuvern7.jl:138
       if constexpr (SAVE == SAVE_AT) {
@@ -2459,7 +2543,7 @@ __device__ __forceinline__ void fixed_body(const sdeh_kargs& a) {
     } else {
       V9S<T, N> S;
       vern9_stages<T, R, false, false, SAVE == SAVE_AT>(uprev, S, u, err, zero, dummy, pl, ps, t,
-                                                         dt, a.quirks != 0);
+                                                         dt, a.quirks != 0, co);
       const double told = t;
       t += (double)dt;  // gpuvern9.jl:185
       if constexpr (SAVE == SAVE_AT) {
