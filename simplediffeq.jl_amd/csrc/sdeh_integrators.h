@@ -622,6 +622,26 @@ SDEH_COEFS(V9C, VERN9)
 #undef SDEH_HOLD
 #undef SDEH_IMM
 
+// The coefficients of a solver's stages, held or not (none: an empty set).
+struct NoCoefs {
+  __device__ static NoCoefs init() { return {}; }
+};
+template <class T, int ALG, bool HELD>
+struct StageCoefs {
+  template <bool B, class X, class Y>
+  struct Pick { typedef X type; };
+  template <class X, class Y>
+  struct Pick<false, X, Y> { typedef Y type; };
+  static constexpr bool TS = ALG == ALG_TSIT5 || ALG == ALG_ATSIT5,
+                        V7 = ALG == ALG_VERN7 || ALG == ALG_AVERN7,
+                        V9 = ALG == ALG_VERN9 || ALG == ALG_AVERN9;
+  typedef typename Pick<HELD, TsHeld<T>, TsImm<T>>::type Tsit5;
+  typedef typename Pick<HELD, V7CHeld<T>, V7CImm<T>>::type Vern7;
+  typedef typename Pick<HELD, V9CHeld<T>, V9CImm<T>>::type Vern9;
+  typedef typename Pick<TS, Tsit5, typename Pick<V7, Vern7,
+                        typename Pick<V9, Vern9, NoCoefs>::type>::type>::type type;
+};
+
 #define TS(x) T(sdeh_tab::tsit5::x)
 
 // Tsit5 stages k2..k7 from k1 (FSAL); gpuatsit5.jl:99-110 / 258-270.
@@ -1417,6 +1437,18 @@ __device__ __forceinline__ X in_vgpr_if(X x) {
   return x;
 }
 
+// The kernel's arguments read again from the kernarg segment, at the places that a
+// trajectory passes only once: the pointers of inputs and outputs then hold no scalar
+// registers in the loop between: the one-lane binary64 kernels keep 12 spilled ones (34
+// before) and have room to hold their stages' coefficients.  Lorenz: 1,024 ATsit5 37.4 /
+// 34.7 us, 2^20 uneven AVern7 9,440 / 9,190 us, the large ATsit5 ensembles as before.
+// (Every kernel takes sdeh_kargs first and by value.)
+__device__ __forceinline__ const sdeh_kargs& cold_args(const sdeh_kargs&) {
+  auto k = __builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(k));
+  return *(const sdeh_kargs*)k;
+}
+
 // Claim queue slots for the lanes flagged in `need` (called in uniform control
 // flow by the whole wave).  Returns this lane's slot or -1.  `base`/`lim` is
 // the wave's current claimed range of `chunk` slots; `drained` becomes true once
@@ -1928,6 +1960,7 @@ __device__ __forceinline__ void adaptive_body(const sdeh_kargs& a) {
   }
   constexpr int N = R::N;
   constexpr int P = R::P > 0 ? R::P : 1;
+  constexpr bool HOLD = sizeof(T) == 8 && R::G == 1 && N <= 4;
   constexpr double DTMIN = (ALG == ALG_AVERN9) ? (double)1.0e-7f : 1.0e-14;  // gpuvern9.jl:466
   constexpr double SNAP = DTMIN;                                              // gpuvern9.jl:591
   // build_adaptive_controller_cache(T), src/SimpleDiffEq.jl:67-77
@@ -1981,6 +2014,9 @@ __device__ __forceinline__ void adaptive_body(const sdeh_kargs& a) {
                                               ? (int64_t)a.stage_cap
                                               : a.maxiters);
 
+  using Coefs = typename StageCoefs<T, ALG, HOLD>::type;
+  const Coefs coef = Coefs::init();
+
   for (;;) {
     if constexpr (RUNS) {
       // Sectors in LDS: each once it is full; the begun ones of ended trajectories
@@ -2005,16 +2041,16 @@ __device__ __forceinline__ void adaptive_body(const sdeh_kargs& a) {
       for (;;) {
         int64_t slot, claimed = -1;
         if constexpr (ORDER_WIN)
-          slot = wave_claim_win(a, want, qbase, qlim, drained, qwin, qword, claimed);
+          slot = wave_claim_win(cold_args(a), want, qbase, qlim, drained, qwin, qword, claimed);
         else
-          slot = wave_claim(a, want, qbase, qlim, drained);
+          slot = wave_claim(cold_args(a), want, qbase, qlim, drained);
         if constexpr (R::G > 1)  // the group leader claimed; its group follows
           slot = (int64_t)__shfl((long long)slot, (int)(__lane_id() & ~(unsigned)(R::G - 1)));
         if (slot >= 0) {
-          traj = ORDER_WIN ? claimed : slot_traj(a, slot);
+          traj = ORDER_WIN ? claimed : slot_traj(cold_args(a), slot);
           active = fresh = traj >= 0;
           // a resumed launch skips the trajectories that ended in the first stage
-          if (STAGED && a.resume && active && Park::flag(a, traj) == 0) active = fresh = false;
+          if (STAGED && a.resume && active && Park::flag(cold_args(a), traj) == 0) active = fresh = false;
         }
         want = !active && lead;
         if (!STAGED || !a.resume || drained || __ballot(want && slot >= 0) == 0ull) break;
@@ -2025,34 +2061,37 @@ __device__ __forceinline__ void adaptive_body(const sdeh_kargs& a) {
 
     if (fresh && STAGED && a.resume) {  // continue a parked trajectory
       fresh = false;
-      note_visit(a, traj);
-      Park::load(a, traj, uprev, fsal, comp, pl, t, tf, dt, qold_pow, nacc, nrej);
+      const sdeh_kargs& ka = cold_args(a);
+      note_visit(ka, traj);
+      Park::load(ka, traj, uprev, fsal, comp, pl, t, tf, dt, qold_pow, nacc, nrej);
       attempts = (int64_t)nacc + nrej;
       cur = 0;
     }
     if (fresh) {  // start trajectory `traj` (gpuatsit5.jl:221-241)
       fresh = false;
-      if (lead) note_visit(a, traj);
-      load_state<T, R>(uprev, a.u0, n, traj);
+      const sdeh_kargs& ka = cold_args(a);
+      const int64_t n = ka.n;
+      if (lead) note_visit(ka, traj);
+      load_state<T, R>(uprev, ka.u0, n, traj);
 #pragma unroll
       for (int c = 0; c < N; ++c) comp[c] = T(0);
-      load_params<T, R>(pl, a, traj);
-      t = a.tspan ? a.tspan[traj] : a.t0;
-      tf = a.tspan ? a.tspan[n + traj] : a.tf;
-      dt = (T)(a.dt0 ? a.dt0[traj] : a.dt);
+      load_params<T, R>(pl, ka, traj);
+      t = ka.tspan ? ka.tspan[traj] : ka.t0;
+      tf = ka.tspan ? ka.tspan[n + traj] : ka.tf;
+      dt = (T)(ka.dt0 ? ka.dt0[traj] : ka.dt);
       qold_pow = qoldinit_pow;
       nacc = nrej = 0;
       attempts = 0;
       cur = 0;
       if constexpr (SAVE == SAVE_AT) {
-        if (a.n_saveat > 0 && t == a.saveat[0]) {
+        if (a.n_saveat > 0 && t == ka.saveat[0]) {
           store_save<T, R>(a, a.u_saveat, 0, a.n_saveat, traj, uprev);
           cur = 1;
         }
         ts_next = saves_at.at(a, cur);
       }
       if constexpr (STEPS) {
-        sink_start<R>(a, sk, traj);
+        sink_start<R>(ka, sk, traj);
         save_step<T, R, RUNS>(a, sk, traj, t, uprev);
       }
       if constexpr (ALG == ALG_ATSIT5) R::f(fsal, uprev, pl, ps, t);  // FSAL seed, :241
@@ -2064,7 +2103,7 @@ __device__ __forceinline__ void adaptive_body(const sdeh_kargs& a) {
     } else if ((double)dt < DTMIN) {  // :256
       ret = RET_DTMIN;
     } else if (attempts >= att_lim) {  // maxiters, or the first stage's cap (parked)
-      ret = attempts >= a.maxiters ? RET_MAXITERS : RET_PARKED;
+      ret = attempts >= cold_args(a).maxiters ? RET_MAXITERS : RET_PARKED;
     } else {
       ++attempts;
       T u[N], err[N], comp_new[N];
@@ -2075,7 +2114,7 @@ __device__ __forceinline__ void adaptive_body(const sdeh_kargs& a) {
       V9S<T, N> S9;                                 // AVern9 stages
       if constexpr (ALG == ALG_ATSIT5) {
         tsit5_stages<T, R, KAHAN>(uprev, fsal, k2, k3, k4, k5, k6, k7, u, comp, comp_new, pl,
-                                  ps, t, dt);
+                                  ps, t, dt, coef);
         // dt * (btilde1*k1 + ... + btilde7*k7), gpuatsit5.jl:272-275
         lsum(err, T(sdeh_tab::tsit5::btilde1), fsal, T(sdeh_tab::tsit5::btilde2), k2,
              T(sdeh_tab::tsit5::btilde3), k3, T(sdeh_tab::tsit5::btilde4), k4,
@@ -2085,9 +2124,9 @@ __device__ __forceinline__ void adaptive_body(const sdeh_kargs& a) {
         // Verner: k1 is evaluated at the start of every attempt (gpuvern7.jl:360,
         // gpuvern9.jl:468).
         vern9_stages<T, R, true, KAHAN, SAVE == SAVE_AT>(uprev, S9, u, err, comp, comp_new, pl,
-                                                          ps, t, dt, false);
+                                                          ps, t, dt, false, coef);
       } else {
-        vern7_stages<T, R, true, KAHAN>(uprev, K7, u, err, comp, comp_new, pl, ps, t, dt);
+        vern7_stages<T, R, true, KAHAN>(uprev, K7, u, err, comp, comp_new, pl, ps, t, dt, coef);
       }
 #pragma unroll
       for (int c = 0; c < N; ++c) err[c] = dt * err[c];
@@ -2187,31 +2226,33 @@ __device__ __forceinline__ void adaptive_body(const sdeh_kargs& a) {
     }
 
     if (ret != -1) {  // trajectory ends or parks: write outputs (gpuatsit5.jl:322-329)
+      const sdeh_kargs& ka = cold_args(a);
+      const int64_t n = ka.n;
       if (STEPS && ret == RET_DEFAULT && sk.kept < sk.n) ret = RET_SAVE_OVERFLOW;
       const bool parked = STAGED && ret == RET_PARKED;
       if (!parked) {
-        store_state<T, R>(a.u_end, 0, n, traj, uprev);
-        if constexpr (SAVE == SAVE_AT) save_unreached<T, R>(a, cur, traj);
-        if constexpr (SAVE == SAVE_STEPS) flush_steps<T, R>(a, sk);
+        store_state<T, R>(ka.u_end, 0, n, traj, uprev);
+        if constexpr (SAVE == SAVE_AT) save_unreached<T, R>(ka, cur, traj);
+        if constexpr (SAVE == SAVE_STEPS) flush_steps<T, R>(ka, sk);
         if (lead) {
-          a.t_end[traj] = t;
-          a.retcode[traj] = ret;
-          if (a.naccept) a.naccept[traj] = nacc;
-          if (a.nreject) a.nreject[traj] = nrej;
-          if constexpr (STEPS) finish_steps(a, sk, traj);
+          ka.t_end[traj] = t;
+          ka.retcode[traj] = ret;
+          if (ka.naccept) ka.naccept[traj] = nacc;
+          if (ka.nreject) ka.nreject[traj] = nrej;
+          if constexpr (STEPS) finish_steps(ka, sk, traj);
         }
       }
-      if (STAGED && a.stage_cap > 0) {
+      if (STAGED && ka.stage_cap > 0) {
         double key = 0.0;
         if (parked) {
-          Park::store(a, traj, uprev, fsal, comp, pl, t, tf, dt, qold_pow, nacc, nrej);
+          Park::store(ka, traj, uprev, fsal, comp, pl, t, tf, dt, qold_pow, nacc, nrej);
           // remaining attempts extrapolated from the first stage's progress
-          const double t0 = a.tspan ? a.tspan[traj] : a.t0;
-          key = (double)a.stage_cap * ((tf - t) / (t - t0));
+          const double t0 = ka.tspan ? ka.tspan[traj] : ka.t0;
+          key = (double)ka.stage_cap * ((tf - t) / (t - t0));
         } else {
-          Park::set_flag(a, traj, 0);
+          Park::set_flag(ka, traj, 0);
         }
-        a.st_key[traj] = key;
+        ka.st_key[traj] = key;
       }
       active = false;
     }
@@ -2416,26 +2457,6 @@ __device__ __forceinline__ double grid_elem(const sdeh_kargs& a, int64_t i) {
   const double e = (a.g_start - (s - bb)) + (hi - bb);
   return s + (e + lo);
 }
-
-// The coefficients of a solver's stages, held or not (none: an empty set).
-struct NoCoefs {
-  __device__ static NoCoefs init() { return {}; }
-};
-template <class T, int ALG, bool HELD>
-struct StageCoefs {
-  template <bool B, class X, class Y>
-  struct Pick { typedef X type; };
-  template <class X, class Y>
-  struct Pick<false, X, Y> { typedef Y type; };
-  static constexpr bool TS = ALG == ALG_TSIT5 || ALG == ALG_ATSIT5,
-                        V7 = ALG == ALG_VERN7 || ALG == ALG_AVERN7,
-                        V9 = ALG == ALG_VERN9 || ALG == ALG_AVERN9;
-  typedef typename Pick<HELD, TsHeld<T>, TsImm<T>>::type Tsit5;
-  typedef typename Pick<HELD, V7CHeld<T>, V7CImm<T>>::type Vern7;
-  typedef typename Pick<HELD, V9CHeld<T>, V9CImm<T>>::type Vern9;
-  typedef typename Pick<TS, Tsit5, typename Pick<V7, Vern7,
-                        typename Pick<V9, Vern9, NoCoefs>::type>::type>::type type;
-};
 
 template <class T, class R, int ALG, int SAVE>
 __device__ __forceinline__ void fixed_body(const sdeh_kargs& a) {
