@@ -29,8 +29,15 @@ const void* adaptive_ptr() {
 // the adaptive endpoint kernels of ATsit5 and AVern7 at 4, 6 and 8 waves per SIMD,
 // for the autotuner; waves = 0 is the default kernel.
 
+// waves = 1: the binary64 kernels of small states for ensembles of a wave or two per SIMD.
+
 template <class T, int ALG, bool KAHAN>
 const void* waves_variant(int waves) {
+#if !defined(SDEH_LIMITED) && !defined(SDEH_WAVE_ONLY)
+  if constexpr (sizeof(T) == 8 && !KAHAN && R::G == 1 && R::N <= 4) {
+    if (waves == 1) return adaptive_ptr<T, ALG, sdeh::SAVE_END, KAHAN, 1>();
+  }
+#endif
 #if defined(SDEH_WAVE_VARIANTS)
   if constexpr (ALG == sdeh::ALG_ATSIT5 || ALG == sdeh::ALG_AVERN7) {
     switch (waves) {

@@ -161,6 +161,15 @@ struct Ops<float> {
   }
 };
 
+// A loop-invariant value held in vector registers.  The one-lane kernels run out
+// of scalar registers first; a scalar the compiler spills is reloaded with a
+// v_readlane (a vector instruction) on every attempt that uses it.
+template <class X>
+__device__ __forceinline__ X in_vgpr(X x) {
+  asm volatile("" : "+v"(x));
+  return x;
+}
+
 // The reduction tables of the binary64 controller's pow in LDS, one array per column
 // (5 KB per block, copied when the kernel starts; every thread of the block calls init).
 // Each attempt gathers three rows at 64 unrelated indices, one after the other.  From
@@ -170,6 +179,7 @@ struct Ops<float> {
 // 37.7 / 35.0 us.
 struct LdsTab {
   const double* t;
+  __device__ double c(int k) const { return sdeh_math::pow_const(k); }
   __device__ void log_row(int i, double* invc, double* lh, double* ll) const {
     *invc = t[i];
     *lh = t[128 + i];
@@ -193,9 +203,22 @@ struct LdsTab {
   }
 };
 // The tables of a kernel: in LDS where ON (binary64), else the constant arrays.
-template <bool ON>
+// The same with the constants of the logarithm and exponential in vector registers.
+struct LoneTab : LdsTab {
+  double k[sdeh_math::PC_COUNT];
+  __device__ double c(int i) const { return k[i]; }
+  __device__ static LoneTab init() {
+    LoneTab tab;
+    tab.t = LdsTab::init().t;
+#pragma unroll
+    for (int i = 0; i < sdeh_math::PC_COUNT; ++i) tab.k[i] = in_vgpr(sdeh_math::pow_const(i));
+    return tab;
+  }
+};
+template <bool ON, bool LONE = false>
 __device__ __forceinline__ auto pow_tables() {
-  if constexpr (ON) return LdsTab::init();
+  if constexpr (ON && LONE) return LoneTab::init();
+  else if constexpr (ON) return LdsTab::init();
   else return sdeh_math::ConstTab{};
 }
 
@@ -569,13 +592,15 @@ __device__ __forceinline__ T poly2(T th, const T (&r)[NR]) {
 #define SDEH_TSIT5_HELD(X)                                                                      \
   X(a21) X(a31) X(a32) X(a41) X(a42) X(a43) X(a51) X(a52) X(a53) X(a54) X(a61) X(a62) X(a63)    \
   X(a64) X(a65) X(a71) X(a72) X(a73) X(a74) X(a75) X(a76)
-#define SDEH_TSIT5_REST(X)
+#define SDEH_TSIT5_REST(X)                                                                      \
+  X(btilde1) X(btilde2) X(btilde3) X(btilde4) X(btilde5) X(btilde6) X(btilde7)
 #define SDEH_VERN7_HELD(X)                                                                      \
   X(a021) X(a031) X(a032) X(a041) X(a043) X(a051) X(a053) X(a054) X(a061) X(a063) X(a064)       \
   X(a065) X(a071) X(a073) X(a074) X(a075) X(a076) X(a081) X(a083) X(a084) X(a085)
 #define SDEH_VERN7_REST(X)                                                                      \
   X(a086) X(a087) X(a091) X(a093) X(a094) X(a095) X(a096) X(a097) X(a098) X(b1) X(b4) X(b5)     \
-  X(b6) X(b7) X(b8) X(b9)
+  X(b6) X(b7) X(b8) X(b9) X(a101) X(a103) X(a104) X(a105) X(a106) X(a107) X(btilde1)            \
+  X(btilde4) X(btilde5) X(btilde6) X(btilde7) X(btilde8) X(btilde9) X(btilde10)
 #define SDEH_VERN9_HELD(X)                                                                      \
   X(a0201) X(a0301) X(a0302) X(a0401) X(a0403) X(a0501) X(a0503) X(a0504) X(a0601) X(a0604)     \
   X(a0605) X(a0701) X(a0704) X(a0705) X(a0706) X(a0801) X(a0806) X(a0807) X(a0901) X(a0906)     \
@@ -586,7 +611,9 @@ __device__ __forceinline__ T poly2(T th, const T (&r)[NR]) {
   X(a1306) X(a1307) X(a1308) X(a1309) X(a1310) X(a1311) X(a1312) X(a1401) X(a1406) X(a1407)     \
   X(a1408) X(a1409) X(a1410) X(a1411) X(a1412) X(a1413) X(a1501) X(a1506) X(a1507) X(a1508)     \
   X(a1509) X(a1510) X(a1511) X(a1512) X(a1513) X(a1514) X(b1) X(b8) X(b9) X(b10) X(b11)         \
-  X(b12) X(b13) X(b14) X(b15)
+  X(b12) X(b13) X(b14) X(b15) X(a1601) X(a1606) X(a1607) X(a1608) X(a1609) X(a1610) X(a1611)    \
+  X(a1612) X(a1613) X(btilde1) X(btilde8) X(btilde9) X(btilde10) X(btilde11) X(btilde12)        \
+  X(btilde13) X(btilde14) X(btilde15) X(btilde16)
 template <class X>
 __device__ __forceinline__ X in_sgpr(X x) {
   asm volatile("" : "+s"(x));
@@ -594,6 +621,7 @@ __device__ __forceinline__ X in_sgpr(X x) {
 }
 #define SDEH_IMM(n) T n = T(TAB::n);
 #define SDEH_HOLD(n) k.n = in_sgpr(k.n);
+#define SDEH_HOLD_V(n) k.n = in_vgpr(k.n);
 #define SDEH_COEFS(NAME, LIST)                          \
   template <class T>                                    \
   struct NAME##Imm {                                    \
@@ -608,6 +636,15 @@ __device__ __forceinline__ X in_sgpr(X x) {
       SDEH_##LIST##_HELD(SDEH_HOLD)                     \
       return k;                                         \
     }                                                   \
+  };                                                    \
+  template <class T>                                    \
+  struct NAME##Lone {                                   \
+    SDEH_##LIST##_HELD(SDEH_IMM) SDEH_##LIST##_REST(SDEH_IMM) \
+    __device__ static NAME##Lone init() {               \
+      NAME##Lone k;                                     \
+      SDEH_##LIST##_HELD(SDEH_HOLD) SDEH_##LIST##_REST(SDEH_HOLD_V) \
+      return k;                                         \
+    }                                                   \
   };
 #define TAB sdeh_tab::tsit5
 SDEH_COEFS(Ts, TSIT5)
@@ -620,13 +657,14 @@ SDEH_COEFS(V9C, VERN9)
 #undef TAB
 #undef SDEH_COEFS
 #undef SDEH_HOLD
+#undef SDEH_HOLD_V
 #undef SDEH_IMM
 
 // The coefficients of a solver's stages, held or not (none: an empty set).
 struct NoCoefs {
   __device__ static NoCoefs init() { return {}; }
 };
-template <class T, int ALG, bool HELD>
+template <class T, int ALG, bool HELD, bool LONE = false>
 struct StageCoefs {
   template <bool B, class X, class Y>
   struct Pick { typedef X type; };
@@ -635,9 +673,9 @@ struct StageCoefs {
   static constexpr bool TS = ALG == ALG_TSIT5 || ALG == ALG_ATSIT5,
                         V7 = ALG == ALG_VERN7 || ALG == ALG_AVERN7,
                         V9 = ALG == ALG_VERN9 || ALG == ALG_AVERN9;
-  typedef typename Pick<HELD, TsHeld<T>, TsImm<T>>::type Tsit5;
-  typedef typename Pick<HELD, V7CHeld<T>, V7CImm<T>>::type Vern7;
-  typedef typename Pick<HELD, V9CHeld<T>, V9CImm<T>>::type Vern9;
+  typedef typename Pick<LONE, TsLone<T>, typename Pick<HELD, TsHeld<T>, TsImm<T>>::type>::type Tsit5;
+  typedef typename Pick<LONE, V7CLone<T>, typename Pick<HELD, V7CHeld<T>, V7CImm<T>>::type>::type Vern7;
+  typedef typename Pick<LONE, V9CLone<T>, typename Pick<HELD, V9CHeld<T>, V9CImm<T>>::type>::type Vern9;
   typedef typename Pick<TS, Tsit5, typename Pick<V7, Vern7,
                         typename Pick<V9, Vern9, NoCoefs>::type>::type>::type type;
 };
@@ -743,8 +781,8 @@ __device__ __forceinline__ void vern7_stages(const T (&uprev)[R::N], V7K<T, R::N
   T k10[N];
   if constexpr (ADAPT) {
     T g10[N];
-    comb(g10, uprev, dt, V7(a101), K.k1, V7(a103), k3, V7(a104), K.k4, V7(a105), K.k5,
-         V7(a106), K.k6, V7(a107), K.k7);
+    comb(g10, uprev, dt, co.a101, K.k1, co.a103, k3, co.a104, K.k4, co.a105, K.k5,
+         co.a106, K.k6, co.a107, K.k7);
     R::f(K.k9, tmp, p, ps, t + (double)dt);
     R::f(k10, g10, p, ps, t + (double)dt);
   } else {
@@ -760,8 +798,8 @@ __device__ __forceinline__ void vern7_stages(const T (&uprev)[R::N], V7K<T, R::N
          co.b8, K.k8, co.b9, K.k9);
   }
   if constexpr (ADAPT) {
-    lsum(err, V7(btilde1), K.k1, V7(btilde4), K.k4, V7(btilde5), K.k5, V7(btilde6), K.k6,
-         V7(btilde7), K.k7, V7(btilde8), K.k8, V7(btilde9), K.k9, V7(btilde10), k10);
+    lsum(err, co.btilde1, K.k1, co.btilde4, K.k4, co.btilde5, K.k5, co.btilde6, K.k6,
+         co.btilde7, K.k7, co.btilde8, K.k8, co.btilde9, K.k9, co.btilde10, k10);
   }
 }
 
@@ -883,8 +921,8 @@ __device__ __forceinline__ void vern9_stages(const T (&uprev)[R::N], V9S<T, R::N
   T k16[N];
   if constexpr (ADAPT) {
     T g16[N];
-    comb(g16, uprev, dt, V9(a1601), k1, V9(a1606), k6, V9(a1607), k7, V9(a1608), k8,
-         V9(a1609), k9, V9(a1610), k10, V9(a1611), k11, V9(a1612), k12, V9(a1613), k13);
+    comb(g16, uprev, dt, co.a1601, k1, co.a1606, k6, co.a1607, k7, co.a1608, k8,
+         co.a1609, k9, co.a1610, k10, co.a1611, k11, co.a1612, k12, co.a1613, k13);
     R::f(k15, tmp, p, ps, t + (double)dt);
     R::f(k16, g16, p, ps, t + (double)dt);
   } else {
@@ -900,9 +938,9 @@ __device__ __forceinline__ void vern9_stages(const T (&uprev)[R::N], V9S<T, R::N
          k12, co.b13, k13, co.b14, k14, co.b15, k15);
   }
   if constexpr (ADAPT) {
-    lsum(err, V9(btilde1), k1, V9(btilde8), k8, V9(btilde9), k9, V9(btilde10), k10,
-         V9(btilde11), k11, V9(btilde12), k12, V9(btilde13), k13, V9(btilde14), k14,
-         V9(btilde15), k15, V9(btilde16), k16);
+    lsum(err, co.btilde1, k1, co.btilde8, k8, co.btilde9, k9, co.btilde10, k10,
+         co.btilde11, k11, co.btilde12, k12, co.btilde13, k13, co.btilde14, k14,
+         co.btilde15, k15, co.btilde16, k16);
   }
   if constexpr (KEEP) {
     copyv(S.s[0], k1);
@@ -1420,14 +1458,6 @@ __device__ __forceinline__ T nan_of() {
 // ---------------------------------------------------------------------------
 // Wave-level work queue for the persistent schedule.
 // ---------------------------------------------------------------------------
-// A loop-invariant value held in vector registers.  The one-lane kernels run out
-// of scalar registers first; a scalar the compiler spills is reloaded with a
-// v_readlane (a vector instruction) on every attempt that uses it.
-template <class X>
-__device__ __forceinline__ X in_vgpr(X x) {
-  asm volatile("" : "+v"(x));
-  return x;
-}
 // in_vgpr where it costs no occupancy: in the binary64 endpoint kernels (the
 // binary32 ones have scalar registers to spare and would cross 64 vector registers,
 // and the save modes' kernels would lose a wave per SIMD).
@@ -1952,7 +1982,7 @@ struct ParkRec {
   }
 };
 
-template <class T, class R, int ALG, int SAVE, bool KAHAN>
+template <class T, class R, int ALG, int SAVE, bool KAHAN, bool LONE = false>
 __device__ __forceinline__ void adaptive_body(const sdeh_kargs& a) {
   if constexpr (IsWave<R>::value) {
     adaptive_body_wave<T, R, ALG, SAVE, KAHAN>(a);
@@ -1968,12 +1998,20 @@ __device__ __forceinline__ void adaptive_body(const sdeh_kargs& a) {
           gamma = T(9.0 / 10), qoldinit = T(1.0e-4);
   const T inv_qmax = T(1) / qmax, inv_qmin = T(1) / qmin;
   const T qoldinit_pow = Ops<T>::pw(qoldinit, beta2);
-  const auto tab = pow_tables<sizeof(T) == 8>();
+  const auto tab = pow_tables<sizeof(T) == 8, LONE>();
   const auto saves_at = SaveTimes<SAVE == SAVE_AT>::init(a);
   constexpr bool PIN = sizeof(T) == 8 && SAVE == SAVE_END;
   const T abstol = in_vgpr_if<PIN>((T)a.abstol), reltol = in_vgpr_if<PIN>((T)a.reltol);
-  const CtrlK<T> ck{beta1, beta2, inv_qmax, inv_qmin, gamma, Ops<T>::rcp_nr(T(NormLen<R>::value)),
-                    Ops<T>::rcp_nr(gamma)};
+  CtrlK<T> ck{beta1, beta2, inv_qmax, inv_qmin, gamma, Ops<T>::rcp_nr(T(NormLen<R>::value)),
+              Ops<T>::rcp_nr(gamma)};
+  if constexpr (LONE) {
+    ck.beta1 = in_vgpr(ck.beta1);
+    ck.beta2 = in_vgpr(ck.beta2);
+    ck.inv_qmin = in_vgpr(ck.inv_qmin);
+    ck.gamma = in_vgpr(ck.gamma);
+    ck.r_len = in_vgpr(ck.r_len);
+    ck.r_gamma = in_vgpr(ck.r_gamma);
+  }
   const T* ps = (const T*)a.ps;
   const int64_t n = a.n;
 
@@ -2014,7 +2052,7 @@ __device__ __forceinline__ void adaptive_body(const sdeh_kargs& a) {
                                               ? (int64_t)a.stage_cap
                                               : a.maxiters);
 
-  using Coefs = typename StageCoefs<T, ALG, HOLD>::type;
+  using Coefs = typename StageCoefs<T, ALG, HOLD, LONE>::type;
   const Coefs coef = Coefs::init();
 
   for (;;) {
@@ -2116,10 +2154,10 @@ __device__ __forceinline__ void adaptive_body(const sdeh_kargs& a) {
         tsit5_stages<T, R, KAHAN>(uprev, fsal, k2, k3, k4, k5, k6, k7, u, comp, comp_new, pl,
                                   ps, t, dt, coef);
         // dt * (btilde1*k1 + ... + btilde7*k7), gpuatsit5.jl:272-275
-        lsum(err, T(sdeh_tab::tsit5::btilde1), fsal, T(sdeh_tab::tsit5::btilde2), k2,
-             T(sdeh_tab::tsit5::btilde3), k3, T(sdeh_tab::tsit5::btilde4), k4,
-             T(sdeh_tab::tsit5::btilde5), k5, T(sdeh_tab::tsit5::btilde6), k6,
-             T(sdeh_tab::tsit5::btilde7), k7);
+        lsum(err, coef.btilde1, fsal, coef.btilde2, k2,
+             coef.btilde3, k3, coef.btilde4, k4,
+             coef.btilde5, k5, coef.btilde6, k6,
+             coef.btilde7, k7);
       } else if constexpr (V9) {
         // Verner: k1 is evaluated at the start of every attempt (gpuvern7.jl:360,
         // gpuvern9.jl:468).
@@ -2622,13 +2660,15 @@ struct WavesHint {
 // ahead-of-time translation unit and by the hipRTC wrapper.  WAVES > 0 asks the
 // compiler for that many waves per SIMD instead of the WavesHint default (at most
 // 512 / WAVES VGPRs per lane, in steps of 8): the autotuner's register-cap
-// variants of the same arithmetic.
+// variants of the same arithmetic.  WAVES = 1 (LONE): for ensembles of a wave or two per
+// SIMD, which waits out each constant's scalar moves and has vector registers to spare:
+// every coefficient and constant of an attempt stays in registers.
 template <class T, class R, int ALG, int SAVE, bool KAHAN, int WAVES = 0>
 __global__ void __launch_bounds__(256)
     __attribute__((amdgpu_waves_per_eu(WAVES > 0 ? WAVES
                                                  : sdeh::WavesHint<T, R, ALG, SAVE>::value)))
     sdeh_adaptive_kernel(sdeh_kargs a) {
-  sdeh::adaptive_body<T, R, ALG, SAVE, KAHAN>(a);
+  sdeh::adaptive_body<T, R, ALG, SAVE, KAHAN, WAVES == 1>(a);
 }
 
 // TPL trajectories per lane (adaptive_body_multi).

@@ -100,7 +100,26 @@ SDEH_HD inline T fast_max(T x, T y) { return y > x ? y : x; }
 // log_norm_dd is the core for a normal x scaled by 2^-kadj (log of x * 2^kadj);
 // log_pos_dd scales subnormal inputs into the normal range first.
 // `tab` holds the reduction tables (ConstTab: the constant arrays).
+// The logarithm's and exponential's constants, by number, so that a table type can keep them
+// in registers.
+enum PowConst {
+  PC_LN2_HI, PC_LN2_LO, PC_L9, PC_L8, PC_L7, PC_L6, PC_L5, PC_L4, PC_L3,  // -1/9, 1/8, ... -1/3
+  PC_INV_LN2N, PC_LN2N_HI, PC_LN2N_LO, PC_E720, PC_E120, PC_E24, PC_E6,   // 1/720 ... 1/6
+  PC_COUNT
+};
+SDEH_HD constexpr double pow_const(int k) {
+  return k == PC_LN2_HI ? sdeh_powtab::LN2_HI : k == PC_LN2_LO ? sdeh_powtab::LN2_LO
+       : k == PC_L9 ? -0x1.c71c71c71c71cp-4 : k == PC_L8 ? 0x1p-3
+       : k == PC_L7 ? -0x1.2492492492492p-3 : k == PC_L6 ? 0x1.5555555555555p-3
+       : k == PC_L5 ? -0x1.999999999999ap-3 : k == PC_L4 ? 0x1p-2
+       : k == PC_L3 ? -0x1.5555555555555p-2 : k == PC_INV_LN2N ? sdeh_powtab::INV_LN2N
+       : k == PC_LN2N_HI ? sdeh_powtab::LN2N_HI : k == PC_LN2N_LO ? sdeh_powtab::LN2N_LO
+       : k == PC_E720 ? 0x1.6c16c16c16c17p-10 : k == PC_E120 ? 0x1.1111111111111p-7
+       : k == PC_E24 ? 0x1.5555555555555p-5 : 0x1.5555555555555p-3;
+}
+
 struct ConstTab {
+  SDEH_HD double c(int k) const { return pow_const(k); }
   SDEH_HD void log_row(int i, double* invc, double* lh, double* ll) const {
     *invc = sdeh_powtab::LOG_TAB[i][0];
     *lh = sdeh_powtab::LOG_TAB[i][1];
@@ -121,7 +140,7 @@ SDEH_HD inline void log_reduced_dd(int i, int k, double z, double* hi, double* l
   tab.log_row(i, &invc, &lh, &ll);
   const double r = fma(z, invc, -1.0);  // exact
   const double dk = (double)k;
-  const double a = dk * LN2_HI;  // exact
+  const double a = dk * tab.c(PC_LN2_HI);  // exact
   // s1 + e1 = a + lh (|a| >= ln 2 > |lh| unless k == 0)
   const double s1 = a + lh;
   const double e1 = (a - s1) + lh;
@@ -137,15 +156,15 @@ SDEH_HD inline void log_reduced_dd(int i, int k, double z, double* hi, double* l
   // otherwise |s2| > 2^-9 > r^2/2)
   const double h = s2 + ar2;
   const double e4 = (s2 - h) + ar2;
-  double p = -0x1.c71c71c71c71cp-4;      // -1/9
-  p = fma(p, r, 0x1p-3);                 //  1/8
-  p = fma(p, r, -0x1.2492492492492p-3);  // -1/7
-  p = fma(p, r, 0x1.5555555555555p-3);   //  1/6
-  p = fma(p, r, -0x1.999999999999ap-3);  // -1/5
-  p = fma(p, r, 0x1p-2);                 //  1/4
-  p = fma(p, r, -0x1.5555555555555p-2);  // -1/3
+  double p = tab.c(PC_L9);
+  p = fma(p, r, tab.c(PC_L8));
+  p = fma(p, r, tab.c(PC_L7));
+  p = fma(p, r, tab.c(PC_L6));
+  p = fma(p, r, tab.c(PC_L5));
+  p = fma(p, r, tab.c(PC_L4));
+  p = fma(p, r, tab.c(PC_L3));
   const double r3 = (r * r) * r;
-  const double t = fma(-r3, p, fma(dk, LN2_LO, ll)) + ((e1 + e2) + (e3 + e4));
+  const double t = fma(-r3, p, fma(dk, tab.c(PC_LN2_LO), ll)) + ((e1 + e2) + (e3 + e4));
   const double y = h + t;
   *hi = y;
   *lo = (h - y) + t;
@@ -179,14 +198,14 @@ SDEH_HD inline void log_pos_dd(double x, double* hi, double* lo) {
 template <class Tab = ConstTab>
 SDEH_HD inline double exp_core(double zc, double zl, int* m_out, const Tab& tab = Tab()) {
   using namespace sdeh_powtab;
-  const double nd = __builtin_rint(zc * INV_LN2N);
+  const double nd = __builtin_rint(zc * tab.c(PC_INV_LN2N));
   const int n = (int)nd;
-  const double r0 = fma(-nd, LN2N_HI, zc);  // exact
-  const double u = r0 + fma(-nd, LN2N_LO, zl);
-  double q = 0x1.6c16c16c16c17p-10;   // 1/720
-  q = fma(q, u, 0x1.1111111111111p-7);  // 1/120
-  q = fma(q, u, 0x1.5555555555555p-5);  // 1/24
-  q = fma(q, u, 0x1.5555555555555p-3);  // 1/6
+  const double r0 = fma(-nd, tab.c(PC_LN2N_HI), zc);  // exact
+  const double u = r0 + fma(-nd, tab.c(PC_LN2N_LO), zl);
+  double q = tab.c(PC_E720);
+  q = fma(q, u, tab.c(PC_E120));
+  q = fma(q, u, tab.c(PC_E24));
+  q = fma(q, u, tab.c(PC_E6));
   q = fma(q, u, 0.5);
   const double em1 = fma(u * u, q, u);
   const int j = n & EXP_MASK;

@@ -844,6 +844,21 @@ int plan_solve(sdeh_ctx* c, const sdeh_solve_desc* d, const sdeh_io* io, Plan* p
       sh.waves = w;
       sh.per_lane = tp;
       pl->default_staged = sh.schedule == SDEH_SCHED_STAGED;
+      // The kernel that keeps its constants in registers, for ensembles of a wave or two
+      // per SIMD (AVern9: one, its 302 registers allow no second).  Lorenz, the default
+      // kernel | this one (us; ATsit5, AVern7, AVern9):
+      //      1,024    89 | 81     197 | 162     391 | 354
+      //     65,536    95 | 86     204 | 165     412 | 370
+      //    131,072   127 | 122    274 | 250     561 | 782
+      //    262,144   205 | 242    467 | 474     951 | 1,252
+      const int64_t simds = 4 * (int64_t)c->cus;
+      if (sh.schedule == SDEH_SCHED_ONE_LAUNCH && pl->save == SAVE_END && !pl->packed &&
+          d->dtype == SDEH_F64 && adaptive && pl->k.lanes == 1 && !w && tp <= 1 &&
+          d->n_traj <= simds * 64 * (d->alg == SDEH_ALG_AVERN9 ? 1 : 2)) {
+        const Builtin* b = find_builtin(d->rhs);
+        const void* lone = b ? b->lookup(d->dtype, d->alg, SAVE_END, 0, 1, 1) : nullptr;
+        if (lone) pl->k.aot = lone;
+      }
       // packed output beyond resident: rank the saving pass by the counting pass
       pl->pk_ranked = pl->packed && pl->k.lanes == 1 && !io->order && !io->visits && n > 1 &&
                       n < (1ll << 32) &&
