@@ -25,19 +25,23 @@ const void* adaptive_ptr() {
   return reinterpret_cast<const void*>(&sdeh_adaptive_kernel<T, R, ALG, SAVE, KAHAN, WAVES>);
 }
 
+// waves = 1: the binary64 kernels of small states for ensembles of a wave or two per SIMD,
+// endpoint and (ATsit5, AVern7) saveat output.
+template <class T, int ALG, int SAVE>
+const void* lone_variant() {
+#if !defined(SDEH_LIMITED) && !defined(SDEH_WAVE_ONLY)
+  if constexpr (sizeof(T) == 8 && R::G == 1 && R::N <= 4 &&
+                (SAVE == sdeh::SAVE_END || ALG != sdeh::ALG_AVERN9))
+    return adaptive_ptr<T, ALG, SAVE, false, 1>();
+#endif
+  return nullptr;
+}
+
 // Register-cap variants (SDEH_WAVE_VARIANTS, built for the Lorenz right-hand side):
 // the adaptive endpoint kernels of ATsit5 and AVern7 at 4, 6 and 8 waves per SIMD,
 // for the autotuner; waves = 0 is the default kernel.
-
-// waves = 1: the binary64 kernels of small states for ensembles of a wave or two per SIMD.
-
 template <class T, int ALG, bool KAHAN>
 const void* waves_variant(int waves) {
-#if !defined(SDEH_LIMITED) && !defined(SDEH_WAVE_ONLY)
-  if constexpr (sizeof(T) == 8 && !KAHAN && R::G == 1 && R::N <= 4) {
-    if (waves == 1) return adaptive_ptr<T, ALG, sdeh::SAVE_END, KAHAN, 1>();
-  }
-#endif
 #if defined(SDEH_WAVE_VARIANTS)
   if constexpr (ALG == sdeh::ALG_ATSIT5 || ALG == sdeh::ALG_AVERN7) {
     switch (waves) {
@@ -122,6 +126,12 @@ const void* by_save(int save, int kahan, int waves, int tpl) {
         return nullptr;
       }
       return multi_variant<T, ALG, false>(tpl);
+    }
+    if (waves == 1) {
+      if (kahan) return nullptr;
+      if (save == sdeh::SAVE_END) return lone_variant<T, ALG, sdeh::SAVE_END>();
+      if (save == sdeh::SAVE_AT) return lone_variant<T, ALG, sdeh::SAVE_AT>();
+      return nullptr;
     }
     if (waves) {
       if (save != sdeh::SAVE_END) return nullptr;

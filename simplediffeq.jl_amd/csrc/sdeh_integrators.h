@@ -2665,7 +2665,8 @@ struct WavesHint {
 // every coefficient and constant of an attempt stays in registers.
 template <class T, class R, int ALG, int SAVE, bool KAHAN, int WAVES = 0>
 __global__ void __launch_bounds__(256)
-    __attribute__((amdgpu_waves_per_eu(WAVES > 0 ? WAVES
+    __attribute__((amdgpu_waves_per_eu(WAVES == 1  ? (ALG == sdeh::ALG_AVERN9 ? 1 : 2)
+                                       : WAVES > 0 ? WAVES
                                                  : sdeh::WavesHint<T, R, ALG, SAVE>::value)))
     sdeh_adaptive_kernel(sdeh_kargs a) {
   sdeh::adaptive_body<T, R, ALG, SAVE, KAHAN, WAVES == 1>(a);

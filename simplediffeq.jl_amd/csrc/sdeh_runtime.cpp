@@ -851,12 +851,16 @@ int plan_solve(sdeh_ctx* c, const sdeh_solve_desc* d, const sdeh_io* io, Plan* p
       //     65,536    95 | 86     204 | 165     412 | 370
       //    131,072   127 | 122    274 | 250     561 | 782
       //    262,144   205 | 242    467 | 474     951 | 1,252
+      // with 11 saved points
+      //      1,024   122 | 110    366 | 345     762 | 836 (AVern9: not built)
+      //    131,072   166 | 157    489 | 473
       const int64_t simds = 4 * (int64_t)c->cus;
-      if (sh.schedule == SDEH_SCHED_ONE_LAUNCH && pl->save == SAVE_END && !pl->packed &&
+      if (sh.schedule == SDEH_SCHED_ONE_LAUNCH &&
+          (pl->save == SAVE_END || pl->save == SAVE_AT) && !pl->packed &&
           d->dtype == SDEH_F64 && adaptive && pl->k.lanes == 1 && !w && tp <= 1 &&
           d->n_traj <= simds * 64 * (d->alg == SDEH_ALG_AVERN9 ? 1 : 2)) {
         const Builtin* b = find_builtin(d->rhs);
-        const void* lone = b ? b->lookup(d->dtype, d->alg, SAVE_END, 0, 1, 1) : nullptr;
+        const void* lone = b ? b->lookup(d->dtype, d->alg, pl->save, 0, 1, 1) : nullptr;
         if (lone) pl->k.aot = lone;
       }
       // packed output beyond resident: rank the saving pass by the counting pass

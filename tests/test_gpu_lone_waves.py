@@ -1,4 +1,4 @@
-"""Binary64 endpoint solves of a wave or two per SIMD run a kernel of their own: around its
+"""Binary64 endpoint and saveat solves of a wave or two per SIMD run a kernel of their own: around its
 sizes' ends, with spans of every length and trajectories that end at once, for every adaptive
 solver and small built-in state, the persistent schedule's results bit for bit."""
 import numpy as np
@@ -13,10 +13,11 @@ RHS = {1: (_abi.RHS_AFFINE1, 2), 2: (_abi.RHS_LINEAR2, 4), 3: (_abi.RHS_LORENZ, 
 SIMD = 4 * 256 * 64  # trajectories of one wave per SIMD
 
 
+@pytest.mark.parametrize("points", [0, 5])
 @pytest.mark.parametrize("alg", [_abi.ALG_ATSIT5, _abi.ALG_AVERN7, _abi.ALG_AVERN9])
 @pytest.mark.parametrize("n_state,n", [(3, 1), (3, 63), (3, 65), (1, 1000), (2, 1000), (3, SIMD),
                                        (3, SIMD + 1), (3, 2 * SIMD), (3, 2 * SIMD + 1)])
-def test_small_ensembles_have_the_same_bits(ctx, alg, n_state, n):
+def test_small_ensembles_have_the_same_bits(ctx, alg, n_state, n, points):
     rhs, n_param = RHS[n_state]
     rng = np.random.default_rng(n)
     u0 = rng.uniform(-1.0, 1.0, (n_state, n))
@@ -30,9 +31,10 @@ def test_small_ensembles_have_the_same_bits(ctx, alg, n_state, n):
     out = []
     for sched in (_abi.SCHED_PERSISTENT, _abi.SCHED_AUTO):
         d = runtime.make_desc(alg, rhs=rhs, n_traj=n, dt=0.1, abstol=1e-9, reltol=1e-7,
-                              schedule=sched, maxiters=60)
+                              schedule=sched, maxiters=60,
+                              saveat=np.linspace(0.0, 3.0, points) if points else None)
         b = runtime.EnsembleBuffers(d, n_state, u0, p, tspan=ts, dt0=dt0)
         ctx.solve(d, b, allow=(_abi.E_DTMIN,))
         out.append(b)
-    for f in ("u_end", "t_end", "retcode", "naccept", "nreject"):
+    for f in ("u_end", "t_end", "retcode", "naccept", "nreject") + (("u_saveat",) if points else ()):
         assert bits_equal(out[0].numpy(f), out[1].numpy(f)), f
