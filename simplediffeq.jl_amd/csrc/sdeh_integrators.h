@@ -175,7 +175,7 @@ __device__ __forceinline__ X in_vgpr(X x) {
 // Each attempt gathers three rows at 64 unrelated indices, one after the other.  From
 // constant memory those gathers went through the vector L1, which was busy as long as the
 // arithmetic was.  Lorenz, from constant memory / from LDS: 2^20 ATsit5 1,042 / 980 us,
-// 2^22 ATsit5 over spans 4,294 / 4,003 us, 2^20 uneven AVern7 9,997 / 9,428 us, 1,024 ATsit5
+// 2^22 ATsit5 over spans 4,294 / 4,003 us, 2^21 uneven AVern7 9,997 / 9,428 us, 1,024 ATsit5
 // 37.7 / 35.0 us.
 struct LdsTab {
   const double* t;
@@ -524,7 +524,7 @@ __device__ __forceinline__ CtrlOut<T> controller(T s, T dt, T qold_pow, const Ct
 // ensemble's first pass ran at the issue rate), so this path was cut to what it needs:
 // no selects for EEst = 0 or special values, 32-bit range checks and bit handling, ldexp,
 // and one-instruction minima and maxima.  Lorenz, before / after: 2^20 ATsit5 988 / 932 us,
-// 2^22 ATsit5 over spans 4,170 / 4,000 us, 2^20 uneven AVern7 9,430 / 9,200 us, 1,024 ATsit5
+// 2^22 ATsit5 over spans 4,170 / 4,000 us, 2^21 uneven AVern7 9,430 / 9,200 us, 1,024 ATsit5
 // 38.6 / 37.4 us.
 __device__ __forceinline__ unsigned hi_word(double x) {
   return (unsigned)(sdeh_math::bits_of(x) >> 32);
@@ -1471,7 +1471,9 @@ __device__ __forceinline__ X in_vgpr_if(X x) {
 // trajectory passes only once: the pointers of inputs and outputs then hold no scalar
 // registers in the loop between: the one-lane binary64 kernels keep 12 spilled ones (34
 // before) and have room to hold their stages' coefficients.  Lorenz: 1,024 ATsit5 37.4 /
-// 34.7 us, 2^20 uneven AVern7 9,440 / 9,190 us, the large ATsit5 ensembles as before.
+// 34.7 us, 2^21 uneven AVern7 9,440 / 9,190 us, the large ATsit5 ensembles as before.  The
+// matrix-core AVern9 kernel with saveat spills 24 bytes instead of 76 (2^17 GLV-16
+// trajectories, 256 points 7,130 / 7,065 us; holding coefficients there took 7,230).
 // (Every kernel takes sdeh_kargs first and by value.)
 __device__ __forceinline__ const sdeh_kargs& cold_args(const sdeh_kargs&) {
   auto k = __builtin_amdgcn_kernarg_segment_ptr();
@@ -1702,38 +1704,40 @@ __device__ __forceinline__ void adaptive_body_wave(const sdeh_kargs& a) {
         const int kmin = a.refill_min < SLOTS ? a.refill_min : SLOTS;
         if (__popcll(__ballot(want)) < kmin) want = false;
       }
-      int64_t slot = wave_claim(a, want, qbase, qlim, drained);
+      int64_t slot = wave_claim(cold_args(a), want, qbase, qlim, drained);
       slot = (int64_t)__shfl((long long)slot, lane & (SLOTS - 1));  // from the slot's lead lane
       if (slot >= 0) {
-        traj = slot_traj(a, slot);
+        traj = slot_traj(cold_args(a), slot);
         active = fresh = traj >= 0;
       }
     }
     if (__ballot(active) == 0ull) break;
 
     if (fresh) {  // start trajectory `traj` (gpuatsit5.jl:221-241)
-      if (lead) note_visit(a, traj);
-      load_state<T, R>(uprev, a.u0, n, traj);
+      const sdeh_kargs& ka = cold_args(a);
+      const int64_t n = ka.n;
+      if (lead) note_visit(ka, traj);
+      load_state<T, R>(uprev, ka.u0, n, traj);
 #pragma unroll
       for (int c = 0; c < N; ++c) comp[c] = T(0);
-      R::template load_lane<T>(pl, (const T*)a.p, ps, n, traj, lane_comp<R>());
-      t = a.tspan ? a.tspan[traj] : a.t0;
-      tf = a.tspan ? a.tspan[n + traj] : a.tf;
-      dt = (T)(a.dt0 ? a.dt0[traj] : a.dt);
+      R::template load_lane<T>(pl, (const T*)ka.p, ps, n, traj, lane_comp<R>());
+      t = ka.tspan ? ka.tspan[traj] : ka.t0;
+      tf = ka.tspan ? ka.tspan[n + traj] : ka.tf;
+      dt = (T)(ka.dt0 ? ka.dt0[traj] : ka.dt);
       qold_pow = qoldinit_pow;
       nacc = nrej = 0;
       attempts = 0;
       cur = 0;
       if constexpr (SAVE == SAVE_AT) {
-        if (a.n_saveat > 0 && t == a.saveat[0]) {
-          store_save<T, R>(a, a.u_saveat, 0, a.n_saveat, traj, uprev);
+        if (ka.n_saveat > 0 && t == ka.saveat[0]) {
+          store_save<T, R>(ka, ka.u_saveat, 0, ka.n_saveat, traj, uprev);
           cur = 1;
         }
-        ts_next = saves_at.at(a, cur);
+        ts_next = saves_at.at(ka, cur);
       }
       if constexpr (SAVE == SAVE_STEPS) {
-        sink_start<R>(a, sk, traj);
-        save_step<T, R>(a, sk, traj, t, uprev);
+        sink_start<R>(ka, sk, traj);
+        save_step<T, R>(ka, sk, traj, t, uprev);
       }
     }
     if constexpr (ALG == ALG_ATSIT5) {  // FSAL seed, :241
@@ -1898,16 +1902,18 @@ __device__ __forceinline__ void adaptive_body_wave(const sdeh_kargs& a) {
     }
 
     if (ret >= 0) {  // trajectory ends: write outputs (gpuatsit5.jl:322-329)
+      const sdeh_kargs& ka = cold_args(a);
+      const int64_t n = ka.n;
       if (SAVE == SAVE_STEPS && ret == RET_DEFAULT && sk.kept < sk.n) ret = RET_SAVE_OVERFLOW;
-      store_state<T, R>(a.u_end, 0, n, traj, uprev);
-      if constexpr (SAVE == SAVE_AT) save_unreached<T, R>(a, cur, traj);
-      if constexpr (SAVE == SAVE_STEPS) flush_steps<T, R>(a, sk);
+      store_state<T, R>(ka.u_end, 0, n, traj, uprev);
+      if constexpr (SAVE == SAVE_AT) save_unreached<T, R>(ka, cur, traj);
+      if constexpr (SAVE == SAVE_STEPS) flush_steps<T, R>(ka, sk);
       if (lead) {
-        a.t_end[traj] = t;
-        a.retcode[traj] = ret;
-        if (a.naccept) a.naccept[traj] = nacc;
-        if (a.nreject) a.nreject[traj] = nrej;
-        if constexpr (SAVE == SAVE_STEPS) finish_steps(a, sk, traj);
+        ka.t_end[traj] = t;
+        ka.retcode[traj] = ret;
+        if (ka.naccept) ka.naccept[traj] = nacc;
+        if (ka.nreject) ka.nreject[traj] = nrej;
+        if constexpr (SAVE == SAVE_STEPS) finish_steps(ka, sk, traj);
       }
       active = false;
     }
@@ -2030,9 +2036,8 @@ __device__ __forceinline__ void adaptive_body(const sdeh_kargs& a) {
   int64_t qbase = 0, qlim = 0;
   bool drained = !a.persistent;
   // the persistent queue's cache of hand-out order entries (wave_claim_win): in the
-  // binary32 one-lane endpoint kernels, whose occupancy is set by scalar registers, so
-  // the vector registers it takes cost no wave (the binary64 and save modes' kernels
-  // would lose one)
+  // binary32 one-lane endpoint kernels, where the vector registers it takes cost no wave
+  // (the binary64 and save modes' kernels would lose one)
   constexpr bool ORDER_WIN = sizeof(T) == 4 && R::G == 1 && SAVE == SAVE_END;
   int64_t qwin = -128, qword = -1;
   const bool lead = lane_comp<R>() == 0;  // writes the per-trajectory scalars
