@@ -26,7 +26,7 @@ const void* adaptive_ptr() {
 }
 
 // waves = 1: the binary64 kernels of small states for ensembles of a wave or two per SIMD,
-// endpoint and (ATsit5, AVern7) saveat output.
+// endpoint and (ATsit5, AVern7) saved output.
 template <class T, int ALG, int SAVE>
 const void* lone_variant() {
 #if !defined(SDEH_LIMITED) && !defined(SDEH_WAVE_ONLY)
@@ -131,6 +131,7 @@ const void* by_save(int save, int kahan, int waves, int tpl) {
       if (kahan) return nullptr;
       if (save == sdeh::SAVE_END) return lone_variant<T, ALG, sdeh::SAVE_END>();
       if (save == sdeh::SAVE_AT) return lone_variant<T, ALG, sdeh::SAVE_AT>();
+      if (save == sdeh::SAVE_STEPS) return lone_variant<T, ALG, sdeh::SAVE_STEPS>();
       return nullptr;
     }
     if (waves) {

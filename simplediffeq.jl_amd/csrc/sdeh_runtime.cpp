@@ -854,14 +854,18 @@ int plan_solve(sdeh_ctx* c, const sdeh_solve_desc* d, const sdeh_io* io, Plan* p
       // with 11 saved points
       //      1,024   122 | 110    366 | 345     762 | 836 (AVern9: not built)
       //    131,072   166 | 157    489 | 473
+      // every step in packed rows (AVern9's counting pass only)
+      //      1,024   202 | 186    419 | 361     793 | 751
+      //    131,072   290 | 280    605 | 580   1,147 | 1,146
       const int64_t simds = 4 * (int64_t)c->cus;
-      if (sh.schedule == SDEH_SCHED_ONE_LAUNCH &&
-          (pl->save == SAVE_END || pl->save == SAVE_AT) && !pl->packed &&
-          d->dtype == SDEH_F64 && adaptive && pl->k.lanes == 1 && !w && tp <= 1 &&
+      if (sh.schedule == SDEH_SCHED_ONE_LAUNCH && d->dtype == SDEH_F64 && adaptive &&
+          pl->k.lanes == 1 && !w && tp <= 1 &&
           d->n_traj <= simds * 64 * (d->alg == SDEH_ALG_AVERN9 ? 1 : 2)) {
         const Builtin* b = find_builtin(d->rhs);
         const void* lone = b ? b->lookup(d->dtype, d->alg, pl->save, 0, 1, 1) : nullptr;
         if (lone) pl->k.aot = lone;
+        lone = b && pl->packed ? b->lookup(d->dtype, d->alg, SAVE_END, 0, 1, 1) : nullptr;
+        if (lone) pl->k_count.aot = lone;
       }
       // packed output beyond resident: rank the saving pass by the counting pass
       pl->pk_ranked = pl->packed && pl->k.lanes == 1 && !io->order && !io->visits && n > 1 &&
