@@ -2535,7 +2535,12 @@ __device__ __forceinline__ void fixed_body(const sdeh_kargs& a) {
   }
   if constexpr (SAVE == SAVE_STEPS) save_step<T, R>(a, sk, traj, t, u);
   T k7[N];
-  using Held = typename StageCoefs<T, ALG, (sizeof(T) == 8 && R::G == 1 && N <= 4)>::type;
+  // Vern7's endpoint kernel holds all its coefficients, the last 16 in vector registers (100
+  // of them, five waves per SIMD still): 1,024 trajectories 52 / 47 us, 2^20 674 / 668.
+  // (Vern9's 55 more leave two waves: 96 / 93, 2^18 328 / 339.)
+  constexpr bool SMALL = sizeof(T) == 8 && R::G == 1 && N <= 4;
+  using Held =
+      typename StageCoefs<T, ALG, SMALL, SMALL && ALG == ALG_VERN7 && SAVE == SAVE_END>::type;
   const Held co = Held::init();
   if constexpr (ALG == ALG_TSIT5) R::f(k7, u, pl, ps, t);  // gpuatsit5.jl:86
   for (int64_t i = 1; i < a.g_len; ++i) {
