@@ -844,29 +844,6 @@ int plan_solve(sdeh_ctx* c, const sdeh_solve_desc* d, const sdeh_io* io, Plan* p
       sh.waves = w;
       sh.per_lane = tp;
       pl->default_staged = sh.schedule == SDEH_SCHED_STAGED;
-      // The kernel that keeps its constants in registers, for ensembles of a wave or two
-      // per SIMD (AVern9: one, its 302 registers allow no second).  Lorenz, the default
-      // kernel | this one (us; ATsit5, AVern7, AVern9):
-      //      1,024    89 | 81     197 | 162     391 | 354
-      //     65,536    95 | 86     204 | 165     412 | 370
-      //    131,072   127 | 122    274 | 250     561 | 782
-      //    262,144   205 | 242    467 | 474     951 | 1,252
-      // with 11 saved points
-      //      1,024   122 | 110    366 | 345     762 | 836 (AVern9: not built)
-      //    131,072   166 | 157    489 | 473
-      // every step in packed rows (AVern9's counting pass only)
-      //      1,024   202 | 186    419 | 361     793 | 751
-      //    131,072   290 | 280    605 | 580   1,147 | 1,146
-      const int64_t simds = 4 * (int64_t)c->cus;
-      if (sh.schedule == SDEH_SCHED_ONE_LAUNCH && d->dtype == SDEH_F64 && adaptive &&
-          pl->k.lanes == 1 && !w && tp <= 1 &&
-          d->n_traj <= simds * 64 * (d->alg == SDEH_ALG_AVERN9 ? 1 : 2)) {
-        const Builtin* b = find_builtin(d->rhs);
-        const void* lone = b ? b->lookup(d->dtype, d->alg, pl->save, 0, 1, 1) : nullptr;
-        if (lone) pl->k.aot = lone;
-        lone = b && pl->packed ? b->lookup(d->dtype, d->alg, SAVE_END, 0, 1, 1) : nullptr;
-        if (lone) pl->k_count.aot = lone;
-      }
       // packed output beyond resident: rank the saving pass by the counting pass
       pl->pk_ranked = pl->packed && pl->k.lanes == 1 && !io->order && !io->visits && n > 1 &&
                       n < (1ll << 32) &&
@@ -896,6 +873,29 @@ int plan_solve(sdeh_ctx* c, const sdeh_solve_desc* d, const sdeh_io* io, Plan* p
   } else {
     sh.schedule = SDEH_SCHED_ONE_LAUNCH;
     if (d->block) sh.block = d->block;
+  }
+  // The kernel that keeps its constants in registers, for ensembles of a wave or two
+  // per SIMD (AVern9: one, its 302 registers allow no second).  Lorenz, the default
+  // kernel | this one (us; ATsit5, AVern7, AVern9):
+  //      1,024    89 | 81     197 | 162     391 | 354
+  //     65,536    95 | 86     204 | 165     412 | 370
+  //    131,072   127 | 122    274 | 250     561 | 782
+  //    262,144   205 | 242    467 | 474     951 | 1,252
+  // with 11 saved points
+  //      1,024   122 | 110    366 | 345     762 | 836 (AVern9: not built)
+  //    131,072   166 | 157    489 | 473
+  // every step in packed rows (AVern9's counting pass only)
+  //      1,024   202 | 186    419 | 361     793 | 751
+  //    131,072   290 | 280    605 | 580   1,147 | 1,146
+  const int64_t simds = 4 * (int64_t)c->cus;
+  if (sh.schedule == SDEH_SCHED_ONE_LAUNCH && d->dtype == SDEH_F64 && adaptive &&
+      pl->k.lanes == 1 && !sh.waves && sh.per_lane <= 1 &&
+      d->n_traj <= simds * 64 * (d->alg == SDEH_ALG_AVERN9 ? 1 : 2)) {
+    const Builtin* b = find_builtin(d->rhs);
+    const void* lone = b ? b->lookup(d->dtype, d->alg, pl->save, 0, 1, 1) : nullptr;
+    if (lone) pl->k.aot = lone;
+    lone = b && pl->packed ? b->lookup(d->dtype, d->alg, SAVE_END, 0, 1, 1) : nullptr;
+    if (lone) pl->k_count.aot = lone;
   }
   if (sh.schedule == SDEH_SCHED_ONE_LAUNCH) {
     const int64_t g = one_launch_groups(d->n_traj, pl->k, sh.block);
