@@ -1048,8 +1048,8 @@ int run_plan(sdeh_ctx* c, Plan& pl, hipStream_t s, unsigned long long* queue, bo
                                        pl.pk_cap, pl.pk_off, a.n_steps, c->counters + 6, s));
       // The counts rank the saving pass exactly: waves of equal lengths, longest first.
       // (Lorenz ATsit5, 2^20 trajectories, 67 M rows: 3,120 us with both passes persistent;
-      // 2,820 with the staged endpoint pass and the ranked saving pass; 2,620 with the
-      // latter writing by runs.)
+      // 2,820 with the staged endpoint pass and the ranked saving pass; 2,220 with the
+      // latter writing whole sectors and the controller's tables in LDS.)
       if (pl.pk_ranked) {
         HIPCHK(c, sdeh_util_count_order(a.naccept, a.nreject, a.n, pl.st_hist, pl.st_order, s));
         a.order = pl.st_order;
