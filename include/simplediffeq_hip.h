@@ -295,7 +295,18 @@ int sdeh_compile_rhs(sdeh_ctx* ctx, const char* src, const char* fn_name, int32_
 
 /* Integrate an ensemble.  `stream` is a hipStream_t (NULL = the context's stream).
  * With SDEH_MEM_HOST the call returns after results are back in host memory;
- * with SDEH_MEM_DEVICE it returns once the work is queued, unless `sync` != 0. */
+ * with SDEH_MEM_DEVICE it returns once the work is queued, unless `sync` != 0.
+ *
+ * Scratch: a context keeps one device allocation, grown (by a quarter more than asked)
+ * to its calls' largest need and given back by sdeh_destroy.  Of the library's own
+ * choices, a staged or packed solve beyond what fits the GPU at once takes a parked
+ * record per trajectory there (at most 1 GiB), and point-major saveat output of 300 MiB
+ * to 2 GiB with many points as much as that output; where that memory cannot be had,
+ * the solve runs without it.  So does a solve whose `stream` the caller is capturing
+ * into a graph (sync = 0): with device buffers, endpoint output, naccept and nreject
+ * given, no order, and no tspan (or span_order = 1), it uses no such scratch and its
+ * replays stay valid after later calls on the context, which they must not overlap
+ * (they share its queue counter). */
 int sdeh_solve(sdeh_ctx* ctx, const sdeh_solve_desc* d, const sdeh_io* io, int32_t memory,
                void* stream, int32_t sync);
 

@@ -1257,18 +1257,33 @@ int solve_impl(sdeh_ctx* c, const sdeh_solve_desc* d, const sdeh_io* io, int32_t
               round256(sz.st_hist);
     return need;
   };
-  r = ensure_arena(c, scratch_need());
-  if (r == SDEH_E_NOMEM && (pl.default_staged || pl.pk_ranked)) {
-    // no room for the parked records: the persistent schedule needs none
+  // the persistent schedule instead of the parked records
+  auto drop_records = [&]() {
     if (pl.pk_ranked) {
       pl.shape.block = d->block ? d->block : 256;
       pl.shape.grid = c->cus * blocks_per_cu(c, pl.k, pl.shape.block);
       a.persistent = 1;
     }
-    pl.staged = pl.pk_ranked = false;
+    pl.staged = pl.default_staged = pl.pk_ranked = false;
     pl.shape.schedule = SDEH_SCHED_PERSISTENT;
-    c->err.clear();
     sz = sizes_of(d, io, pl);
+  };
+  // A caller's capture of `s` records the launches for later replays.  The records and rows
+  // live in the arena, which cannot be allocated during a capture and which a later, larger
+  // solve frees while the graph still writes to it, so a captured solve does without them.
+  if (!host && (pl.default_staged || pl.pk_ranked || pl.by_rows)) {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    HIPCHK(c, hipStreamIsCapturing(s, &cs));
+    if (cs != hipStreamCaptureStatusNone) {
+      if (pl.default_staged || pl.pk_ranked) drop_records();
+      pl.by_rows = false;
+    }
+  }
+  r = ensure_arena(c, scratch_need());
+  if (r == SDEH_E_NOMEM && (pl.default_staged || pl.pk_ranked)) {
+    // no room for the parked records
+    drop_records();
+    c->err.clear();
     r = ensure_arena(c, scratch_need());
   }
   if (r == SDEH_E_NOMEM && pl.by_rows) {  // no room for the rows: stored where they belong
