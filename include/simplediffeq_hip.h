@@ -123,8 +123,10 @@ typedef enum sdeh_save_layout {
 /* Scheduling of trajectories onto lanes. */
 typedef enum sdeh_schedule {
   SDEH_SCHED_AUTO = 0,       /* the tuned schedule (sdeh_autotune); without one, by size:
-                                one launch while the ensemble is a few times what fits
-                                the GPU at once, beyond that staged where it applies and
+                                one launch while the ensemble fits the GPU at once (three
+                                times that for endpoint output handed out longest span
+                                first, twice in binary32 with several lanes per
+                                trajectory), beyond that staged where it applies and
                                 persistent elsewhere (persistent at any size when grid,
                                 chunk or refill is set) */
   SDEH_SCHED_ONE_LAUNCH = 1, /* one lane per trajectory, grid covers the ensemble */

@@ -604,41 +604,44 @@ size_t staged_stride(const sdeh_solve_desc* d, const Plan& pl) {
 }
 
 // The launch shape of an adaptive solve that names none and has not been tuned, for `n`
-// trajectories of which `sorted` says whether they are handed out longest first (the
-// span order, or an order that sdeh_plan_order made) and `can_stage` whether the staged
-// schedule is open to the solve.  `resident` = lanes that fit the GPU at once.
-//   one launch   up to 3 x resident lanes (4 x in the layouts with several lanes per
-//                trajectory, and for binary32 in a planned order at any size, binary64
-//                up to 8 x).  While every wave is resident the queue only costs: its
-//                atomics, its reset, and waves that take 64 slots each while others
-//                get none.  Beyond that the hardware's block dispatch serves as the
-//                queue until the waves' unequal lengths cost more than lane refills.
+// trajectories of which `sorted` says whether they are handed out longest span first and
+// `can_stage` whether the staged schedule is open to the solve.  `resident` = lanes that fit
+// the GPU at once.
+//   one launch   up to 1 x resident lanes (3 x for endpoint output in the span order, 2 x
+//                in binary32 with several lanes per trajectory).  While every wave is
+//                resident the queue only costs: its atomics, its reset, and waves that take
+//                64 slots each while others get none.
 //   staged       one tspan, endpoint output, beyond resident: its first pass ranks the
 //                trajectories (scratch bounded by kStagedBytes; no visit counters, which
 //                would count a resumed trajectory twice).
 //   persistent   the rest.
-// Measured (us, persistent | one launch | staged; Lorenz, tolerances 1e-7/1e-5 for
-// ATsit5, 1e-8/1e-6 AVern7, 1e-9 AVern9):
-//   one tspan  ATsit5 binary64   n = 1,024     617 |   487 |   630
-//              (resident 327,680)  65,536      834 |   543 |   672
-//                                 262,144    1,406 | 1,066 | 1,025
-//                                 524,288    1,896 | 1,860 | 1,505
-//                               2,097,152    5,428 | 6,542 | 4,810
-//   own spans  ATsit5 binary64    524,288      838 |   723 |   859
-//                               1,048,576    1,265 | 1,266 | 1,248
-//                               4,194,304    4,381 | 5,068 | 4,332
-//              AVern9 binary64    700,001    1,732 | 1,656 | 1,775
-//              AVern7 binary64  4,194,304    4,393 | 5,152 | 4,600
-//              ATsit5 binary32  1,048,576      585 |   509 |   651
-//   planned    ATsit5 binary64  1,048,576    1,256 | 1,055
-//                               4,194,304    4,192 | 4,289
-//              binary32 compensated, same    1,759 | 1,646
-//   saveat 31  AVern7 binary64    524,288    3,437 | 3,455
-//              (resident 196,608) 1,048,576  5,534 | 6,553
-//   GLV-16, 256 points, AVern9 on the matrix cores (resident 32,768 trajectories)
-//                                   1,024    5,570 | 1,506
-//                                  65,536    8,293 | 4,400
-//                                 131,072    8,173 | 7,943
+// Beyond resident one launch gains while a wave's trajectories are about as long as each
+// other and loses once they are not, which only the solve itself shows, so the line is where
+// an ensemble of unlike lengths is not slower than on the queue by more than one of like
+// lengths gains.  Queue | one launch (us):
+//   resident x                          1             2             3 or 4
+//   Lorenz saveat 31 points AVern7, one tspan (196,608 trajectories resident)
+//     rho log-uniform in 0.5 .. 200     3,523 | 3,471   4,892 | 6,161   5,888 | 8,835
+//   Lorenz ATsit5 binary64, own spans, in the span order (327,680)
+//     spans 0.5 .. 10                     592 |   503     815 |   757   1,070 | 1,063
+//     the same, rho in 0.5 .. 200                         931 |   851   1,063 | 1,167
+//     spans 9 .. 10, rho in 0.5 .. 200  (1.3 x: 1,547 | 1,702)          2,231 | 3,355
+//   Lorenz ATsit5 over spans, in the order of a caller's keys, binary32 (524,288)
+//     keys the true lengths               398 |   242     494 |   320     849 |   668
+//     keys at random                      763 |   566     961 | 1,012   1,288 | 1,836
+//   and binary64: 2^20 (3.2 x) 956 | 806 and 1,637 | 2,448; binary32 2^22 (8 x) 1,614 |
+//   1,373 and 2,038 | 3,484.  A key that predicts nothing costs more than a true one gains,
+//   and the library cannot tell them apart, so a planned order counts as any other.
+//   GLV-16, 256 points, AVern9 binary64 on the matrix cores (32,768)
+//     like growth rates                 2,224 | 2,157   4,362 | 3,987   7,247 | 6,492
+//     rates over two decades            6,406 | 6,252   8,668 | 11,213 10,967 | 16,735
+//   the same, ATsit5 binary32 (65,536)
+//     like growth rates                   547 |   480     911 |   780   1,740 | 1,513
+//     rates over two decades            2,146 | 2,039   2,358 | 2,735   4,104 | 5,780
+// Staged, one tspan ATsit5 binary64 (persistent | one launch | staged):
+//     262,144    1,406 | 1,066 | 1,025
+//     524,288    1,896 | 1,860 | 1,505
+//   2,097,152    5,428 | 6,542 | 4,810
 // One-lane kernels launch blocks of 64 (small ensembles spread over more CUs: 487
 // against 538 us at n = 1,024; the same beyond 65,536), the others blocks of 256 (their
 // LDS exchange buffers are sized for four waves: 12.9 against 7.9 ms in blocks of 64).
@@ -646,14 +649,14 @@ size_t staged_stride(const sdeh_solve_desc* d, const Plan& pl) {
 // (GLV-16 ATsit5, 500,000: 2,972 against 3,491 us claiming 64).
 constexpr size_t kStagedBytes = size_t(1) << 30;
 
-Shape default_shape(sdeh_ctx* c, const Plan& pl, int dtype, int64_t n, bool sorted, bool planned,
+Shape default_shape(sdeh_ctx* c, const Plan& pl, int dtype, int64_t n, bool sorted,
                     bool can_stage) {
   Shape sh;
   const int lanes = pl.k.lanes > 0 ? pl.k.lanes : 1;
   const int64_t work = (n + pl.k.tpl - 1) / pl.k.tpl * lanes;
   const int64_t resident = (int64_t)c->cus * blocks_per_cu(c, pl.k, 256) * 256;
-  int64_t times = lanes > 1 ? 4 : 3;
-  if (planned) times = dtype == SDEH_F32 ? INT64_MAX / resident : 8;
+  const int64_t times = lanes > 1 ? (dtype == SDEH_F32 ? 2 : 1)
+                                  : (sorted && pl.save == SAVE_END ? 3 : 1);
   sh.chunk = 64 / lanes;
   if (can_stage && !sorted && work > resident) {
     sh.schedule = SDEH_SCHED_STAGED;
@@ -833,14 +836,11 @@ int plan_solve(sdeh_ctx* c, const sdeh_solve_desc* d, const sdeh_io* io, Plan* p
       const bool piped =
           path == Path::kHost && d->n_traj >= kPipeMin && !io->order && !pl->packed;
       const int64_t n = piped ? (d->n_traj + kPipeChunks - 1) / kPipeChunks : d->n_traj;
-      const bool planned = path == Path::kDevice && io->order && io->order == c->planned_order &&
-                           d->n_traj == c->planned_n;
       const bool can_stage = (path == Path::kDevice || (path == Path::kHost && !piped)) &&
                              stageable(d, io, *pl) && !io->visits &&
                              (size_t)n * (staged_stride(d, *pl) + 16) <= kStagedBytes;
       const int32_t w = sh.waves, tp = sh.per_lane;
-      sh = default_shape(c, *pl, d->dtype, n, planned || (pl->span && path != Path::kStatic),
-                         planned, can_stage);
+      sh = default_shape(c, *pl, d->dtype, n, pl->span && path != Path::kStatic, can_stage);
       sh.waves = w;
       sh.per_lane = tp;
       pl->default_staged = sh.schedule == SDEH_SCHED_STAGED;

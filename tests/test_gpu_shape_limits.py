@@ -1,0 +1,70 @@
+"""Where the default launch shape leaves one launch for the queue: as soon as the ensemble does
+not fit the GPU at once, unless the library orders it by its spans (endpoint output) or it runs
+several binary32 lanes per trajectory.  On ensembles whose trajectories differ in length one
+launch is slower there: saved output, unsorted spans, the allocation-free solve, a planned
+order whose keys need not predict anything, the matrix-core layout.  On both sides of each line
+the results are the explicit schedule's, bit for bit."""
+import numpy as np
+import pytest
+
+from helpers import bits_equal
+from simplediffeq_hip import _abi, inputs, runtime
+
+pytestmark = pytest.mark.gpu
+
+FIELDS = ("u_end", "t_end", "retcode", "naccept", "nreject")
+
+
+def _inputs(rhs, n):
+    if rhs == _abi.RHS_GLV16:
+        u0, r, A = inputs.glv16(64, seed=1)
+        return np.resize(u0, (16, n)), np.resize(r, (16, n)), A
+    return inputs.lorenz_wide(n, seed=5) + (None,)
+
+
+@pytest.mark.parametrize("add", [0, 1])
+@pytest.mark.parametrize("name,rhs,alg,dtype,points,spans,times", [
+    ("saveat", _abi.RHS_LORENZ, _abi.ALG_AVERN7, _abi.F64, 3, False, 1),
+    ("saveat", _abi.RHS_LORENZ, _abi.ALG_ATSIT5, _abi.F32, 3, True, 1),
+    ("static", _abi.RHS_LORENZ, _abi.ALG_ATSIT5, _abi.F64, 0, False, 1),
+    ("static", _abi.RHS_LORENZ, _abi.ALG_AVERN7, _abi.F64, 0, True, 1),
+    ("planned", _abi.RHS_LORENZ, _abi.ALG_ATSIT5, _abi.F64, 0, True, 1),
+    ("planned", _abi.RHS_LORENZ, _abi.ALG_ATSIT5, _abi.F32, 0, True, 1),
+    ("lanes", _abi.RHS_GLV16, _abi.ALG_AVERN9, _abi.F64, 3, False, 1),
+    ("lanes", _abi.RHS_GLV16, _abi.ALG_ATSIT5, _abi.F32, 0, False, 2)])
+def test_one_launch_ends_where_unlike_lengths_lose(name, rhs, alg, dtype, points, spans, times,
+                                                   add):
+    import torch
+    c = runtime.Context(0)
+    kw = dict(rhs=rhs, dtype=dtype, tspan=(0.0, 0.3), dt=0.1, abstol=1e-6, reltol=1e-5,
+              saveat=np.linspace(0.0, 0.3, points) if points else None)
+
+    def solve(n, sched, order=None, **more):
+        u0, p, ps = _inputs(rhs, n)
+        ts = None
+        if spans:
+            ts = np.zeros((2, n))
+            ts[1] = np.linspace(0.0, 0.3, n)
+        d = runtime.make_desc(alg, n_traj=n, schedule=sched, **kw, **more)
+        b = runtime.EnsembleBuffers(d, u0.shape[0], u0, p, ps, ts, order=order, backend="torch",
+                                    device="cuda:0")
+        torch.cuda.synchronize()
+        if order is not None:
+            key = torch.as_tensor(np.random.default_rng(3).normal(-3.0, 1.0, n).astype(np.float32),
+                                  device="cuda:0")
+            c.plan_order(key.data_ptr(), n, b.order.data_ptr())
+        (c.solve_static if name == "static" else c.solve)(d, b)
+        return b, c.stats()
+
+    # the persistent grid is the lanes that fit the GPU at once
+    lanes = 4 if rhs == _abi.RHS_GLV16 else 1
+    _, st = solve(100, _abi.SCHED_PERSISTENT, lanes=lanes, block=256)
+    n = times * st["grid"] * 256 // lanes + add
+    order = torch.zeros(n, dtype=torch.int64, device="cuda:0") if name == "planned" else None
+    got, st = solve(n, _abi.SCHED_AUTO, order)
+    assert st["lanes"] == lanes
+    assert st["schedule"] == (_abi.SCHED_PERSISTENT if add else _abi.SCHED_ONE_LAUNCH)
+    ref, _ = solve(n, _abi.SCHED_ONE_LAUNCH if add else _abi.SCHED_PERSISTENT, lanes=lanes)
+    for f in FIELDS + (("u_saveat",) if points else ()):
+        assert bits_equal(got.numpy(f), ref.numpy(f)), f
+    c.close()
