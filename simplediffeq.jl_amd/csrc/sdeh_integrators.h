@@ -1614,6 +1614,22 @@ struct SaveTimes {
     }
     return r;
   }
+  // The same where every lane is at the same point (the fixed-step solvers): the later times
+  // are scalar loads, which wait for no store.  at()'s vector loads there wait for the stores
+  // of the point before: Tsit5, 1,024 trajectories, 4,000 points 2,690 / 1,660 us (1,930 with
+  // every time a vector load one point ahead), 700 points 403 / 307 (380).
+  __device__ __forceinline__ double at_uniform(const sdeh_kargs& a, int64_t i) const {
+    typedef const double __attribute__((address_space(4))) scalar_double;
+    double r;
+    if (i < SAVE_LDS) {
+      r = lds[i];
+    } else {
+      const int32_t k = __builtin_amdgcn_readfirstlane((int32_t)i);
+      r = k < a.n_saveat ? ((scalar_double*)(uint64_t)a.saveat)[k] : 0.0;
+      asm volatile("" ::"v"(r));
+    }
+    return r;
+  }
 };
 template <>
 struct SaveTimes<false> {
@@ -2539,7 +2555,7 @@ __device__ __forceinline__ void fixed_body(const sdeh_kargs& a) {
       store_save<T, R>(a, a.u_saveat, 0, a.n_saveat, traj, u);
       cur = 1;
     }
-    ts_next = saves_at.at(a, cur);
+    ts_next = saves_at.at_uniform(a, cur);
   }
   if constexpr (SAVE == SAVE_STEPS) save_step<T, R>(a, sk, traj, t, u);
   T k7[N];
@@ -2588,7 +2604,7 @@ __device__ __forceinline__ void fixed_body(const sdeh_kargs& a) {
       t += (double)dt;
       if constexpr (SAVE == SAVE_AT) {  // :116-127
         while (cur < a.n_saveat && ts_next <= t) {
-          const double ts_after = saves_at.at(a, cur + 1);
+          const double ts_after = saves_at.at_uniform(a, cur + 1);
           const T th = (T)((ts_next - (t - (double)dt)) / (double)dt);
           T o[N];
           tsit5_dense(o, uprev, dt, th, k1, k2, k3, k4, k5, k6, k7);
@@ -2607,7 +2623,7 @@ __device__ __forceinline__ void fixed_body(const sdeh_kargs& a) {
           T x[6][N];
           vern7_extra<T, R>(uprev, K, x, pl, ps, a.quirks ? t : told, dt);  // quirk :160
           while (cur < a.n_saveat && ts_next <= t) {
-            const double ts_after = saves_at.at(a, cur + 1);
+            const double ts_after = saves_at.at_uniform(a, cur + 1);
             const T th = (T)((ts_next - (t - (double)dt)) / (double)dt);
             T o[N];
             vern7_dense(o, uprev, dt, th, K, x);
@@ -2628,7 +2644,7 @@ __device__ __forceinline__ void fixed_body(const sdeh_kargs& a) {
           T x[10][N];
           vern9_extra<T, R>(uprev, S, x, pl, ps, a.quirks ? t : told, dt);  // quirk :222
           while (cur < a.n_saveat && ts_next <= t) {
-            const double ts_after = saves_at.at(a, cur + 1);
+            const double ts_after = saves_at.at_uniform(a, cur + 1);
             const T th = (T)((ts_next - (t - (double)dt)) / (double)dt);
             T o[N];
             vern9_dense(o, uprev, dt, th, S, x);
