@@ -126,9 +126,10 @@ typedef enum sdeh_schedule {
                                 one launch while the ensemble fits the GPU at once (three
                                 times that for endpoint output handed out longest span
                                 first, twice in binary32 with several lanes per
-                                trajectory), beyond that staged where it applies and
-                                persistent elsewhere (persistent at any size when grid,
-                                chunk or refill is set) */
+                                trajectory), then staged up to four times (binary64,
+                                one tspan, endpoint output) and persistent elsewhere
+                                (persistent at any size when grid, chunk or refill is
+                                set) */
   SDEH_SCHED_ONE_LAUNCH = 1, /* one lane per trajectory, grid covers the ensemble */
   SDEH_SCHED_PERSISTENT = 2, /* resident grid; lanes refill from a device atomic queue */
   SDEH_SCHED_STAGED = 3      /* adaptive solvers with endpoint output, one lane per

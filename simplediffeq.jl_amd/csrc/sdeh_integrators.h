@@ -1945,19 +1945,13 @@ __device__ __forceinline__ void adaptive_body_wave(const sdeh_kargs& a) {
 }
 
 // A staged solve's parked trajectory, one record per trajectory (layout and size
-// SDEH_PARK_BYTES in sdeh_kargs.h): t, tf, counts and flag, then u, fsal, comp,
+// SDEH_PARK_BYTES in sdeh_kargs.h): t, tf and counts, then u, fsal, comp,
 // p, dt and qold^beta2.
 template <class T, class R, bool F, bool K>
 struct ParkRec {
   static constexpr int N = R::N, P = R::P > 0 ? R::P : 1, NP = R::P;
   __device__ static char* at(const sdeh_kargs& a, int64_t traj) {
     return (char*)a.st_rec + traj * a.st_stride;
-  }
-  __device__ static int32_t flag(const sdeh_kargs& a, int64_t traj) {
-    return ((const int32_t*)at(a, traj))[6];  // byte 24
-  }
-  __device__ static void set_flag(const sdeh_kargs& a, int64_t traj, int32_t f) {
-    ((int32_t*)at(a, traj))[6] = f;
   }
   __device__ static void store(const sdeh_kargs& a, int64_t traj, const T (&u)[N],
                                const T (&fsal)[N], const T (&comp)[N], const T (&pl)[P],
@@ -1967,7 +1961,6 @@ struct ParkRec {
     ((double*)r)[1] = tf;
     ((int32_t*)r)[4] = nacc;
     ((int32_t*)r)[5] = nrej;
-    ((int32_t*)r)[6] = 1;
     T* v = (T*)(r + 32);
 #pragma unroll
     for (int c = 0; c < N; ++c) *v++ = u[c];
@@ -2105,22 +2098,16 @@ __device__ __forceinline__ void adaptive_body(const sdeh_kargs& a) {
         const int kmin = a.refill_min < 64 / R::G ? a.refill_min : 64 / R::G;
         if (__popcll(__ballot(want)) < kmin) want = false;
       }
-      for (;;) {
-        int64_t slot, claimed = -1;
-        if constexpr (ORDER_WIN)
-          slot = wave_claim_win(cold_args<T>(a), want, qbase, qlim, drained, qwin, qword, claimed);
-        else
-          slot = wave_claim(cold_args<T>(a), want, qbase, qlim, drained);
-        if constexpr (R::G > 1)  // the group leader claimed; its group follows
-          slot = (int64_t)__shfl((long long)slot, (int)(__lane_id() & ~(unsigned)(R::G - 1)));
-        if (slot >= 0) {
-          traj = ORDER_WIN ? claimed : slot_traj(cold_args<T>(a), slot);
-          active = fresh = traj >= 0;
-          // a resumed launch skips the trajectories that ended in the first stage
-          if (STAGED && a.resume && active && Park::flag(cold_args<T>(a), traj) == 0) active = fresh = false;
-        }
-        want = !active && lead;
-        if (!STAGED || !a.resume || drained || __ballot(want && slot >= 0) == 0ull) break;
+      int64_t slot, claimed = -1;
+      if constexpr (ORDER_WIN)
+        slot = wave_claim_win(cold_args<T>(a), want, qbase, qlim, drained, qwin, qword, claimed);
+      else
+        slot = wave_claim(cold_args<T>(a), want, qbase, qlim, drained);
+      if constexpr (R::G > 1)  // the group leader claimed; its group follows
+        slot = (int64_t)__shfl((long long)slot, (int)(__lane_id() & ~(unsigned)(R::G - 1)));
+      if (slot >= 0) {
+        traj = ORDER_WIN ? claimed : slot_traj(cold_args<T>(a), slot);
+        active = fresh = traj >= 0;
       }
     }
     if (__ballot(active) == 0ull) break;
@@ -2316,8 +2303,7 @@ __device__ __forceinline__ void adaptive_body(const sdeh_kargs& a) {
           // remaining attempts extrapolated from the first stage's progress
           const double t0 = ka.tspan ? ka.tspan[traj] : ka.t0;
           key = (double)ka.stage_cap * ((tf - t) / (t - t0));
-        } else {
-          Park::set_flag(ka, traj, 0);
+          if (!(key > 0.0)) key = 1.0;  // 0 says ended
         }
         ka.st_key[traj] = key;
       }

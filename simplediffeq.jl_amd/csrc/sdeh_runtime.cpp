@@ -48,8 +48,8 @@ SDEH_HIDDEN hipError_t sdeh_util_check_order(const int64_t*, int64_t, int32_t*, 
                                              hipStream_t);
 SDEH_HIDDEN hipError_t sdeh_util_span_order(const double*, int64_t, unsigned*, int64_t*,
                                             hipStream_t);
-SDEH_HIDDEN hipError_t sdeh_util_key_order(const double*, int64_t, unsigned*, int64_t*,
-                                           hipStream_t);
+SDEH_HIDDEN hipError_t sdeh_util_resume_order(const double*, int64_t, unsigned*, int64_t*,
+                                              unsigned long long*, hipStream_t);
 SDEH_HIDDEN hipError_t sdeh_util_logkey_order(const float*, int64_t, unsigned*, int64_t*,
                                               hipStream_t);
 SDEH_HIDDEN size_t sdeh_util_span_scratch_bytes();
@@ -611,9 +611,9 @@ size_t staged_stride(const sdeh_solve_desc* d, const Plan& pl) {
 //                in binary32 with several lanes per trajectory).  While every wave is
 //                resident the queue only costs: its atomics, its reset, and waves that take
 //                64 slots each while others get none.
-//   staged       one tspan, endpoint output, beyond resident: its first pass ranks the
-//                trajectories (scratch bounded by kStagedBytes; no visit counters, which
-//                would count a resumed trajectory twice).
+//   staged       binary64, one tspan, endpoint output, from there to 4 x: its first pass
+//                ranks the trajectories (scratch bounded by kStagedBytes; no visit
+//                counters, which would count a resumed trajectory twice).
 //   persistent   the rest.
 // Beyond resident one launch gains while a wave's trajectories are about as long as each
 // other and loses once they are not, which only the solve itself shows, so the line is where
@@ -638,10 +638,18 @@ size_t staged_stride(const sdeh_solve_desc* d, const Plan& pl) {
 //   the same, ATsit5 binary32 (65,536)
 //     like growth rates                   547 |   480     911 |   780   1,740 | 1,513
 //     rates over two decades            2,146 | 2,039   2,358 | 2,735   4,104 | 5,780
-// Staged, one tspan ATsit5 binary64 (persistent | one launch | staged):
-//     262,144    1,406 | 1,066 | 1,025
-//     524,288    1,896 | 1,860 | 1,505
-//   2,097,152    5,428 | 6,542 | 4,810
+// Parking a trajectory and resuming it costs most where it was nearly done, at mean attempts
+// about the first pass's kStageAttempts, the more the further the records outgrow the caches.
+// Queue | staged (us), Lorenz ATsit5 (n = 2 x, 4 x, 6.4 x resident):
+//   binary64  16 attempts   286 |   268
+//             31            405 |   417     673 |   727     946 | 1,108
+//             44            532 |   490     923 |   874   1,301 | 1,339
+//             161         2,016 | 1,525                   (5 x: 4,667 | 3,302)
+//   binary32  31            366 |   383     584 |   654     814 |   993
+//             56            512 |   501     814 |   877   1,153 | 1,272
+//             161         1,218 |   991           (5 x: 2,808 | 2,173)
+//   binary32, affine, 50    399 |   449     605 |   727     848 | 1,079
+// (binary32 attempts are half as dear and their records not half as large.)
 // One-lane kernels launch blocks of 64 (small ensembles spread over more CUs: 487
 // against 538 us at n = 1,024; the same beyond 65,536), the others blocks of 256 (their
 // LDS exchange buffers are sized for four waves: 12.9 against 7.9 ms in blocks of 64).
@@ -658,7 +666,7 @@ Shape default_shape(sdeh_ctx* c, const Plan& pl, int dtype, int64_t n, bool sort
   const int64_t times = lanes > 1 ? (dtype == SDEH_F32 ? 2 : 1)
                                   : (sorted && pl.save == SAVE_END ? 3 : 1);
   sh.chunk = 64 / lanes;
-  if (can_stage && !sorted && work > resident) {
+  if (can_stage && !sorted && dtype == SDEH_F64 && work > resident && work <= 4 * resident) {
     sh.schedule = SDEH_SCHED_STAGED;
   } else if (work <= times * resident) {
     sh.schedule = SDEH_SCHED_ONE_LAUNCH;
@@ -994,9 +1002,12 @@ int check_order_host(sdeh_ctx* c, const int64_t* order, int64_t n) {
 // running park their state and an estimate of the attempts they still need, the
 // estimates are counting-sorted (largest first), and a persistent launch resumes the
 // parked trajectories in that order, so the longest start first and the end of the
-// launch drains less.  Parking stores the whole per-trajectory state (one record each,
-// so the resumed pass reads one or two cache lines per trajectory whatever the order),
-// and every trajectory takes the same steps as in one launch.
+// launch drains less.  Its queue starts behind the trajectories that have ended, which
+// the order does not name: with them in it, an ensemble of short trajectories paid for
+// a queue of ended ones (linear decay, 14 attempts each, 2.6 M trajectories 1,090 us, now 561).
+// Parking stores the whole per-trajectory state (one record each, so the resumed pass
+// reads one or two cache lines per trajectory whatever the order), and every trajectory
+// takes the same steps as in one launch.
 int launch_staged(sdeh_ctx* c, const Plan& pl, const KernelRef& k, int grid, int block,
                   unsigned long long* queue, hipStream_t s) {
   sdeh_kargs a1 = pl.a;
@@ -1006,14 +1017,13 @@ int launch_staged(sdeh_ctx* c, const Plan& pl, const KernelRef& k, int grid, int
   a1.resume = 0;
   const int64_t g1 = (a1.n * k.lanes + block - 1) / block;
   HIPCHK(c, launch(k, (int)g1, block, &a1, s));
-  HIPCHK(c, sdeh_util_key_order(a1.st_key, a1.n, pl.st_hist, pl.st_order, s));
+  HIPCHK(c, sdeh_util_resume_order(a1.st_key, a1.n, pl.st_hist, pl.st_order, queue, s));
   sdeh_kargs a2 = pl.a;
   a2.persistent = 1;
   a2.order = pl.st_order;
   a2.stage_cap = 0;
   a2.resume = 1;
   if (a2.refill_min == 0) a2.refill_min = kRefill;  // the plan's own launch has no queue
-  HIPCHK(c, sdeh_util_zero_u64(queue, 1, s));
   HIPCHK(c, launch(k, grid, block, &a2, s));
   return SDEH_OK;
 }

@@ -193,6 +193,9 @@ struct BucketSrc {
   const int32_t* cnt;   // [n]: weight cnt[i] + cnt2[i]
   const int32_t* cnt2;
   int64_t n;
+  // key only: bucket 0 holds the keys of 0 (ended trajectories) and nothing else, comes
+  // first in the order and is counted, but not written
+  bool resume;
   __device__ __forceinline__ int operator()(int64_t i) const {
     if (lkey) {
       // 16 * log2(exp(-k)) = -k * 16 / ln 2: 16 buckets per octave, evenly spaced
@@ -205,6 +208,11 @@ struct BucketSrc {
       return b < 1 ? 1 : b;
     }
     if (cnt) return weight_bucket((double)cnt[i] + (double)cnt2[i]);
+    if (resume) {
+      const double k = key[i];
+      const int b = weight_bucket(k);
+      return k == 0.0 ? 0 : (b < 1 ? 1 : b);
+    }
     return weight_bucket(key ? key[i] : tspan[n + i] - tspan[i]);
   }
 };
@@ -248,22 +256,25 @@ __global__ void __launch_bounds__(SPAN_THREADS) span_hist(BucketSrc src, unsigne
 // the order (bucket SPAN_BUCKETS-1 .. 0, then block 0 .. SPAN_BLOCKS-1), in three
 // passes over tiles of SPAN_TILE entries of that order: the tile sums, their scan in
 // one block, then each tile scanned and offset in place.  Entry e of the order is
-// bucket SPAN_BUCKETS-1 - e / SPAN_BLOCKS of block e % SPAN_BLOCKS.
+// bucket SPAN_BUCKETS-1 - e / SPAN_BLOCKS of block e % SPAN_BLOCKS; a resumed solve's
+// order starts with bucket 0 (`first` = 1) and goes on with SPAN_BUCKETS-1 .. 1.
 constexpr int SPAN_TILE = 1024;  // 256 threads x 4 entries
 constexpr int SPAN_TILES = SPAN_BUCKETS * SPAN_BLOCKS / SPAN_TILE;
 static_assert(SPAN_BUCKETS * SPAN_BLOCKS % SPAN_TILE == 0, "whole tiles");
 static_assert(SPAN_TILES == 256, "one 256-thread block scans the tile sums");
 
-__device__ __forceinline__ size_t span_entry(int64_t e) {
-  const int64_t k = SPAN_BUCKETS - 1 - e / SPAN_BLOCKS, b = e % SPAN_BLOCKS;
+__device__ __forceinline__ size_t span_entry(int64_t e, int first) {
+  const int64_t k = (SPAN_BUCKETS - 1 + first - e / SPAN_BLOCKS) % SPAN_BUCKETS,
+                b = e % SPAN_BLOCKS;
   return (size_t)b * SPAN_BUCKETS + (size_t)k;
 }
 
-__global__ void __launch_bounds__(256) span_tile_sums(const unsigned* bh, unsigned* tsum) {
+__global__ void __launch_bounds__(256) span_tile_sums(const unsigned* bh, unsigned* tsum,
+                                                      int first) {
   const int64_t e0 = (int64_t)blockIdx.x * SPAN_TILE + 4 * threadIdx.x;
   int64_t v = 0;
 #pragma unroll
-  for (int j = 0; j < 4; ++j) v += bh[span_entry(e0 + j)];
+  for (int j = 0; j < 4; ++j) v += bh[span_entry(e0 + j, first)];
   int64_t total = 0;
   (void)block_exclusive_scan(v, &total);
   if (threadIdx.x == 0) tsum[blockIdx.x] = (unsigned)total;
@@ -276,27 +287,31 @@ __global__ void __launch_bounds__(256) span_scan_tiles(unsigned* tsum) {
   tsum[threadIdx.x] = (unsigned)ex;
 }
 
-__global__ void __launch_bounds__(256) span_tile_offsets(unsigned* bh, const unsigned* tsum) {
+__global__ void __launch_bounds__(256) span_tile_offsets(unsigned* bh, const unsigned* tsum,
+                                                         int first) {
   const int64_t e0 = (int64_t)blockIdx.x * SPAN_TILE + 4 * threadIdx.x;
   unsigned c[4];
   int64_t v = 0;
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
-    c[j] = bh[span_entry(e0 + j)];
+    c[j] = bh[span_entry(e0 + j, first)];
     v += c[j];
   }
   int64_t total = 0;
   unsigned o = tsum[blockIdx.x] + (unsigned)block_exclusive_scan(v, &total);
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
-    bh[span_entry(e0 + j)] = o;
+    bh[span_entry(e0 + j, first)] = o;
     o += c[j];
   }
 }
 
 __global__ void __launch_bounds__(SPAN_THREADS) span_scatter(BucketSrc src, const unsigned* bh,
-                                                             int64_t* order) {
+                                                             int64_t* order,
+                                                             unsigned long long* queue) {
   __shared__ unsigned cur[SPAN_BUCKETS];
+  // a resumed launch's queue starts at the first trajectory that has not ended
+  if (src.resume && blockIdx.x == 0 && threadIdx.x == 0) *queue = bh[SPAN_BUCKETS - 1];
   for (int k = threadIdx.x; k < SPAN_BUCKETS; k += blockDim.x)
     cur[k] = bh[(size_t)blockIdx.x * SPAN_BUCKETS + k];
   __syncthreads();
@@ -311,7 +326,8 @@ __global__ void __launch_bounds__(SPAN_THREADS) span_scatter(BucketSrc src, cons
     }
 #pragma unroll
     for (int j = 0; j < SPAN_BATCH; ++j)
-      if (b[j] >= 0) order[atomicAdd(cur + b[j], 1u)] = i0 + (int64_t)j * blockDim.x;
+      if (b[j] > 0 || (b[j] == 0 && !src.resume))
+        order[atomicAdd(cur + b[j], 1u)] = i0 + (int64_t)j * blockDim.x;
   }
 }
 
@@ -424,27 +440,33 @@ extern "C" __attribute__((visibility("hidden"))) hipError_t sdeh_util_pack_offse
 
 // order[0..n) = trajectories by decreasing weight (see span_hist).  bh: scratch of
 // sdeh_util_span_scratch_bytes().  n must fit in 32 bits (the slot counters).
-static hipError_t bucket_order(BucketSrc src, unsigned* bh, int64_t* order, hipStream_t s) {
+static hipError_t bucket_order(BucketSrc src, unsigned* bh, int64_t* order, hipStream_t s,
+                               unsigned long long* queue = nullptr) {
   if (src.n <= 0) return hipSuccess;
   unsigned* tsum = bh + (size_t)SPAN_BLOCKS * SPAN_BUCKETS;
+  const int first = src.resume ? 1 : 0;
   hipLaunchKernelGGL(span_hist, dim3(SPAN_BLOCKS), dim3(SPAN_THREADS), 0, s, src, bh);
-  hipLaunchKernelGGL(span_tile_sums, dim3(SPAN_TILES), dim3(256), 0, s, bh, tsum);
+  hipLaunchKernelGGL(span_tile_sums, dim3(SPAN_TILES), dim3(256), 0, s, bh, tsum, first);
   hipLaunchKernelGGL(span_scan_tiles, dim3(1), dim3(SPAN_TILES), 0, s, tsum);
-  hipLaunchKernelGGL(span_tile_offsets, dim3(SPAN_TILES), dim3(256), 0, s, bh, tsum);
-  hipLaunchKernelGGL(span_scatter, dim3(SPAN_BLOCKS), dim3(SPAN_THREADS), 0, s, src, bh, order);
+  hipLaunchKernelGGL(span_tile_offsets, dim3(SPAN_TILES), dim3(256), 0, s, bh, tsum, first);
+  hipLaunchKernelGGL(span_scatter, dim3(SPAN_BLOCKS), dim3(SPAN_THREADS), 0, s, src, bh, order,
+                     queue);
   return hipGetLastError();
 }
 
 extern "C" __attribute__((visibility("hidden"))) hipError_t sdeh_util_span_order(
     const double* tspan, int64_t n, unsigned* bh, int64_t* order, hipStream_t s) {
-  return bucket_order(BucketSrc{tspan, nullptr, nullptr, nullptr, nullptr, n}, bh, order, s);
+  return bucket_order(BucketSrc{tspan, nullptr, nullptr, nullptr, nullptr, n, false}, bh, order, s);
 }
 
-// order[0..n) = trajectories by decreasing key[i] (keys <= 0 and NaN last), on the
-// same buckets and scratch as sdeh_util_span_order.
-extern "C" __attribute__((visibility("hidden"))) hipError_t sdeh_util_key_order(
-    const double* key, int64_t n, unsigned* bh, int64_t* order, hipStream_t s) {
-  return bucket_order(BucketSrc{nullptr, key, nullptr, nullptr, nullptr, n}, bh, order, s);
+// A resumed solve's order: order[e..n) = the trajectories whose key is not 0, by decreasing key
+// (keys < 0 and NaN last), e the number of those whose key is 0, and *queue = e.  order[0..e)
+// is not written.  Same buckets and scratch as sdeh_util_span_order.
+extern "C" __attribute__((visibility("hidden"))) hipError_t sdeh_util_resume_order(
+    const double* key, int64_t n, unsigned* bh, int64_t* order, unsigned long long* queue,
+    hipStream_t s) {
+  return bucket_order(BucketSrc{nullptr, key, nullptr, nullptr, nullptr, n, true}, bh, order, s,
+                      queue);
 }
 
 // order[0..n) = trajectories by decreasing cnt[i] + cnt2[i] (the attempts a counting pass
@@ -452,7 +474,7 @@ extern "C" __attribute__((visibility("hidden"))) hipError_t sdeh_util_key_order(
 extern "C" __attribute__((visibility("hidden"))) hipError_t sdeh_util_count_order(
     const int32_t* cnt, const int32_t* cnt2, int64_t n, unsigned* bh, int64_t* order,
     hipStream_t s) {
-  return bucket_order(BucketSrc{nullptr, nullptr, nullptr, cnt, cnt2, n}, bh, order, s);
+  return bucket_order(BucketSrc{nullptr, nullptr, nullptr, cnt, cnt2, n, false}, bh, order, s);
 }
 
 // order[0..n) = trajectories by increasing lkey[i] (the cost model's -log predicted
@@ -460,7 +482,7 @@ extern "C" __attribute__((visibility("hidden"))) hipError_t sdeh_util_count_orde
 // keys last.  Same scratch as sdeh_util_span_order.
 extern "C" __attribute__((visibility("hidden"))) hipError_t sdeh_util_logkey_order(
     const float* lkey, int64_t n, unsigned* bh, int64_t* order, hipStream_t s) {
-  return bucket_order(BucketSrc{nullptr, nullptr, lkey, nullptr, nullptr, n}, bh, order, s);
+  return bucket_order(BucketSrc{nullptr, nullptr, lkey, nullptr, nullptr, n, false}, bh, order, s);
 }
 
 // Scratch of the bucket sorts: the per-block counts and the tile sums.

@@ -68,3 +68,59 @@ def test_one_launch_ends_where_unlike_lengths_lose(name, rhs, alg, dtype, points
     for f in FIELDS + (("u_saveat",) if points else ()):
         assert bits_equal(got.numpy(f), ref.numpy(f)), f
     c.close()
+
+
+@pytest.mark.parametrize("dtype,times,add,want", [
+    (_abi.F64, 1, 0, _abi.SCHED_ONE_LAUNCH), (_abi.F64, 1, 1, _abi.SCHED_STAGED),
+    (_abi.F64, 4, 0, _abi.SCHED_STAGED), (_abi.F64, 4, 1, _abi.SCHED_PERSISTENT),
+    (_abi.F32, 1, 0, _abi.SCHED_ONE_LAUNCH), (_abi.F32, 1, 1, _abi.SCHED_PERSISTENT)])
+def test_where_the_staged_schedule_is_taken(dtype, times, add, want):
+    c = runtime.Context(0)
+
+    def solve(n, sched, **more):
+        u0, p = inputs.lorenz_wide(n, seed=5)
+        d = runtime.make_desc(_abi.ALG_ATSIT5, n_traj=n, dtype=dtype, tspan=(0.0, 0.2), dt=0.1,
+                              abstol=1e-6, reltol=1e-4, schedule=sched, **more)
+        b = runtime.EnsembleBuffers(d, 3, u0, p, backend="torch", device="cuda:0")
+        c.solve(d, b)
+        return b, c.stats()
+
+    _, st = solve(100, _abi.SCHED_PERSISTENT, block=256)
+    n = times * st["grid"] * 256 + add
+    got, st = solve(n, _abi.SCHED_AUTO)
+    assert st["schedule"] == want
+    ref, _ = solve(n, _abi.SCHED_ONE_LAUNCH)
+    for f in FIELDS:
+        assert bits_equal(got.numpy(f), ref.numpy(f)), f
+    c.close()
+
+
+@pytest.mark.parametrize("alg,kahan", [(_abi.ALG_ATSIT5, False), (_abi.ALG_AVERN7, False),
+                                       (_abi.ALG_ATSIT5, True)])
+@pytest.mark.parametrize("parked", ["none", "some", "all", "endless"])
+@pytest.mark.parametrize("n", [2, 63, 65, 5003])
+def test_a_staged_solve_resumes_exactly_the_parked(ctx, alg, kahan, parked, n):
+    """Its second launch starts behind the trajectories that ended in the first: none, some or
+    all of them, and trajectories whose estimate of the attempts still to come is infinite."""
+    u0, p = inputs.lorenz_wide(n, seed=9)
+    span = {"none": 0.01, "some": 3.0, "all": 30.0, "endless": 3.0}[parked]
+    ts = np.zeros((2, n))
+    ts[1] = np.linspace(0.0, span, n) if parked == "some" else span
+    if parked == "endless":
+        ts[1, ::3] = np.inf
+    out = []
+    for sched in (_abi.SCHED_ONE_LAUNCH, _abi.SCHED_STAGED):
+        d = runtime.make_desc(alg, dtype=_abi.F32 if kahan else _abi.F64, n_traj=n, dt=0.1,
+                              abstol=1e-7, reltol=1e-6, schedule=sched, maxiters=200,
+                              precision=_abi.PREC_KAHAN if kahan else _abi.PREC_PLAIN)
+        b = runtime.EnsembleBuffers(d, 3, u0, p, tspan=ts)
+        ctx.solve(d, b, allow=(_abi.E_DTMIN,))
+        assert ctx.stats()["schedule"] == sched
+        out.append(b)
+    att = out[0].naccept + out[0].nreject
+    if parked == "none":
+        assert att.max() < 32
+    elif parked != "some":
+        assert att.max() > 32
+    for f in FIELDS:
+        assert bits_equal(out[0].numpy(f), out[1].numpy(f)), f
