@@ -1476,11 +1476,13 @@ __device__ __forceinline__ X in_vgpr_if(X x) {
 // trajectories, 256 points 7,130 / 7,065 us; holding coefficients there took 7,230).
 // The binary32 kernels have scalar registers for all of them, and a wave that refills its
 // lanes from the queue waits for the reloads each time (2^20 ATsit5 trajectories in the order
-// of random keys 871 / 959 us), so they keep the arguments as passed.
+// of random keys 871 / 959 us), so they keep the arguments as passed, except in the group
+// layout, which runs its chunk's trajectories four at a time (GLV-16 on 16 lanes, 300
+// trajectories on the queue 646 / 577 us).
 // (Every kernel takes sdeh_kargs first and by value.)
-template <class T>
+template <class T, class R>
 __device__ __forceinline__ const sdeh_kargs& cold_args(const sdeh_kargs& a) {
-  if constexpr (sizeof(T) == 4) {
+  if constexpr (sizeof(T) == 4 && (R::G == 1 || IsWave<R>::value)) {
     return a;
   } else {
     auto k = __builtin_amdgcn_kernarg_segment_ptr();
@@ -1728,17 +1730,17 @@ __device__ __forceinline__ void adaptive_body_wave(const sdeh_kargs& a) {
         const int kmin = a.refill_min < SLOTS ? a.refill_min : SLOTS;
         if (__popcll(__ballot(want)) < kmin) want = false;
       }
-      int64_t slot = wave_claim(cold_args<T>(a), want, qbase, qlim, drained);
+      int64_t slot = wave_claim(cold_args<T, R>(a), want, qbase, qlim, drained);
       slot = (int64_t)__shfl((long long)slot, lane & (SLOTS - 1));  // from the slot's lead lane
       if (slot >= 0) {
-        traj = slot_traj(cold_args<T>(a), slot);
+        traj = slot_traj(cold_args<T, R>(a), slot);
         active = fresh = traj >= 0;
       }
     }
     if (__ballot(active) == 0ull) break;
 
     if (fresh) {  // start trajectory `traj` (gpuatsit5.jl:221-241)
-      const sdeh_kargs& ka = cold_args<T>(a);
+      const sdeh_kargs& ka = cold_args<T, R>(a);
       const int64_t n = ka.n;
       if (lead) note_visit(ka, traj);
       load_state<T, R>(uprev, ka.u0, n, traj);
@@ -1926,7 +1928,7 @@ __device__ __forceinline__ void adaptive_body_wave(const sdeh_kargs& a) {
     }
 
     if (ret >= 0) {  // trajectory ends: write outputs (gpuatsit5.jl:322-329)
-      const sdeh_kargs& ka = cold_args<T>(a);
+      const sdeh_kargs& ka = cold_args<T, R>(a);
       const int64_t n = ka.n;
       if (SAVE == SAVE_STEPS && ret == RET_DEFAULT && sk.kept < sk.n) ret = RET_SAVE_OVERFLOW;
       store_state<T, R>(ka.u_end, 0, n, traj, uprev);
@@ -2100,13 +2102,13 @@ __device__ __forceinline__ void adaptive_body(const sdeh_kargs& a) {
       }
       int64_t slot, claimed = -1;
       if constexpr (ORDER_WIN)
-        slot = wave_claim_win(cold_args<T>(a), want, qbase, qlim, drained, qwin, qword, claimed);
+        slot = wave_claim_win(cold_args<T, R>(a), want, qbase, qlim, drained, qwin, qword, claimed);
       else
-        slot = wave_claim(cold_args<T>(a), want, qbase, qlim, drained);
+        slot = wave_claim(cold_args<T, R>(a), want, qbase, qlim, drained);
       if constexpr (R::G > 1)  // the group leader claimed; its group follows
         slot = (int64_t)__shfl((long long)slot, (int)(__lane_id() & ~(unsigned)(R::G - 1)));
       if (slot >= 0) {
-        traj = ORDER_WIN ? claimed : slot_traj(cold_args<T>(a), slot);
+        traj = ORDER_WIN ? claimed : slot_traj(cold_args<T, R>(a), slot);
         active = fresh = traj >= 0;
       }
     }
@@ -2115,7 +2117,7 @@ __device__ __forceinline__ void adaptive_body(const sdeh_kargs& a) {
 
     if (fresh && STAGED && a.resume) {  // continue a parked trajectory
       fresh = false;
-      const sdeh_kargs& ka = cold_args<T>(a);
+      const sdeh_kargs& ka = cold_args<T, R>(a);
       note_visit(ka, traj);
       Park::load(ka, traj, uprev, fsal, comp, pl, t, tf, dt, qold_pow, nacc, nrej);
       attempts = (int64_t)nacc + nrej;
@@ -2123,7 +2125,7 @@ __device__ __forceinline__ void adaptive_body(const sdeh_kargs& a) {
     }
     if (fresh) {  // start trajectory `traj` (gpuatsit5.jl:221-241)
       fresh = false;
-      const sdeh_kargs& ka = cold_args<T>(a);
+      const sdeh_kargs& ka = cold_args<T, R>(a);
       const int64_t n = ka.n;
       if (lead) note_visit(ka, traj);
       load_state<T, R>(uprev, ka.u0, n, traj);
@@ -2157,7 +2159,7 @@ __device__ __forceinline__ void adaptive_body(const sdeh_kargs& a) {
     } else if ((double)dt < DTMIN) {  // :256
       ret = RET_DTMIN;
     } else if (attempts >= att_lim) {  // maxiters, or the first stage's cap (parked)
-      ret = attempts >= cold_args<T>(a).maxiters ? RET_MAXITERS : RET_PARKED;
+      ret = attempts >= cold_args<T, R>(a).maxiters ? RET_MAXITERS : RET_PARKED;
     } else {
       ++attempts;
       T u[N], err[N], comp_new[N];
@@ -2280,7 +2282,7 @@ __device__ __forceinline__ void adaptive_body(const sdeh_kargs& a) {
     }
 
     if (ret != -1) {  // trajectory ends or parks: write outputs (gpuatsit5.jl:322-329)
-      const sdeh_kargs& ka = cold_args<T>(a);
+      const sdeh_kargs& ka = cold_args<T, R>(a);
       const int64_t n = ka.n;
       if (STEPS && ret == RET_DEFAULT && sk.kept < sk.n) ret = RET_SAVE_OVERFLOW;
       const bool parked = STAGED && ret == RET_PARKED;
