@@ -2007,7 +2007,7 @@ struct ParkRec {
   }
 };
 
-template <class T, class R, int ALG, int SAVE, bool KAHAN, bool LONE = false>
+template <class T, class R, int ALG, int SAVE, bool KAHAN, bool LONE = false, int WAVES = 0>
 __device__ __forceinline__ void adaptive_body(const sdeh_kargs& a) {
   if constexpr (IsWave<R>::value) {
     adaptive_body_wave<T, R, ALG, SAVE, KAHAN>(a);
@@ -2015,7 +2015,11 @@ __device__ __forceinline__ void adaptive_body(const sdeh_kargs& a) {
   }
   constexpr int N = R::N;
   constexpr int P = R::P > 0 ? R::P : 1;
-  constexpr bool HOLD = sizeof(T) == 8 && R::G == 1 && N <= 4;
+  // Not where the scalar registers are short already: held to eight waves per SIMD (Lorenz
+  // AVern7, 400,003 trajectories 4,050 / 2,770 us without), and AVern9's dense output (a traced
+  // right-hand side, 5,003 trajectories with 101 points 1,263 / 1,205; 1,210 before any were).
+  constexpr bool HOLD = sizeof(T) == 8 && R::G == 1 && N <= 4 && WAVES < 8 &&
+                        !(ALG == ALG_AVERN9 && SAVE == SAVE_AT);
   constexpr double DTMIN = (ALG == ALG_AVERN9) ? (double)1.0e-7f : 1.0e-14;  // gpuvern9.jl:466
   constexpr double SNAP = DTMIN;                                              // gpuvern9.jl:591
   // build_adaptive_controller_cache(T), src/SimpleDiffEq.jl:67-77
@@ -2691,7 +2695,7 @@ __global__ void __launch_bounds__(256)
                                        : WAVES > 0 ? WAVES
                                                  : sdeh::WavesHint<T, R, ALG, SAVE>::value)))
     sdeh_adaptive_kernel(sdeh_kargs a) {
-  sdeh::adaptive_body<T, R, ALG, SAVE, KAHAN, WAVES == 1>(a);
+  sdeh::adaptive_body<T, R, ALG, SAVE, KAHAN, WAVES == 1, WAVES>(a);
 }
 
 // TPL trajectories per lane (adaptive_body_multi).

@@ -293,8 +293,8 @@ int user_kernel(sdeh_ctx* c, int64_t rhs, int alg, int dtype, int save, int kaha
     snprintf(wrap, sizeof wrap,
              "extern \"C\" __global__ void __launch_bounds__(256) "
              "__attribute__((amdgpu_waves_per_eu(%d))) sdeh_user_kernel(sdeh_kargs a) "
-             "{ sdeh::adaptive_body<%s, sdeh_user_rhs, %d, %d, %s>(a); }\n",
-             waves, T, alg, save, kahan ? "true" : "false");
+             "{ sdeh::adaptive_body<%s, sdeh_user_rhs, %d, %d, %s, false, %d>(a); }\n",
+             waves, T, alg, save, kahan ? "true" : "false", waves);
   else if (is_adaptive(alg))
     snprintf(wrap, sizeof wrap,
              "extern \"C\" __global__ void __launch_bounds__(256) "
