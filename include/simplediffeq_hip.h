@@ -187,7 +187,9 @@ typedef struct sdeh_solve_desc {
                                lane holds a whole trajectory; or either layout's size
                                (4, 16) itself (4 also runs binary32 ATsit5, on
                                v_mfma_f32_16x16x4f32: 0 takes it beyond 64
-                               trajectories).  Results are identical. */
+                               trajectories unless the persistent or staged schedule,
+                               grid, chunk or refill is asked for).  Results are
+                               identical. */
   int32_t save_layout;      /* sdeh_save_layout of u_saveat, u_steps and t_steps */
   int32_t span_order;       /* 0: with per-trajectory tspans (io->tspan) and no io->order,
                                hand trajectories to lanes longest span first (fewer

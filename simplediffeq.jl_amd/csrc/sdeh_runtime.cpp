@@ -462,10 +462,14 @@ int resolve_kernel(sdeh_ctx* c, int64_t rhs, int alg, int dtype, int save, int k
 //    524,288   1,840 | 1,400   2,037 | 1,733
 // (f32 matrix products run at twice the vector rate and beside it, a wave holds a quarter of
 // the trajectories, and the kernel's 107 registers leave four waves per SIMD instead of two.)
-// An ensemble of at most 64, one wave either way, stays on one lane.
+// A caller that asks for the queue, whose default chunk is four of this layout's waves, keeps
+// one lane (120,001 trajectories over 20 time units 264 | 329).  An ensemble of at most 64
+// keeps one lane too, although the layout is the faster one there as well (1 trajectory 396 |
+// 90, 64 trajectories 390 | 97): callers of `lanes` = 0 have been promised it; lanes = 4 asks.
 int auto_lanes(const sdeh_solve_desc* d, int save, int kahan) {
-  if (d->lanes != 0 || d->dtype != SDEH_F32 || d->n_traj <= 64 || d->waves || d->per_lane ||
-      d->schedule == SDEH_SCHED_STAGED)
+  const bool queue = d->schedule == SDEH_SCHED_PERSISTENT || d->schedule == SDEH_SCHED_STAGED ||
+                     (d->schedule == SDEH_SCHED_AUTO && (d->grid || d->chunk || d->refill));
+  if (d->lanes != 0 || d->dtype != SDEH_F32 || d->n_traj <= 64 || d->waves || d->per_lane || queue)
     return d->lanes;
   const Builtin* b = find_builtin(d->rhs);
   return b && b->mgroup > 1 && b->mgroup_lookup(d->dtype, d->alg, save, kahan, 0, 1) ? b->mgroup
