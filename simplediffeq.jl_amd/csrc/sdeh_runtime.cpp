@@ -1919,13 +1919,19 @@ int sdeh_autotune(sdeh_ctx* c, const sdeh_solve_desc* d, const sdeh_io* io, sdeh
   Shape best_shape;
   sdeh_stats best_stats{};
   TuneKey key;
+  // The layout is resolved once, from the caller's descriptor: every candidate runs on it, and
+  // so does the solve that takes the winner (its schedule is not the candidate's, and lanes = 0
+  // may stand for another layout there).
+  sdeh_solve_desc base_desc = *d;
   {  // the shape search runs the caller's kernel choice, not an earlier tuning's
     Plan pl;
     int r = plan_solve(c, d, io, &pl);
     if (r) return r;
     key = TuneKey(d->rhs, d->alg, d->dtype, pl.save, pl.kahan, pl.k.lanes);
     c->tuned.erase(key);
+    base_desc.lanes = pl.k.lanes;
   }
+  d = &base_desc;
   for (const Cand& k : cands) {
     sdeh_solve_desc dd = *d;
     dd.schedule = k.sched;
