@@ -344,7 +344,9 @@ int sdeh_graph_destroy(sdeh_ctx* ctx, int64_t graph_handle);
  * for the given problem on device buffers, then the register-cap variants (waves)
  * of the best one and the two-trajectories-per-lane variant (one launch and
  * persistent) where they are built, and store the best for (alg, rhs, dtype, save
- * mode, precision, lanes).  Later solves with tuned fields left 0 use it. */
+ * mode, precision, lanes, packed layout or not).  Later solves with tuned fields left 0
+ * use it.  A packed solve beyond what fits the GPU at once keeps its default passes
+ * (counted, then saved by decreasing attempts) unless they were timed here and lost. */
 int sdeh_autotune(sdeh_ctx* ctx, const sdeh_solve_desc* d, const sdeh_io* io,
                   sdeh_stats* best);
 

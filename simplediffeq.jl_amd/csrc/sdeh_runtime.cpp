@@ -140,6 +140,9 @@ struct KernelRef {
 struct Shape {
   int32_t schedule = SDEH_SCHED_ONE_LAUNCH, block = 256, grid = 0, chunk = 64, waves = 0,
           per_lane = 1, refill = 0;
+  // a tuned packed solve's ranked passes (see run_plan) against its shape: 1 faster, 0 not,
+  // -1 not timed (the tuned ensemble was too small for them)
+  int32_t ranked = -1;
 };
 
 // Workgroups of a one-launch grid: every trajectory a lane (or TPL per lane).
@@ -148,7 +151,8 @@ int64_t one_launch_groups(int64_t n, const KernelRef& k, int block) {
   return (lanes + block - 1) / block;
 }
 
-using TuneKey = std::tuple<int64_t, int, int, int, int, int>;  // rhs, alg, dtype, save, kahan, lanes
+// rhs, alg, dtype, save, kahan, lanes, packed
+using TuneKey = std::tuple<int64_t, int, int, int, int, int, bool>;
 
 struct GraphRec {
   hipGraph_t graph = nullptr;
@@ -821,7 +825,8 @@ int plan_solve(sdeh_ctx* c, const sdeh_solve_desc* d, const sdeh_io* io, Plan* p
                 "register-cap and several-trajectories-per-lane variants are adaptive endpoint "
                 "kernels");
   if (adaptive) {
-    auto it = c->tuned.find(TuneKey(d->rhs, d->alg, d->dtype, pl->save, pl->kahan, pl->k.lanes));
+    auto it = c->tuned.find(TuneKey(d->rhs, d->alg, d->dtype, pl->save, pl->kahan, pl->k.lanes,
+                                     pl->packed));
     if (it != c->tuned.end()) sh = it->second;
     else sh.schedule = SDEH_SCHED_PERSISTENT;
     // the kernel variant: the caller's register cap or trajectories per lane, else
@@ -843,8 +848,9 @@ int plan_solve(sdeh_ctx* c, const sdeh_solve_desc* d, const sdeh_io* io, Plan* p
       }
     }
     // (a caller that sets the queue's grid, chunk or refill batch gets the queue)
-    if (it == c->tuned.end() && d->schedule == SDEH_SCHED_AUTO && !d->grid && !d->chunk &&
-        !d->refill && d->n_traj > 0) {
+    const bool open = d->schedule == SDEH_SCHED_AUTO && !d->grid && !d->chunk && !d->refill &&
+                      d->n_traj > 0;
+    if (it == c->tuned.end() && open) {
       const bool piped =
           path == Path::kHost && d->n_traj >= kPipeMin && !io->order && !pl->packed;
       const int64_t n = piped ? (d->n_traj + kPipeChunks - 1) / kPipeChunks : d->n_traj;
@@ -856,21 +862,23 @@ int plan_solve(sdeh_ctx* c, const sdeh_solve_desc* d, const sdeh_io* io, Plan* p
       sh.waves = w;
       sh.per_lane = tp;
       pl->default_staged = sh.schedule == SDEH_SCHED_STAGED;
-      // packed output beyond resident: rank the saving pass by the counting pass
-      pl->pk_ranked = pl->packed && pl->k.lanes == 1 && !io->order && !io->visits && n > 1 &&
-                      n < (1ll << 32) &&
-                      n > (int64_t)c->cus * blocks_per_cu(c, pl->k, 256) * 256 &&
-                      (size_t)n * (staged_stride(d, *pl) + 16) <= kStagedBytes;
-      if (pl->pk_ranked) {
-        sh.schedule = SDEH_SCHED_ONE_LAUNCH;
-        sh.block = 256;
-        pl->span = false;
-        // the kernel that writes its rows by whole sectors, for states of at most 32 bytes
-        KernelRef kr;
-        if ((size_t)pl->n_state * pl->es <= 32 &&
-            !resolve_kernel(c, d->rhs, d->alg, d->dtype, SAVE_RUNS, pl->kahan, 1, &kr))
-          pl->k_runs = kr;
-      }
+    }
+    // Packed output beyond resident: rank the saving pass by the counting pass, unless the
+    // tuner has found this solve's shape to be faster.
+    const int64_t n = d->n_traj;
+    if (open && (it == c->tuned.end() || it->second.ranked != 0) && pl->packed &&
+        pl->k.lanes == 1 && !io->order && !io->visits && n > 1 && n < (1ll << 32) &&
+        n > (int64_t)c->cus * blocks_per_cu(c, pl->k, 256) * 256 &&
+        (size_t)n * (staged_stride(d, *pl) + 16) <= kStagedBytes) {
+      pl->pk_ranked = true;
+      sh.schedule = SDEH_SCHED_ONE_LAUNCH;
+      sh.block = 256;
+      pl->span = false;
+      // the kernel that writes its rows by whole sectors, for states of at most 32 bytes
+      KernelRef kr;
+      if ((size_t)pl->n_state * pl->es <= 32 &&
+          !resolve_kernel(c, d->rhs, d->alg, d->dtype, SAVE_RUNS, pl->kahan, 1, &kr))
+        pl->k_runs = kr;
     }
     if (d->schedule != SDEH_SCHED_AUTO) sh.schedule = d->schedule;
     if (d->block) sh.block = d->block;
@@ -1927,7 +1935,7 @@ int sdeh_autotune(sdeh_ctx* c, const sdeh_solve_desc* d, const sdeh_io* io, sdeh
     Plan pl;
     int r = plan_solve(c, d, io, &pl);
     if (r) return r;
-    key = TuneKey(d->rhs, d->alg, d->dtype, pl.save, pl.kahan, pl.k.lanes);
+    key = TuneKey(d->rhs, d->alg, d->dtype, pl.save, pl.kahan, pl.k.lanes, pl.packed);
     c->tuned.erase(key);
     base_desc.lanes = pl.k.lanes;
   }
@@ -2057,6 +2065,25 @@ int sdeh_autotune(sdeh_ctx* c, const sdeh_solve_desc* d, const sdeh_io* io, sdeh
         best_shape.per_lane = 2;
         best_stats = c->stats;
       }
+    }
+  }
+  // Packed output: the ranked passes, which no schedule names, where they are open to this solve.
+  if (!d->grid && !d->chunk && !d->refill) {
+    sdeh_solve_desc dd = *d;
+    dd.schedule = SDEH_SCHED_AUTO;
+    dd.block = 0;
+    Plan pl;
+    int r = plan_solve(c, &dd, io, &pl);
+    if (r) return r;
+    if (pl.pk_ranked) {
+      double ms = 1e300;
+      for (int rep = 0; rep < 2; ++rep) {
+        r = sdeh_solve(c, &dd, io, SDEH_MEM_DEVICE, nullptr, 1);
+        if (r && r != SDEH_E_DTMIN) return r;
+        ms = c->stats.kernel_ms;
+      }
+      best_shape.ranked = ms < best_ms ? 1 : 0;
+      if (best_shape.ranked) best_stats = c->stats;
     }
   }
   c->err.clear();
