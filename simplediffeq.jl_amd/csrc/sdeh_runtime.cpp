@@ -20,6 +20,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <map>
+#include <set>
 #include <string>
 #include <tuple>
 #include <vector>
@@ -198,6 +199,8 @@ struct sdeh_ctx {
   std::vector<UserRhs> user;
   std::map<std::string, std::pair<hipModule_t, hipFunction_t>> rtc;
   std::map<TuneKey, Shape> tuned;
+  // (rhs, alg, dtype, kahan) whose kernel of whole sectors could not be had
+  std::set<std::tuple<int64_t, int, int, int>> no_runs;
   std::map<int64_t, GraphRec> graphs;
   int64_t next_graph = 1;
   // The device address of the library's static scratch on this context's device
@@ -875,10 +878,17 @@ int plan_solve(sdeh_ctx* c, const sdeh_solve_desc* d, const sdeh_io* io, Plan* p
       sh.block = 256;
       pl->span = false;
       // the kernel that writes its rows by whole sectors, for states of at most 32 bytes
-      KernelRef kr;
-      if ((size_t)pl->n_state * pl->es <= 32 &&
-          !resolve_kernel(c, d->rhs, d->alg, d->dtype, SAVE_RUNS, pl->kahan, 1, &kr))
-        pl->k_runs = kr;
+      const auto id = std::make_tuple(d->rhs, d->alg, d->dtype, pl->kahan);
+      if ((size_t)pl->n_state * pl->es <= 32 && !c->no_runs.count(id)) {
+        KernelRef kr;
+        const std::string err = c->err;
+        if (!resolve_kernel(c, d->rhs, d->alg, d->dtype, SAVE_RUNS, pl->kahan, 1, &kr)) {
+          pl->k_runs = kr;
+        } else {  // row by row, then: no error of this call, and not tried again
+          c->err = err;
+          c->no_runs.insert(id);
+        }
+      }
     }
     if (d->schedule != SDEH_SCHED_AUTO) sh.schedule = d->schedule;
     if (d->block) sh.block = d->block;
