@@ -1146,10 +1146,10 @@ __device__ __forceinline__ void store_row(const sdeh_kargs& a, T* at, const T (&
   }
 }
 
-// saveat: NaN in the rows a trajectory ended before (from `row` on), written when it
-// ends.  Filling the whole output beforehand moved every byte of it twice: GLV-16, 2^17
-// trajectories, 256 points, the fill alone took 404 us of 1,437 in binary32 (2.1 GB) and
-// 830 us of 9,250 in binary64.
+// saveat, where the output was not filled beforehand: NaN in the rows a trajectory ended
+// before (from `row` on), written when it ends.  A fill moves every byte of the output twice:
+// GLV-16, 2^17 trajectories, 256 points, the fill alone took 404 us of 1,437 in binary32
+// (2.1 GB) and 830 us of 9,250 in binary64.
 template <class T, class R>
 __device__ __forceinline__ void save_unreached(const sdeh_kargs& a, int64_t row, int64_t traj) {
   T x[R::N];
@@ -1932,7 +1932,7 @@ __device__ __forceinline__ void adaptive_body_wave(const sdeh_kargs& a) {
       const int64_t n = ka.n;
       if (SAVE == SAVE_STEPS && ret == RET_DEFAULT && sk.kept < sk.n) ret = RET_SAVE_OVERFLOW;
       store_state<T, R>(ka.u_end, 0, n, traj, uprev);
-      if constexpr (SAVE == SAVE_AT) save_unreached<T, R>(ka, cur, traj);
+      if (SAVE == SAVE_AT && !ka.filled) save_unreached<T, R>(ka, cur, traj);
       if constexpr (SAVE == SAVE_STEPS) flush_steps<T, R>(ka, sk);
       if (lead) {
         ka.t_end[traj] = t;
@@ -2292,7 +2292,7 @@ __device__ __forceinline__ void adaptive_body(const sdeh_kargs& a) {
       const bool parked = STAGED && ret == RET_PARKED;
       if (!parked) {
         store_state<T, R>(ka.u_end, 0, n, traj, uprev);
-        if constexpr (SAVE == SAVE_AT) save_unreached<T, R>(ka, cur, traj);
+        if (SAVE == SAVE_AT && !ka.filled) save_unreached<T, R>(ka, cur, traj);
         if constexpr (SAVE == SAVE_STEPS) flush_steps<T, R>(ka, sk);
         if (lead) {
           ka.t_end[traj] = t;
@@ -2650,7 +2650,7 @@ __device__ __forceinline__ void fixed_body(const sdeh_kargs& a) {
     if constexpr (SAVE == SAVE_STEPS) save_step<T, R>(a, sk, traj, t, u);
   }
   store_state<T, R>(a.u_end, 0, n, traj, u);
-  if constexpr (SAVE == SAVE_AT) save_unreached<T, R>(a, cur, traj);
+  if (SAVE == SAVE_AT && !a.filled) save_unreached<T, R>(a, cur, traj);
   if constexpr (SAVE == SAVE_STEPS) flush_steps<T, R>(a, sk);
   if (!lead) return;
   a.t_end[traj] = t;

@@ -74,6 +74,9 @@ struct sdeh_kargs {
   // then divide the scaled errors by bare Newton iterations (the error sum of
   // squares is the IEEE one whenever it lies in the controller's checked range).
   int32_t err_bare;
+  // saveat: 1 when u_saveat holds NaN before the launch, so that a trajectory leaves the
+  // rows it does not reach alone; 0: it writes NaN there.
+  int32_t filled;
   // Optional [n] debug counters: a lane that takes trajectory i up in a launch
   // (a fresh start, or a staged solve resuming it) adds 1 to visits[i].
   int32_t* visits;

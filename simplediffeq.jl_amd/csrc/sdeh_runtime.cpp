@@ -713,6 +713,27 @@ bool row_scratch(const sdeh_solve_desc* d, const Plan& pl, size_t bytes) {
          d->save_layout == SDEH_SAVE_POINT_MAJOR && bytes > kRowsFrom && bytes <= kRowsTo;
 }
 
+// Whether u_saveat is filled with NaN before the launch, or each trajectory writes NaN to
+// the rows it ended before.  The fill moves every byte of the output once more.  The kernel's
+// own rows cost nothing where the save times end with the span, and more than the fill once
+// there are some: a lane at a time, lines apart.  In the kernel | beforehand (us, point-major,
+// by how many of the save times lie beyond the end):
+//                                               none          3 %         25 %        90 %
+//   Lorenz ATsit5 binary64    1,024 x 101    209 | 213    217 | 207    239 | 185    314 | 116
+//                            20,001 x 101    215 | 223    222 | 219    250 | 195    356 | 129
+//                           150,001 x 101    604 | 666    609 | 660    622 | 616    800 | 512
+//   and with spans of 0.2 to 3 against save times up to 3: 234 | 205, 246 | 229, 540 | 532;
+//   GLV-16 ATsit5 binary64  131,072 x 128, spans of 2 to 20: 10,657 | 3,940.
+// The kernels with several lanes per trajectory write whole rows in the trajectory-major
+// layout and have no need of the fill there (the same spans: 1,435), and a fixed-step
+// ensemble ends all at once.
+bool nan_beforehand(const sdeh_solve_desc* d, const sdeh_io* io, const Plan& pl) {
+  if (pl.save != SAVE_AT || !is_adaptive(d->alg)) return false;
+  if (pl.k.lanes > 1 && d->save_layout != SDEH_SAVE_POINT_MAJOR) return false;
+  const double* end = d->saveat + d->n_saveat;
+  return io->tspan || 16 * (end - std::upper_bound(d->saveat, end, d->tf)) > d->n_saveat;
+}
+
 // Validate the descriptor and fill everything except the device pointers.
 // `path`: which entry point runs the plan (the default launch shape depends on it).
 enum class Path { kDevice, kHost, kStatic, kGraph };
@@ -810,6 +831,7 @@ int plan_solve(sdeh_ctx* c, const sdeh_solve_desc* d, const sdeh_io* io, Plan* p
   r = resolve_kernel(c, d->rhs, d->alg, d->dtype, pl->save, pl->kahan,
                      auto_lanes(d, pl->save, pl->kahan), &pl->k);
   if (r) return r;
+  a.filled = nan_beforehand(d, io, *pl);
   if (pl->packed && adaptive) {  // the counting pass: the endpoint kernel, same layout
     r = resolve_kernel(c, d->rhs, d->alg, d->dtype, SAVE_END, pl->kahan, pl->k.lanes,
                        &pl->k_count);
@@ -1053,9 +1075,9 @@ int launch_staged(sdeh_ctx* c, const Plan& pl, const KernelRef& k, int grid, int
 // Launch the prepared plan on `s` (kernel bracketed by the context events).
 int run_plan(sdeh_ctx* c, Plan& pl, hipStream_t s, unsigned long long* queue, bool timed) {
   sdeh_kargs& a = pl.a;
-  // The kernels write NaN to the rows a trajectory does not reach, so only an order that
-  // may leave trajectories out (one not checked to be a permutation) needs the fill.
-  if (pl.save == SAVE_AT && pl.unchecked_order) {
+  // NaN for the rows not reached, unless the kernel writes it (see nan_beforehand); and for
+  // those of trajectories that an order not checked to be a permutation may leave out.
+  if (pl.save == SAVE_AT && (a.filled || pl.unchecked_order)) {
     const int64_t cnt = a.n_saveat * pl.n_state * a.n;
     if (pl.es == 8) HIPCHK(c, sdeh_util_fill_f64((double*)a.u_saveat, __builtin_nan(""), cnt, s));
     else HIPCHK(c, sdeh_util_fill_f32((float*)a.u_saveat, __builtin_nanf(""), cnt, s));
@@ -1390,6 +1412,7 @@ int solve_impl(sdeh_ctx* c, const sdeh_solve_desc* d, const sdeh_io* io, int32_t
   }
   if (pl.by_rows && n > 0) {
     pl.rows_out = a.u_saveat;
+    if (pl.k.lanes > 1) a.filled = 0;  // whole rows now
     a.u_saveat = ar.take(sz.u_saveat);
     a.traj_major = 1;
   }

@@ -79,3 +79,62 @@ def test_rows_of_trajectories_left_out_are_nan(ctx):
     rows = b.numpy("u_saveat")
     assert np.isnan(rows[lost]).all()
     assert np.isfinite(np.delete(rows, lost, axis=0)).all()
+
+
+# The save times' share beyond the end decides whether the rows not reached are written by
+# the trajectories or beforehand: both sides of the line, and trajectories that end before
+# their span does, which no share foretells.
+@pytest.mark.parametrize("layout", [_abi.SAVE_POINT_MAJOR, _abi.SAVE_TRAJ_MAJOR])
+@pytest.mark.parametrize("rhs,alg,dtype,lanes", [
+    (_abi.RHS_LORENZ, _abi.ALG_ATSIT5, _abi.F64, 1),
+    (_abi.RHS_LORENZ, _abi.ALG_AVERN9, _abi.F64, 1),
+    (_abi.RHS_LORENZ, _abi.ALG_AVERN7, _abi.F32, 1),
+    (_abi.RHS_GLV16, _abi.ALG_ATSIT5, _abi.F64, 4)])
+@pytest.mark.parametrize("last,maxiters", [(1.0, 1000), (1.03, 1000), (1.1, 1000), (9.0, 1000),
+                                           (1.0, 9), (9.0, 9)])
+def test_rows_beyond_a_common_end_are_nan(ctx, rhs, alg, dtype, lanes, layout, last, maxiters):
+    n, saveat = 331, np.linspace(0.0, last, 33)
+    u0, p, ps = problem(rhs, n, seed=11)
+    d = runtime.make_desc(alg, dtype=dtype, rhs=rhs, n_traj=n, tspan=(0.0, 1.0),
+                          dt=float(np.float32(0.1)), abstol=1e-6, reltol=1e-5,
+                          maxiters=maxiters, saveat=saveat,
+                          lanes=lanes, save_layout=layout)
+    g, c = _solve_pair(ctx, d, u0.shape[0], u0, p, ps)
+    if dtype == _abi.F64:
+        assert_bit_identical(g, c, ("u_end", "t_end", "retcode", "naccept", "u_saveat"))
+    rows = g.numpy("u_saveat")
+    rows = rows if layout == _abi.SAVE_TRAJ_MAJOR else np.moveaxis(rows, -1, 0)
+    beyond = saveat[None, :] > g.numpy("t_end")[:, None]
+    assert np.array_equal(np.isnan(rows), np.broadcast_to(beyond[:, :, None], rows.shape))
+    assert not (rows == POISON).any()
+
+
+@pytest.mark.parametrize("own", [False, True])
+def test_rows_not_reached_are_nan_on_every_path(ctx, own):
+    import torch
+    n, saveat = 1003, np.linspace(0.0, 3.0, 17)
+    u0, p, _ = problem(_abi.RHS_LORENZ, n, seed=12)
+    ts = np.vstack([np.zeros(n), np.linspace(0.1, 3.2, n)]) if own else None
+    d = runtime.make_desc(_abi.ALG_ATSIT5, n_traj=n, tspan=(0.0, 1.0), dt=0.1, abstol=1e-6,
+                          reltol=1e-5, saveat=saveat)
+    g, c = _solve_pair(ctx, d, 3, u0, p, None, ts)
+    want = c.numpy("u_saveat")
+    h = runtime.EnsembleBuffers(d, 3, u0, p, tspan=ts)
+    h.u_saveat[...] = POISON
+    ctx.solve(d, h)
+    assert want.tobytes() == h.numpy("u_saveat").tobytes()
+    for call in ("static", "graph"):
+        g.u_saveat.fill_(POISON)
+        torch.cuda.synchronize()
+        if call == "static":
+            ctx.solve_static(d, g)
+        else:
+            h = ctx.graph_capture(d, g)
+            for _ in range(2):
+                g.u_saveat.fill_(POISON)
+                torch.cuda.synchronize()
+                ctx.graph_launch(h)
+                ctx.synchronize()
+            ctx.graph_destroy(h)
+        torch.cuda.synchronize()
+        assert want.tobytes() == g.numpy("u_saveat").tobytes(), call
