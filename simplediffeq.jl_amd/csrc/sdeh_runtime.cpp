@@ -705,12 +705,35 @@ Shape default_shape(sdeh_ctx* c, const Plan& pl, int dtype, int64_t n, bool sort
 //                            524,288 x 160         5,671 | 5,392
 //   AVern9  Lorenz           524,288 x 160         9,968 | 10,125
 //           GLV-16           131,072 x 120         5,535 | 5,806
+// Where only some of the save times lie in the span, the copy and the transpose move the rest
+// for nothing, so they are not counted, and the half has to be reached (ATsit5 Lorenz, of how
+// many points reached; in place, filled beforehand):
+//   262,144 x 200   100: 1,370 | 1,397   50:   818 | 1,236     700,001 x 101  50: 1,876 | 2,268
+//   131,072 x 400   200: 1,442 | 1,311  100:   811 | 1,157     150,001 x 101  50:   417 |   567
+// In an order (the caller's, or the longest span first) a wave's lanes hold trajectories far
+// apart, no store shares a line with another lane's, and rows win from fewer points on, once
+// the output is clear of that cache; with spans of their own nobody knows what is reached:
+//   ATsit5 Lorenz   random order | spans of 0.2 to 3 (us, in place | by way of rows)
+//     binary64  600,001 x  50 (90 M values)  3,180 | 1,430    1,190 |   980
+//               300,001 x  70 (63 M)         1,660 |   910      680 |   710
+//               150,001 x 101 (45 M)             not run        382 |   533
+//     binary32  600,001 x 100 (180 M)        5,700 | 1,330    1,800 | 1,020
+//   AVern7      300,001 x 100 (90 M)         3,020 | 1,750    1,110 | 1,100
+//     binary32  300,001 x 100 (90 M)         1,510 |   930      640 |   630
+//   AVern9      600,001 x  50 (90 M)         3,530 | 2,970    1,210 | 1,370  (in place, then)
 // (Fixed-step solvers reach a point with all lanes at once.)
 constexpr size_t kRowsFrom = size_t(300) << 20, kRowsTo = size_t(2) << 30;
-bool row_scratch(const sdeh_solve_desc* d, const Plan& pl, size_t bytes) {
-  const int64_t from = d->alg == SDEH_ALG_ATSIT5 ? 80 : d->alg == SDEH_ALG_AVERN7 ? 160 : 0;
-  return pl.save == SAVE_AT && from && d->n_saveat >= from &&
-         d->save_layout == SDEH_SAVE_POINT_MAJOR && bytes > kRowsFrom && bytes <= kRowsTo;
+constexpr size_t kOrderedRowsFrom = 75'000'000;  // values
+bool row_scratch(const sdeh_solve_desc* d, const sdeh_io* io, const Plan& pl, size_t bytes) {
+  if (pl.save != SAVE_AT || d->save_layout != SDEH_SAVE_POINT_MAJOR || bytes > kRowsTo ||
+      (d->alg != SDEH_ALG_ATSIT5 && d->alg != SDEH_ALG_AVERN7))
+    return false;
+  const int64_t reached =
+      io->tspan ? d->n_saveat : std::upper_bound(d->saveat, d->saveat + d->n_saveat, d->tf) -
+                                    d->saveat;
+  if (2 * reached < d->n_saveat) return false;
+  if (pl.span || io->order) return reached >= 32 && bytes / pl.es > kOrderedRowsFrom;
+  return reached >= (d->alg == SDEH_ALG_ATSIT5 ? 80 : 160) && bytes > kRowsFrom;
 }
 
 // Whether u_saveat is filled with NaN before the launch, or each trajectory writes NaN to
@@ -721,8 +744,7 @@ bool row_scratch(const sdeh_solve_desc* d, const Plan& pl, size_t bytes) {
 //                                               none          3 %         25 %        90 %
 //   Lorenz ATsit5 binary64    1,024 x 101    209 | 213    217 | 207    239 | 185    314 | 116
 //                            20,001 x 101    215 | 223    222 | 219    250 | 195    356 | 129
-//                           150,001 x 101    604 | 666    609 | 660    622 | 616    800 | 512
-//   and with spans of 0.2 to 3 against save times up to 3: 234 | 205, 246 | 229, 540 | 532;
+//   and with spans of 0.2 to 3 against save times up to 3: 234 | 205, 246 | 229;
 //   GLV-16 ATsit5 binary64  131,072 x 128, spans of 2 to 20: 10,657 | 3,940.
 // The kernels with several lanes per trajectory write whole rows in the trajectory-major
 // layout and have no need of the fill there (the same spans: 1,435), and a fixed-step
@@ -1287,7 +1309,7 @@ int solve_impl(sdeh_ctx* c, const sdeh_solve_desc* d, const sdeh_io* io, int32_t
     pl.shape.schedule = SDEH_SCHED_PERSISTENT;
   }
 
-  pl.by_rows = !host && row_scratch(d, pl, sz.u_saveat);
+  pl.by_rows = !host && row_scratch(d, io, pl, sz.u_saveat);
   // Device layout: saveat copy + (host mode) all buffers + counters always.
   const bool own_counts = !io->naccept || !io->nreject || host;
   auto scratch_need = [&]() {
