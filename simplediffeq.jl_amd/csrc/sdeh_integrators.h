@@ -202,7 +202,6 @@ struct LdsTab {
     return LdsTab{t};
   }
 };
-// The tables of a kernel: in LDS where ON (binary64), else the constant arrays.
 // The same with the constants of the logarithm and exponential in vector registers.
 struct LoneTab : LdsTab {
   double k[sdeh_math::PC_COUNT];
@@ -215,6 +214,7 @@ struct LoneTab : LdsTab {
     return tab;
   }
 };
+// The tables of a kernel: in LDS where ON (binary64), else the constant arrays.
 template <bool ON, bool LONE = false>
 __device__ __forceinline__ auto pow_tables() {
   if constexpr (ON && LONE) return LoneTab::init();
@@ -1076,7 +1076,7 @@ __device__ __forceinline__ void store_save(const sdeh_kargs& a, void* base, int6
 // Trajectory-major binary32 rows of four lanes with four components each are transposed:
 // lane q, which holds components q, q + 4, q + 8, q + 12, gets 4q .. 4q + 3, stored at
 // once, so that one store instruction writes a trajectory's 64-byte row end to end: with
-// shared weights 1,005 to 850 us for GLV-16 ATsit5, 2^17 trajectories, 256 points.  (binary64
+// shared weights 1,005 to 880 us for GLV-16 ATsit5, 2^17 trajectories, 256 points.  (binary64
 // rows, whose stores already write 32 bytes in a piece, lost by it: AVern9 7,150 / 7,250 us.)
 template <class T, class R>
 struct RowTr {  // the row's transpose: 4 x 4 over lanes 16 apart
@@ -1099,19 +1099,6 @@ __device__ __forceinline__ void transpose4(float (&u)[4]) {
   transpose4(r);
 #pragma unroll
   for (int c = 0; c < 4; ++c) u[c] = __builtin_bit_cast(float, r[c]);
-}
-__device__ __forceinline__ void transpose4(double (&u)[4]) {
-  unsigned lo[4], hi[4];
-#pragma unroll
-  for (int c = 0; c < 4; ++c) {
-    const uint64_t b = __builtin_bit_cast(uint64_t, u[c]);
-    lo[c] = (unsigned)b;
-    hi[c] = (unsigned)(b >> 32);
-  }
-  transpose4(lo);
-  transpose4(hi);
-#pragma unroll
-  for (int c = 0; c < 4; ++c) u[c] = __builtin_bit_cast(double, (uint64_t)hi[c] << 32 | lo[c]);
 }
 template <class T, class R>
 __device__ __forceinline__ T* save_row(const sdeh_kargs& a, void* base, int64_t row, int64_t rows,

@@ -86,20 +86,6 @@ SDEH_HD inline T fast_min(T x, T y) { return y < x ? y : x; }
 template <class T>
 SDEH_HD inline T fast_max(T x, T y) { return y > x ? y : x; }
 
-// Natural log of a finite x > 0 (normal or subnormal) as an unevaluated sum
-// hi + lo, |error| < 2^-66 |log x| + 2^-90 (table-driven, Tang's construction):
-//   x = 2^k z, z in [0x1.6ap-1, 0x1.6ap0), the subinterval index i taken from
-//   the top 7 bits of the bit pattern of z relative to 0x1.6ap-1;
-//   r = z * invc_i - 1 is exact (invc_i has 8 significant bits, |r| < 2^-7);
-//   log x = k ln2 + lc_i + log1p(r), lc_i = -log(invc_i) = lh_i + ll_i;
-//   log1p(r) = r - r^2/2 + r^3 P(r), P the Taylor series 1/3 - r/4 + ... - r^6/9
-//   (truncation below |r|^10/10 < 2^-70).
-// The large terms are added with error-free transformations (Knuth's two-sum;
-// the fast form where the first operand dominates or is zero): k ln2_hi is exact
-// (ln2_hi has 42 significant bits, |k| < 2^11).
-// log_norm_dd is the core for a normal x scaled by 2^-kadj (log of x * 2^kadj);
-// log_pos_dd scales subnormal inputs into the normal range first.
-// `tab` holds the reduction tables (ConstTab: the constant arrays).
 // The logarithm's and exponential's constants, by number, so that a table type can keep them
 // in registers.
 enum PowConst {
@@ -118,6 +104,7 @@ SDEH_HD constexpr double pow_const(int k) {
        : k == PC_E24 ? 0x1.5555555555555p-5 : 0x1.5555555555555p-3;
 }
 
+// The reduction tables as constant arrays.
 struct ConstTab {
   SDEH_HD double c(int k) const { return pow_const(k); }
   SDEH_HD void log_row(int i, double* invc, double* lh, double* ll) const {
@@ -131,7 +118,21 @@ struct ConstTab {
   }
 };
 
-// The logarithm from its reduction: x = 2^k z, subinterval i of z.
+// Natural log of a finite x > 0 (normal or subnormal) as an unevaluated sum
+// hi + lo, |error| < 2^-66 |log x| + 2^-90 (table-driven, Tang's construction):
+//   x = 2^k z, z in [0x1.6ap-1, 0x1.6ap0), the subinterval index i taken from
+//   the top 7 bits of the bit pattern of z relative to 0x1.6ap-1;
+//   r = z * invc_i - 1 is exact (invc_i has 8 significant bits, |r| < 2^-7);
+//   log x = k ln2 + lc_i + log1p(r), lc_i = -log(invc_i) = lh_i + ll_i;
+//   log1p(r) = r - r^2/2 + r^3 P(r), P the Taylor series 1/3 - r/4 + ... - r^6/9
+//   (truncation below |r|^10/10 < 2^-70).
+// The large terms are added with error-free transformations (Knuth's two-sum;
+// the fast form where the first operand dominates or is zero): k ln2_hi is exact
+// (ln2_hi has 42 significant bits, |k| < 2^11).
+// log_norm_dd is the core for a normal x scaled by 2^-kadj (log of x * 2^kadj);
+// log_pos_dd scales subnormal inputs into the normal range first.
+// `tab` holds the reduction tables.
+// log_reduced_dd: from the reduction, x = 2^k z and subinterval i of z.
 template <class Tab>
 SDEH_HD inline void log_reduced_dd(int i, int k, double z, double* hi, double* lo,
                                    const Tab& tab) {
