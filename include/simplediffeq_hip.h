@@ -126,7 +126,8 @@ typedef enum sdeh_schedule {
                                 one launch while the ensemble fits the GPU at once (three
                                 times that for endpoint output handed out longest span
                                 first, twice in binary32 with several lanes per
-                                trajectory), then staged up to four times (binary64,
+                                trajectory, four times for dense point-major saveat
+                                output over one tspan), then staged up to four times (binary64,
                                 one tspan, endpoint output) and persistent elsewhere
                                 (persistent at any size when grid, chunk or refill is
                                 set) */

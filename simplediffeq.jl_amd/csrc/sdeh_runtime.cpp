@@ -616,10 +616,10 @@ size_t staged_stride(const sdeh_solve_desc* d, const Plan& pl) {
 
 // The launch shape of an adaptive solve that names none and has not been tuned, for `n`
 // trajectories of which `sorted` says whether they are handed out longest span first and
-// `can_stage` whether the staged schedule is open to the solve.  `resident` = lanes that fit
-// the GPU at once.
+// `can_stage` whether the staged schedule is open to the solve and `dense` whether its output
+// is (see dense_output).  `resident` = lanes that fit the GPU at once.
 //   one launch   up to 1 x resident lanes (3 x for endpoint output in the span order, 2 x
-//                in binary32 with several lanes per trajectory).  While every wave is
+//                in binary32 with several lanes per trajectory, 4 x for dense output).  While every wave is
 //                resident the queue only costs: its atomics, its reset, and waves that take
 //                64 slots each while others get none.
 //   staged       binary64, one tspan, endpoint output, from there to 4 x: its first pass
@@ -669,13 +669,14 @@ size_t staged_stride(const sdeh_solve_desc* d, const Plan& pl) {
 constexpr size_t kStagedBytes = size_t(1) << 30;
 
 Shape default_shape(sdeh_ctx* c, const Plan& pl, int dtype, int64_t n, bool sorted,
-                    bool can_stage) {
+                    bool can_stage, bool dense) {
   Shape sh;
   const int lanes = pl.k.lanes > 0 ? pl.k.lanes : 1;
   const int64_t work = (n + pl.k.tpl - 1) / pl.k.tpl * lanes;
   const int64_t resident = (int64_t)c->cus * blocks_per_cu(c, pl.k, 256) * 256;
-  const int64_t times = lanes > 1 ? (dtype == SDEH_F32 ? 2 : 1)
-                                  : (sorted && pl.save == SAVE_END ? 3 : 1);
+  const int64_t times = dense       ? 4
+                        : lanes > 1 ? (dtype == SDEH_F32 ? 2 : 1)
+                                    : (sorted && pl.save == SAVE_END ? 3 : 1);
   sh.chunk = 64 / lanes;
   if (can_stage && !sorted && dtype == SDEH_F64 && work > resident && work <= 4 * resident) {
     sh.schedule = SDEH_SCHED_STAGED;
@@ -724,16 +725,48 @@ Shape default_shape(sdeh_ctx* c, const Plan& pl, int dtype, int64_t n, bool sort
 // (Fixed-step solvers reach a point with all lanes at once.)
 constexpr size_t kRowsFrom = size_t(300) << 20, kRowsTo = size_t(2) << 30;
 constexpr size_t kOrderedRowsFrom = 75'000'000;  // values
+
+// Save times in the common span; with spans of their own, all.
+int64_t reached_points(const sdeh_solve_desc* d, const sdeh_io* io) {
+  if (io->tspan) return d->n_saveat;
+  return std::upper_bound(d->saveat, d->saveat + d->n_saveat, d->tf) - d->saveat;
+}
+
 bool row_scratch(const sdeh_solve_desc* d, const sdeh_io* io, const Plan& pl, size_t bytes) {
   if (pl.save != SAVE_AT || d->save_layout != SDEH_SAVE_POINT_MAJOR || bytes > kRowsTo ||
       (d->alg != SDEH_ALG_ATSIT5 && d->alg != SDEH_ALG_AVERN7))
     return false;
-  const int64_t reached =
-      io->tspan ? d->n_saveat : std::upper_bound(d->saveat, d->saveat + d->n_saveat, d->tf) -
-                                    d->saveat;
+  const int64_t reached = reached_points(d, io);
   if (2 * reached < d->n_saveat) return false;
   if (pl.span || io->order) return reached >= 32 && bytes / pl.es > kOrderedRowsFrom;
   return reached >= (d->alg == SDEH_ALG_ATSIT5 ? 80 : 160) && bytes > kRowsFrom;
+}
+
+// Whether an adaptive solve of `n` trajectories over one span, in index order, stores in
+// place point-major output so dense that one launch is the faster up to 4 x the lanes that
+// fit the GPU at once, also for trajectories of unlike lengths: the lanes of a wave then stay
+// near the same save times, where refilled ones do not, and such a solve waits for its stores,
+// each a piece of a line.  Queue | one launch (us), like lengths and unlike ones:
+//   GLV-16, 131,072, binary64 (rates over two decades)
+//     AVern9  256 points  9,119 | 6,554  21,262 | 16,346     64  3,327 | 3,507   6,660 | 9,382
+//     ATsit5  256 points  6,854 | 5,913  18,214 | 14,855     64  1,272 | 1,132   3,243 | 2,609
+//                                                            32    836 |   781   1,579 | 2,213
+//   Lorenz, 800,000, binary64 (rho log-uniform in 0.5 .. 200)
+//     ATsit5   64 points  2,040 | 1,877   3,234 |  2,612     16    892 |   871   1,367 | 1,923
+//     AVern7  150 points  6,829 | 5,305  10,923 |  8,953     64  2,693 | 2,570   4,229 | 5,281
+//     AVern9  150 points  7,196 | 7,142   9,979 | 12,153
+bool dense_output(const sdeh_solve_desc* d, const sdeh_io* io, const Plan& pl, int64_t n,
+                  bool rows_open) {
+  if (pl.save != SAVE_AT || d->save_layout != SDEH_SAVE_POINT_MAJOR || io->tspan || io->order ||
+      (pl.k.lanes > 1 && d->dtype == SDEH_F32))
+    return false;
+  const size_t bytes = (size_t)d->n_saveat * pl.n_state * n * pl.es;
+  const int64_t from = d->alg == SDEH_ALG_ATSIT5   ? 64
+                       : d->alg == SDEH_ALG_AVERN7 ? 150
+                       : pl.k.lanes > 1            ? 256
+                                                   : INT64_MAX;
+  return reached_points(d, io) >= from && bytes > kRowsFrom &&
+         !(rows_open && row_scratch(d, io, pl, bytes));
 }
 
 // Whether u_saveat is filled with NaN before the launch, or each trajectory writes NaN to
@@ -905,7 +938,8 @@ int plan_solve(sdeh_ctx* c, const sdeh_solve_desc* d, const sdeh_io* io, Plan* p
                              stageable(d, io, *pl) && !io->visits &&
                              (size_t)n * (staged_stride(d, *pl) + 16) <= kStagedBytes;
       const int32_t w = sh.waves, tp = sh.per_lane;
-      sh = default_shape(c, *pl, d->dtype, n, pl->span && path != Path::kStatic, can_stage);
+      sh = default_shape(c, *pl, d->dtype, n, pl->span && path != Path::kStatic, can_stage,
+                         dense_output(d, io, *pl, n, path == Path::kDevice));
       sh.waves = w;
       sh.per_lane = tp;
       pl->default_staged = sh.schedule == SDEH_SCHED_STAGED;

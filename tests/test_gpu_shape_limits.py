@@ -124,3 +124,38 @@ def test_a_staged_solve_resumes_exactly_the_parked(ctx, alg, kahan, parked, n):
         assert att.max() > 32
     for f in FIELDS:
         assert bits_equal(out[0].numpy(f), out[1].numpy(f)), f
+
+
+@pytest.mark.parametrize("rhs,alg,points,layout,last,times,add,want", [
+    (_abi.RHS_GLV16, _abi.ALG_AVERN9, 256, _abi.SAVE_POINT_MAJOR, 0.3, 1, 1, 1),
+    (_abi.RHS_GLV16, _abi.ALG_AVERN9, 255, _abi.SAVE_POINT_MAJOR, 0.3, 1, 1, 2),
+    (_abi.RHS_GLV16, _abi.ALG_AVERN9, 256, _abi.SAVE_TRAJ_MAJOR, 0.3, 1, 1, 2),
+    (_abi.RHS_GLV16, _abi.ALG_AVERN9, 256, _abi.SAVE_POINT_MAJOR, 0.31, 1, 1, 2),
+    (_abi.RHS_LORENZ, _abi.ALG_ATSIT5, 64, _abi.SAVE_POINT_MAJOR, 0.3, 4, 0, 1),
+    (_abi.RHS_LORENZ, _abi.ALG_ATSIT5, 64, _abi.SAVE_POINT_MAJOR, 0.3, 4, 1, 2),
+    (_abi.RHS_LORENZ, _abi.ALG_ATSIT5, 63, _abi.SAVE_POINT_MAJOR, 0.3, 2, 0, 2),
+    (_abi.RHS_LORENZ, _abi.ALG_AVERN7, 150, _abi.SAVE_POINT_MAJOR, 0.3, 2, 0, 1)])
+def test_dense_output_stored_in_place_keeps_one_launch(rhs, alg, points, layout, last, times,
+                                                       add, want):
+    import torch
+    c = runtime.Context(0)
+
+    def solve(n, sched, **more):
+        u0, p, ps = _inputs(rhs, n)
+        d = runtime.make_desc(alg, rhs=rhs, n_traj=n, tspan=(0.0, 0.3), dt=0.1, abstol=1e-6,
+                              reltol=1e-5, saveat=np.linspace(0.0, last, points),
+                              save_layout=layout, schedule=sched, **more)
+        b = runtime.EnsembleBuffers(d, u0.shape[0], u0, p, ps, backend="torch", device="cuda:0")
+        c.solve(d, b)
+        return b, c.stats()
+
+    lanes = 4 if rhs == _abi.RHS_GLV16 else 1
+    _, st = solve(100, _abi.SCHED_PERSISTENT, lanes=lanes, block=256)
+    n = times * st["grid"] * 256 // lanes + add
+    got, st = solve(n, _abi.SCHED_AUTO)
+    assert st["schedule"] == (_abi.SCHED_ONE_LAUNCH if want == 1 else _abi.SCHED_PERSISTENT)
+    ref, _ = solve(n, _abi.SCHED_PERSISTENT if want == 1 else _abi.SCHED_ONE_LAUNCH, lanes=lanes)
+    for f in FIELDS:
+        assert bits_equal(got.numpy(f), ref.numpy(f)), f
+    assert torch.equal(got.u_saveat.view(torch.int64), ref.u_saveat.view(torch.int64))
+    c.close()
