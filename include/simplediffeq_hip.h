@@ -177,8 +177,9 @@ typedef struct sdeh_solve_desc {
   int32_t block;            /* 0 = tuned, else by schedule and layout (64 or 256); else
                                workgroup size (64, 128, 192 or 256) */
   int32_t grid;             /* 0 = tuned; persistent schedule: number of workgroups */
-  int32_t chunk;            /* 0 = tuned; persistent schedule: trajectories per queue
-                               grab (the last grab takes what is left) */
+  int32_t chunk;            /* 0 = tuned, else one wave's slots; persistent schedule:
+                               trajectories per queue grab (the last grab takes what is
+                               left) */
   int32_t lanes;            /* lanes per trajectory: 0 = for binary64, the right-hand
                                side's matrix-core layout where it has a kernel for the
                                solver and output (GLV16: 4 lanes 16 apart, 4 components

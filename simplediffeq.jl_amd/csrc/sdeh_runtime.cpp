@@ -469,8 +469,9 @@ int resolve_kernel(sdeh_ctx* c, int64_t rhs, int alg, int dtype, int save, int k
 //    524,288   1,840 | 1,400   2,037 | 1,733
 // (f32 matrix products run at twice the vector rate and beside it, a wave holds a quarter of
 // the trajectories, and the kernel's 107 registers leave four waves per SIMD instead of two.)
-// A caller that asks for the queue, whose default chunk is four of this layout's waves, keeps
-// one lane (120,001 trajectories over 20 time units 264 | 329).  An ensemble of at most 64
+// A caller that asks for the queue keeps one lane: a grid, chunk or batch is made for the
+// layout it has had, and a chunk of 64 is four of this layout's waves (120,001 trajectories
+// over 20 time units 264 | 329; with the chunk left open 259 | 229).  An ensemble of at most 64
 // keeps one lane too, although the layout is the faster one there as well (1 trajectory 396 |
 // 90, 64 trajectories 390 | 97): callers of `lanes` = 0 have been promised it; lanes = 4 asks.
 int auto_lanes(const sdeh_solve_desc* d, int save, int kahan) {
@@ -664,8 +665,10 @@ size_t staged_stride(const sdeh_solve_desc* d, const Plan& pl) {
 // One-lane kernels launch blocks of 64 (small ensembles spread over more CUs: 487
 // against 538 us at n = 1,024; the same beyond 65,536), the others blocks of 256 (their
 // LDS exchange buffers are sized for four waves: 12.9 against 7.9 ms in blocks of 64).
-// Persistent layouts with several lanes per trajectory claim one wave's slots at a time
-// (GLV-16 ATsit5, 500,000: 2,972 against 3,491 us claiming 64).
+// Persistent layouts with several lanes per trajectory claim one wave's slots at a time,
+// asked for or by default: claiming 64, a wave takes the work of several, others get none,
+// and which ones get it decides the time (GLV-16 ATsit5 binary64, 500,000: 2,972 against 3,491
+// us; 40,001 over 20 time units 203 against 360-436).
 constexpr size_t kStagedBytes = size_t(1) << 30;
 
 Shape default_shape(sdeh_ctx* c, const Plan& pl, int dtype, int64_t n, bool sorted,
@@ -907,8 +910,12 @@ int plan_solve(sdeh_ctx* c, const sdeh_solve_desc* d, const sdeh_io* io, Plan* p
   if (adaptive) {
     auto it = c->tuned.find(TuneKey(d->rhs, d->alg, d->dtype, pl->save, pl->kahan, pl->k.lanes,
                                      pl->packed));
-    if (it != c->tuned.end()) sh = it->second;
-    else sh.schedule = SDEH_SCHED_PERSISTENT;
+    if (it != c->tuned.end()) {
+      sh = it->second;
+    } else {
+      sh.schedule = SDEH_SCHED_PERSISTENT;
+      if (pl->k.lanes > 1) sh.chunk = 64 / pl->k.lanes;  // one wave's slots
+    }
     // the kernel variant: the caller's register cap or trajectories per lane, else
     // the tuned ones (where they exist for this solve), else the default kernel
     const bool mine = d->waves || d->per_lane;
@@ -2052,7 +2059,7 @@ int sdeh_autotune(sdeh_ctx* c, const sdeh_solve_desc* d, const sdeh_io* io, sdeh
       best_ms = ms;
       best_shape.schedule = k.sched;
       best_shape.block = k.block;
-      best_shape.chunk = k.chunk ? k.chunk : 64;
+      best_shape.chunk = c->stats.chunk;
       best_shape.grid = c->stats.grid;
       best_shape.waves = c->stats.waves;
       best_shape.per_lane = c->stats.per_lane;
@@ -2149,7 +2156,7 @@ int sdeh_autotune(sdeh_ctx* c, const sdeh_solve_desc* d, const sdeh_io* io, sdeh
         best_shape = Shape{};
         best_shape.schedule = k.sched;
         best_shape.block = k.block;
-        best_shape.chunk = k.chunk ? k.chunk : 64;
+        best_shape.chunk = c->stats.chunk;
         best_shape.grid = c->stats.grid;
         best_shape.per_lane = 2;
         best_stats = c->stats;

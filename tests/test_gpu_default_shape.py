@@ -141,3 +141,22 @@ def test_visit_counters_and_queue_fields_keep_the_queue(ctx):
     c.solve(d, b)
     assert (seen.cpu().numpy() == 1).all()
     c.close()
+
+
+@pytest.mark.parametrize("lanes,sched,more,chunk", [
+    (4, _abi.SCHED_PERSISTENT, {}, 16), (16, _abi.SCHED_PERSISTENT, {}, 4),
+    (4, _abi.SCHED_AUTO, dict(refill=2), 16), (16, _abi.SCHED_STAGED, {}, 4),
+    (4, _abi.SCHED_PERSISTENT, dict(chunk=64), 64), (1, _abi.SCHED_PERSISTENT, {}, 64)])
+def test_a_wave_claims_its_slots_where_the_queue_is_asked_for(ctx, lanes, sched, more, chunk):
+    """A wave that claimed several waves' slots at a time left others without work."""
+    n = 4001
+    u0, r, A = inputs.glv16(n, seed=1)
+    out = []
+    for s, kw in ((_abi.SCHED_ONE_LAUNCH, {}), (sched, more)):
+        d = runtime.make_desc(_abi.ALG_ATSIT5, rhs=_abi.RHS_GLV16, n_traj=n, tspan=(0.0, 2.0),
+                              dt=0.1, abstol=1e-6, reltol=1e-6, lanes=lanes, schedule=s, **kw)
+        b = runtime.EnsembleBuffers(d, 16, u0, r, A, backend="torch", device="cuda:0")
+        ctx.solve(d, b)
+        out.append(b)
+    assert ctx.stats()["schedule"] == _abi.SCHED_PERSISTENT and ctx.stats()["chunk"] == chunk
+    _same(out[1], out[0])
