@@ -1605,15 +1605,16 @@ struct SaveTimes {
   }
   // The same where every lane is at the same point (the fixed-step solvers): the later times
   // are scalar loads, which wait for no store.  at()'s vector loads there wait for the stores
-  // of the point before: Tsit5, 1,024 trajectories, 4,000 points 2,690 / 1,660 us (1,930 with
-  // every time a vector load one point ahead), 700 points 403 / 307 (380).
+  // of the point before: Tsit5, 1,024 trajectories, 4,000 points 2,690 / 1,670 us (1,930 with
+  // every time a vector load one point ahead), 700 points 403 / 314 (380).
   __device__ __forceinline__ double at_uniform(const sdeh_kargs& a, int64_t i) const {
     typedef const double __attribute__((address_space(4))) scalar_double;
     double r;
     if (i < SAVE_LDS) {
       r = lds[i];
     } else {
-      const int32_t k = __builtin_amdgcn_readfirstlane((int32_t)i);
+      const int64_t k = (int64_t)__builtin_amdgcn_readfirstlane((int32_t)(i >> 32)) << 32 |
+                        (uint32_t)__builtin_amdgcn_readfirstlane((int32_t)i);
       r = k < a.n_saveat ? ((scalar_double*)(uint64_t)a.saveat)[k] : 0.0;
       asm volatile("" ::"v"(r));
     }
