@@ -127,10 +127,10 @@ typedef enum sdeh_schedule {
                                 times that for endpoint output handed out longest span
                                 first, twice in binary32 with several lanes per
                                 trajectory, four times for dense point-major saveat
-                                output over one tspan), then staged up to four times (binary64,
-                                one tspan, endpoint output) and persistent elsewhere
-                                (persistent at any size when grid, chunk or refill is
-                                set) */
+                                output over one tspan), then staged up to four times
+                                (binary64, one tspan, endpoint output) and persistent
+                                elsewhere (persistent at any size when grid, chunk or
+                                refill is set) */
   SDEH_SCHED_ONE_LAUNCH = 1, /* one lane per trajectory, grid covers the ensemble */
   SDEH_SCHED_PERSISTENT = 2, /* resident grid; lanes refill from a device atomic queue */
   SDEH_SCHED_STAGED = 3      /* adaptive solvers with endpoint output, one lane per
@@ -307,8 +307,8 @@ int sdeh_compile_rhs(sdeh_ctx* ctx, const char* src, const char* fn_name, int32_
  * Scratch: a context keeps one device allocation, grown (by a quarter more than asked)
  * to its calls' largest need and given back by sdeh_destroy.  Of the library's own
  * choices, a staged or packed solve beyond what fits the GPU at once takes a parked
- * record per trajectory there (at most 1 GiB), and point-major saveat output of 300 MiB
- * to 2 GiB with many points as much as that output; where that memory cannot be had,
+ * record per trajectory there (at most 1 GiB), and point-major saveat output of some
+ * 300 MiB to 2 GiB with many points as much as that output; where that memory cannot be had,
  * the solve runs without it.  So does a solve whose `stream` the caller is capturing
  * into a graph (sync = 0): with device buffers, endpoint output, naccept and nreject
  * given, no order, and no tspan (or span_order = 1), it uses no such scratch and its

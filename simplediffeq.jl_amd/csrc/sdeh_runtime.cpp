@@ -616,13 +616,13 @@ size_t staged_stride(const sdeh_solve_desc* d, const Plan& pl) {
 }
 
 // The launch shape of an adaptive solve that names none and has not been tuned, for `n`
-// trajectories of which `sorted` says whether they are handed out longest span first and
+// trajectories of which `sorted` says whether they are handed out longest span first,
 // `can_stage` whether the staged schedule is open to the solve and `dense` whether its output
-// is (see dense_output).  `resident` = lanes that fit the GPU at once.
+// is dense (see dense_output).  `resident` = lanes that fit the GPU at once.
 //   one launch   up to 1 x resident lanes (3 x for endpoint output in the span order, 2 x
-//                in binary32 with several lanes per trajectory, 4 x for dense output).  While every wave is
-//                resident the queue only costs: its atomics, its reset, and waves that take
-//                64 slots each while others get none.
+//                in binary32 with several lanes per trajectory, 4 x for dense output).
+//                While every wave is resident the queue only costs: its atomics, its
+//                reset, and waves that take 64 slots each while others get none.
 //   staged       binary64, one tspan, endpoint output, from there to 4 x: its first pass
 //                ranks the trajectories (scratch bounded by kStagedBytes; no visit
 //                counters, which would count a resumed trajectory twice).
