@@ -125,7 +125,7 @@ typedef enum sdeh_schedule {
   SDEH_SCHED_AUTO = 0,       /* the tuned schedule (sdeh_autotune); without one, by size:
                                 one launch while the ensemble fits the GPU at once (three
                                 times that for endpoint output handed out longest span
-                                first, twice in binary32 with several lanes per
+                                first, one and a half in io->order, twice in binary32 with several lanes per
                                 trajectory, four times for dense point-major saveat
                                 output over one tspan), then staged up to four times
                                 (binary64, one tspan, endpoint output) and persistent

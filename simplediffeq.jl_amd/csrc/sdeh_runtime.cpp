@@ -617,10 +617,11 @@ size_t staged_stride(const sdeh_solve_desc* d, const Plan& pl) {
 
 // The launch shape of an adaptive solve that names none and has not been tuned, for `n`
 // trajectories of which `sorted` says whether they are handed out longest span first,
-// `can_stage` whether the staged schedule is open to the solve and `dense` whether its output
-// is dense (see dense_output).  `resident` = lanes that fit the GPU at once.
-//   one launch   up to 1 x resident lanes (3 x for endpoint output in the span order, 2 x
-//                in binary32 with several lanes per trajectory, 4 x for dense output).
+// `ordered` whether in a caller's order, `can_stage` whether the staged schedule is open to the
+// solve and `dense` whether its output is dense (see dense_output).  `resident` = lanes that fit the GPU at once.
+//   one launch   up to 1 x resident lanes (endpoint output: 3 x in the span order, 1.5 x in
+//                a caller's order; 2 x in binary32 with several lanes per trajectory, 4 x
+//                for dense output).
 //                While every wave is resident the queue only costs: its atomics, its
 //                reset, and waves that take 64 slots each while others get none.
 //   staged       binary64, one tspan, endpoint output, from there to 4 x: its first pass
@@ -638,12 +639,18 @@ size_t staged_stride(const sdeh_solve_desc* d, const Plan& pl) {
 //     spans 0.5 .. 10                     592 |   503     815 |   757   1,070 | 1,063
 //     the same, rho in 0.5 .. 200                         931 |   851   1,063 | 1,167
 //     spans 9 .. 10, rho in 0.5 .. 200  (1.3 x: 1,547 | 1,702)          2,231 | 3,355
-//   Lorenz ATsit5 over spans, in the order of a caller's keys, binary32 (524,288)
-//     keys the true lengths               398 |   242     494 |   320     849 |   668
-//     keys at random                      763 |   566     961 | 1,012   1,288 | 1,836
-//   and binary64: 2^20 (3.2 x) 956 | 806 and 1,637 | 2,448; binary32 2^22 (8 x) 1,614 |
-//   1,373 and 2,038 | 3,484.  A key that predicts nothing costs more than a true one gains,
-//   and the library cannot tell them apart, so a planned order counts as any other.
+//   Lorenz ATsit5, spans 0.5 .. 10, in the order of a caller's keys, at 1.25, 1.5 and 2 x
+//   binary32 compensated (458,752)
+//     keys 10 % off the lengths           652 |   376     745 |   416     851 |   503
+//     40 % off                            655 |   511     794 |   572     808 |   707
+//     keys at random                      700 |   662     762 |   744     832 |   955
+//     at random, rho in 0.5 .. 200      2,074 | 2,316   2,231 | 2,758   2,488 | 3,433
+//   binary64
+//     keys 10 % off the lengths           938 |   655   1,159 |   730   1,080 |   839
+//     keys at random                    1,102 | 1,170   1,153 | 1,343   1,268 | 1,637
+//   and 2^22 in binary32 (8 x): true lengths 1,614 | 1,373, at random 2,038 | 3,484.  A key that
+//   predicts nothing costs the more the larger the ensemble, and the library cannot tell it
+//   from a good one; an order that sdeh_plan_order made counts as any other.
 //   GLV-16, 256 points, AVern9 binary64 on the matrix cores (32,768)
 //     like growth rates                 2,224 | 2,157   4,362 | 3,987   7,247 | 6,492
 //     rates over two decades            6,406 | 6,252   8,668 | 11,213 10,967 | 16,735
@@ -672,18 +679,19 @@ size_t staged_stride(const sdeh_solve_desc* d, const Plan& pl) {
 constexpr size_t kStagedBytes = size_t(1) << 30;
 
 Shape default_shape(sdeh_ctx* c, const Plan& pl, int dtype, int64_t n, bool sorted,
-                    bool can_stage, bool dense) {
+                    bool can_stage, bool dense, bool ordered) {
   Shape sh;
   const int lanes = pl.k.lanes > 0 ? pl.k.lanes : 1;
   const int64_t work = (n + pl.k.tpl - 1) / pl.k.tpl * lanes;
   const int64_t resident = (int64_t)c->cus * blocks_per_cu(c, pl.k, 256) * 256;
-  const int64_t times = dense       ? 4
-                        : lanes > 1 ? (dtype == SDEH_F32 ? 2 : 1)
-                                    : (sorted && pl.save == SAVE_END ? 3 : 1);
+  const bool end = pl.save == SAVE_END;
+  const double times = dense       ? 4.0
+                       : lanes > 1 ? (dtype == SDEH_F32 ? 2.0 : 1.0)
+                                   : (end && sorted ? 3.0 : end && ordered ? 1.5 : 1.0);
   sh.chunk = 64 / lanes;
   if (can_stage && !sorted && dtype == SDEH_F64 && work > resident && work <= 4 * resident) {
     sh.schedule = SDEH_SCHED_STAGED;
-  } else if (work <= times * resident) {
+  } else if (work <= (int64_t)(times * (double)resident)) {
     sh.schedule = SDEH_SCHED_ONE_LAUNCH;
     if (lanes == 1) sh.block = 64;
   } else {
@@ -946,7 +954,7 @@ int plan_solve(sdeh_ctx* c, const sdeh_solve_desc* d, const sdeh_io* io, Plan* p
                              (size_t)n * (staged_stride(d, *pl) + 16) <= kStagedBytes;
       const int32_t w = sh.waves, tp = sh.per_lane;
       sh = default_shape(c, *pl, d->dtype, n, pl->span && path != Path::kStatic, can_stage,
-                         dense_output(d, io, *pl, n, path == Path::kDevice));
+                         dense_output(d, io, *pl, n, path == Path::kDevice), io->order != nullptr);
       sh.waves = w;
       sh.per_lane = tp;
       pl->default_staged = sh.schedule == SDEH_SCHED_STAGED;
